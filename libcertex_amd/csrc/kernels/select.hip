@@ -12,6 +12,7 @@
 //   finish     certex.cu:224-250.
 
 #include "../kernels.hpp"
+#include "lanes.hpp"
 
 #include <cfloat>
 #include <climits>
@@ -22,22 +23,23 @@ namespace {
 
 constexpr int kThreads = 256;
 
-/** Inclusive prefix sum over the 256 threads of a block (4 waves). */
-__device__ inline int block_scan_incl(int v, int* wave_tot)
+/** Inclusive prefix sum over the T threads of a block of T = 64 (one wave), kThreads or 1024. */
+template <int T>
+__device__ inline int scan_incl_t(int v, int* wave_tot)
 {
+  static_assert(T == 64 || T == kThreads || T == 1024, "block shapes of the selects");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int incl = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int t = __shfl_up(incl, off);
-    if (lane >= off) { incl += t; }
+  const int incl = lanes::scan_incl(v);
+  if constexpr (T == 64) {
+    return incl;
+  } else {
+    if (lane == 63) { wave_tot[wave] = incl; }
+    __syncthreads();
+    int add = 0;
+    for (int w = 0; w < wave; ++w) { add += wave_tot[w]; }
+    __syncthreads();
+    return incl + add;
   }
-  if (lane == 63) { wave_tot[wave] = incl; }
-  __syncthreads();
-  int add = 0;
-  for (int w = 0; w < wave; ++w) { add += wave_tot[w]; }
-  __syncthreads();
-  return incl + add;
 }
 
 /** The largest of key[0, n) over the block (every thread gets it); scratch: 4 LDS words x 2. */
@@ -45,11 +47,7 @@ __device__ inline uint64_t block_max_key(const uint64_t* key, int n, uint64_t* w
 {
   uint64_t m = 0;
   for (int e = threadIdx.x; e < n; e += kThreads) { m = key[e] > m ? key[e] : m; }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const uint64_t o = __shfl_xor(m, off);
-    m                = o > m ? o : m;
-  }
+  m = lanes::max<64>(m);
   if ((threadIdx.x & 63) == 0) { wave_max[threadIdx.x >> 6] = m; }
   __syncthreads();
   uint64_t r = wave_max[0];
@@ -140,7 +138,7 @@ __global__ void max_kernel(const uint32_t* c, int64_t n, uint32_t* out)
        i += int64_t(gridDim.x) * blockDim.x) {
     m = max(m, c[i]);
   }
-  for (int off = 32; off; off >>= 1) { m = max(m, uint32_t(__shfl_xor(int(m), off))); }
+  m = lanes::max<64>(m);
   if ((threadIdx.x & 63) == 0) { atomicMax(out, m); }
 }
 
@@ -151,9 +149,7 @@ __global__ void sum_kernel(const uint32_t* c, int64_t n, int64_t cap, unsigned l
        i += int64_t(gridDim.x) * blockDim.x) {
     s += c[i] < cap ? c[i] : uint64_t(cap);
   }
-  for (int off = 32; off; off >>= 1) {
-    s += (unsigned long long)__shfl_xor((long long)s, off);
-  }
+  s = lanes::sum<64>(s);
   if ((threadIdx.x & 63) == 0) { atomicAdd(out, s); }
 }
 
@@ -322,8 +318,8 @@ __device__ __forceinline__ void bitonic_stage_regs(uint64_t (&k)[E], uint32_t (&
     const bool lower = (t & D) == 0;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const uint64_t ok  = __shfl_xor(k[e], D);
-      const uint32_t orr = __shfl_xor(r[e], D);
+      const uint64_t ok  = lanes::exchange<D>(k[e]);
+      const uint32_t orr = lanes::exchange<D>(r[e]);
       const bool up      = ((t * E + e) & SIZE) == 0;
       if (pair_less(k[e], r[e], ok, orr) != (lower == up)) {  // the lower one keeps the minimum
         k[e] = ok;                                             // going up
@@ -442,12 +438,8 @@ __device__ inline void select_pair(const uint64_t* key, const uint32_t* row, int
     lo                = kk < lo ? kk : lo;
     hi                = kk > hi ? kk : hi;
   }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const uint64_t l = __shfl_xor(lo, off), h = __shfl_xor(hi, off);
-    lo               = l < lo ? l : lo;
-    hi               = h > hi ? h : hi;
-  }
+  lo = lanes::min<64>(lo);
+  hi = lanes::max<64>(hi);
   if ((tid & 63) == 0) {
     rng[tid >> 6]                 = lo;
     rng[kThreads / 64 + (tid >> 6)] = hi;
@@ -476,7 +468,7 @@ __device__ inline void select_pair(const uint64_t* key, const uint32_t* row, int
     }
     __syncthreads();
     const int c    = hist[tid];
-    const int incl = block_scan_incl(c, wave_tot);
+    const int incl = scan_incl_t<kThreads>(c, wave_tot);
     if (incl - c < rank && rank <= incl) {
       *sel_digit = uint32_t(tid);
       *sel_rank  = rank - (incl - c);
@@ -511,7 +503,7 @@ __device__ inline void select_pair(const uint64_t* key, const uint32_t* row, int
       }
       __syncthreads();
       const int c    = hist[tid];
-      const int incl = block_scan_incl(c, wave_tot);
+      const int incl = scan_incl_t<kThreads>(c, wave_tot);
       if (incl - c < rank && rank <= incl) {
         *sel_digit = uint32_t(tid);
         *sel_rank  = rank - (incl - c);
@@ -781,200 +773,215 @@ __device__ inline double fcoord(const void* p, elem t, int64_t i)
                         : double(static_cast<const _Float16*>(p)[i]);
 }
 
+/** P consecutive coordinates of a stored row as loaded. */
+template <typename T, int P>
+struct raw_coords {
+  T v[P];
+};
+
 /**
- * Coordinates j .. j + P - 1 of a stored row as doubles (zero past dim): one vector load when
- * `aligned` (dim a multiple of P, so that j is too), else one coordinate at a time.
- */
-/**
- * Coordinates j .. j + P - 1 of stored row `row` as doubles, zero at and past dim. ALIGNED (dim a
- * multiple of P, so that j is too): one vector load, from a clamped position when j >= dim; else
- * one coordinate at a time, each from a clamped position. The loads are unconditional, so that a
- * row's loads are issued together rather than each behind a branch.
+ * Coordinates j .. j + P - 1 of stored row `row`, zero at and past dim. ALIGNED (dim a multiple
+ * of P, so that j is too): one vector load, from a clamped position when j >= dim; else one
+ * coordinate at a time, each from a clamped position. The loads are unconditional, so that a row's
+ * loads are issued together rather than each behind a branch.
  */
 template <typename T, int P, bool ALIGNED>
-__device__ __forceinline__ void load_coords(const T* x, int64_t row, int64_t dim, int64_t j, double (&b)[P])
+__device__ __forceinline__ raw_coords<T, P> load_coords(const T* x, int64_t row, int64_t dim, int64_t j)
 {
-  if constexpr (ALIGNED) {
-    const bool ok    = j < dim;
-    const T* src     = x + row * dim + (ok ? j : dim - P);
-    if constexpr (P == 1) {
-      const double v = double(src[0]);
-      b[0]           = ok ? v : 0.0;
-    } else {
-      typedef T tp __attribute__((ext_vector_type(P)));
-      const tp v = *reinterpret_cast<const tp*>(src);
+  raw_coords<T, P> c;
+  if constexpr (ALIGNED && P > 1) {
+    typedef T tp __attribute__((ext_vector_type(P)));
+    const bool ok = j < dim;
+    tp v          = *reinterpret_cast<const tp*>(x + row * dim + (ok ? j : dim - P));
+    v             = ok ? v : tp(T(0));
 #pragma unroll
-      for (int u = 0; u < P; ++u) { b[u] = ok ? double(v[u]) : 0.0; }
-    }
+    for (int u = 0; u < P; ++u) { c.v[u] = v[u]; }
   } else {
 #pragma unroll
     for (int u = 0; u < P; ++u) {
-      const bool ok  = j + u < dim;
-      const double v = double(x[row * dim + (ok ? j + u : dim - 1)]);
-      b[u]           = ok ? v : 0.0;
+      const bool ok = j + u < dim;
+      const T v     = x[row * dim + (ok ? j + u : dim - 1)];
+      c.v[u]        = ok ? v : T(0);
     }
   }
+  return c;
+}
+
+/** 64-coordinate blocks that a slot of L lanes loads of a row at once: whole rows of up to 128
+ *  coordinates with 16 lanes, of up to 256 with 32; 256 coordinates at a time with 64. */
+constexpr int slot_blocks(int L) { return L == 16 ? 2 : 4; }
+/** Coordinates of the query copy in LDS (zeros past dim): a multiple of what a slot loads at once. */
+__host__ __device__ inline int64_t query_coords(int L, int64_t dim)
+{
+  const int64_t c = 64 * slot_blocks(L);
+  return (dim + c - 1) / c * c;
 }
 
 /**
- * Exact fp64 scores of stored rows against the query whose coordinates sit in LDS as doubles, in
- * the oracle's canonical order: 64 partial sums, partial p accumulating coordinates p, p + 64, ...
- * in increasing order with fused multiply-adds, combined by the xor butterfly (for off = 32 .. 1:
- * p[i] + p[i ^ off]). A row is scored by L lanes of a wave (a slot): lane g of the slot keeps the
- * P = 64 / L consecutive partials P g .. P g + P - 1, read with one vector load per 64
- * coordinates; the butterfly levels off >= P pair lane g with lane g ^ (off / P) and the levels
- * below P combine partials inside a lane, so every lane of the slot ends with the same bits. With
- * L < 64 a wave scores 64 / L rows at once, NR rows per slot, U 64-coordinate blocks per
- * iteration. l2: sum (q - x)^2; inner: -sum q x; cosine: -sum q x / sqrt(sum q^2 sum x^2).
- * The element type, the metric and the alignment are template parameters: the loop holds no
- * branch, and the loads of an iteration go out together.
+ * Exact fp64 scores of stored rows against the query whose coordinates sit in LDS as doubles
+ * (zeros up to query_coords), in the oracle's canonical order: 64 partial sums, partial p
+ * accumulating coordinates p, p + 64, ... in increasing order with fused multiply-adds, combined
+ * by the xor butterfly (for off = 32 .. 1: p[i] + p[i ^ off]). A row is scored by L lanes of a wave
+ * (a slot): lane g of the slot keeps the P = 64 / L consecutive partials P g .. P g + P - 1, read
+ * with one vector load per 64 coordinates; the butterfly levels off >= P pair lane g with lane
+ * g ^ (off / P), the levels below P partials of one lane. Terms past dim add +0 (the coordinates
+ * and the query are zero there), which leaves every sum's value. A wave scores 64 / L slots of NR
+ * rows at once. l2: sum (q - x)^2; inner: -sum q x; cosine: -sum q x / sqrt(sum q^2 sum x^2), with
+ * qq = sum q^2 of the query, the same for every row.
+ *
+ * What bounds it: with few coordinates per lane the butterfly costs more than the products. Its
+ * sums (P partials of NR rows, and of the rows' squares for cosine) are split over the lanes as
+ * the levels go down (lanes::split_sums), on the VALU: as __shfl_xor levels of every sum they were
+ * 64 LDS-pipe exchanges for 8 rows of 128 coordinates, and 60 for 2 rows of 768. A whole search
+ * with the shuffles and now: 2,048 queries, k = 2,048 of 131,072 bf16 keys x 128, 1,075 -> 853 us;
+ * 10,000 queries, k = 100 of 16 labels, 768 float32 coordinates, 2,000 -> 1,870 us.
  */
-template <int L, int NR, typename T, metric_kind M, bool ALIGNED>
-__device__ __forceinline__ void slot_scores(const double* qv, const T* x, const int64_t (&rows)[NR],
-                                   int64_t dim, int g, double (&out)[NR])
+template <int L, typename T, metric_kind M, bool ALIGNED, int NT>
+__device__ __forceinline__ void score_rows_t(const double* qv, double qq, const T* x, int64_t dim,
+                                             const uint32_t* rid, uint64_t* key, int from, int to)
 {
-  constexpr int P = 64 / L;            // partials per lane
-  constexpr int U = 64 / L >= 2 ? 2 : 4;  // 64-coordinate blocks per iteration
-  double acc[NR][P], xx[NR][P], qq[P];
+  constexpr int P    = 64 / L;  // partials per lane
+  constexpr int U    = slot_blocks(L);
+  constexpr int NR   = 2;  // rows per slot
+  constexpr int S    = M == metric_kind::cosine ? 2 : 1;  // sums per row: products, squares
+  constexpr int N    = P * NR * S;  // sums per lane; sum (u, r, s) is w[(u NR + r) S + s]
+  constexpr int PER  = (64 / L) * NR;  // rows per wave at a time
+  constexpr bool ONE = L < 64;         // a whole row is one load (launched for dim <= 64 U)
+  static_assert(N <= L, "split_sums");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g    = lane % L;
+  const int slot = lane / L;
+  // after split_sums the lanes of sum (u, r, s) spell it from bit L / 2 down: u, then r, then s
+  constexpr int DR = L / 2 / P;  // the lane bit of r (NR = 2)
+  const int my_r   = (g & DR) != 0 ? 1 : 0;
+  const bool put   = (g & ~DR) == 0;  // one lane per row: u = 0, s = 0, no further bit
+
+  double q1[ONE ? U * P : 1];  // the lane's query coordinates, the same for every row
+  if constexpr (ONE) {
 #pragma unroll
-  for (int u = 0; u < P; ++u) {
-    qq[u] = 0;
+    for (int v = 0; v < U; ++v) {
 #pragma unroll
-    for (int r = 0; r < NR; ++r) { acc[r][u] = xx[r][u] = 0; }
+      for (int u = 0; u < P; ++u) { q1[v * P + u] = qv[64 * v + P * g + u]; }
+    }
   }
-  for (int64_t j0 = int64_t(P) * g; j0 < dim; j0 += 64 * U) {
-    double b[NR][U][P];
+  raw_coords<T, P> b[NR][U];
+  auto load = [&](int e0, int64_t j0) {
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
+      const int e       = e0 + slot * NR + r;
+      const int64_t row = int64_t(rid[e < to ? e : to - 1]);
 #pragma unroll
-      for (int v = 0; v < U; ++v) { load_coords<T, P, ALIGNED>(x, rows[r], dim, j0 + 64 * v, b[r][v]); }
+      for (int v = 0; v < U; ++v) { b[r][v] = load_coords<T, P, ALIGNED>(x, row, dim, j0 + 64 * v + P * g); }
     }
+  };
+  double w[N];
+  auto add = [&](int64_t j0) {
 #pragma unroll
     for (int v = 0; v < U; ++v) {
 #pragma unroll
       for (int u = 0; u < P; ++u) {
-        const int64_t j = j0 + 64 * v + u;
-        if (j < dim) {
-          const double a = qv[j];
-          if constexpr (M == metric_kind::cosine) { qq[u] = fma(a, a, qq[u]); }
+        double a;
+        if constexpr (ONE) {
+          a = q1[v * P + u];
+        } else {
+          a = qv[j0 + 64 * v + P * g + u];
+        }
 #pragma unroll
-          for (int r = 0; r < NR; ++r) {
-            const double xv = b[r][v][u];
-            if constexpr (M == metric_kind::l2) {
-              const double d = a - xv;
-              acc[r][u]      = fma(d, d, acc[r][u]);
-            } else {
-              acc[r][u] = fma(a, xv, acc[r][u]);
-              if constexpr (M == metric_kind::cosine) { xx[r][u] = fma(xv, xv, xx[r][u]); }
+        for (int r = 0; r < NR; ++r) {
+          double& s       = w[(u * NR + r) * S];
+          const double xv = double(b[r][v].v[u]);
+          if constexpr (M == metric_kind::l2) {
+            const double d = a - xv;
+            s              = fma(d, d, s);
+          } else {
+            s = fma(a, xv, s);
+            if constexpr (M == metric_kind::cosine) {
+              double& xx = w[(u * NR + r) * S + 1];
+              xx         = fma(xv, xv, xx);
             }
           }
         }
       }
     }
-  }
-  // butterfly levels off = 32 .. P across the lanes of the slot: partner lane g ^ (off / P)
+  };
+  int e0 = from + wave * PER;
+  if (e0 >= to) { return; }
+  if constexpr (ONE) { load(e0, 0); }
+  while (true) {
 #pragma unroll
-  for (int lx = 32 / P; lx >= 1; lx >>= 1) {
-#pragma unroll
-    for (int u = 0; u < P; ++u) {
-      if constexpr (M == metric_kind::cosine) { qq[u] += __shfl_xor(qq[u], lx); }
-#pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        acc[r][u] += __shfl_xor(acc[r][u], lx);
-        if constexpr (M == metric_kind::cosine) { xx[r][u] += __shfl_xor(xx[r][u], lx); }
-      }
-    }
-  }
-  // levels off < P inside the lane: partial u pairs with u ^ off
-#pragma unroll
-  for (int h = P / 2; h >= 1; h >>= 1) {
-#pragma unroll
-    for (int u = 0; u < P; ++u) {
-      if (u & h) { continue; }
-      qq[u] += qq[u | h];
-#pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        acc[r][u] += acc[r][u | h];
-        xx[r][u] += xx[r][u | h];
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    if constexpr (M == metric_kind::l2) {
-      out[r] = acc[r][0];
-    } else if constexpr (M == metric_kind::inner) {
-      out[r] = -acc[r][0];
+    for (int i = 0; i < N; ++i) { w[i] = 0; }
+    const int e1 = e0 + PER * (NT / 64);
+    if constexpr (ONE) {
+      add(0);
+      if (e1 < to) { load(e1, 0); }  // the next rows' loads fly while these sums are combined
     } else {
-      out[r] = -acc[r][0] / sqrt(qq[0] * xx[r][0]);
-    }
-  }
-}
-
-/** score_rows_l for one element type, metric and alignment. */
-template <int L, typename T, metric_kind M, bool ALIGNED>
-__device__ __forceinline__ void score_rows_t(const double* qv, const T* x, int64_t dim, const uint32_t* rid,
-                                    uint64_t* key, int from, int to)
-{
-  constexpr int NR   = 2;  // rows per slot (1, 3 and 4 measured slower at configs 3 and 4)
-  constexpr int PER  = (64 / L) * NR;  // rows per wave at a time
-  const int lane     = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g        = lane % L;
-  const int slot     = lane / L;
-  for (int e0 = from + wave * PER; e0 < to; e0 += PER * (kThreads / 64)) {
-    int64_t rows[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int e = e0 + slot * NR + r;
-      rows[r]     = int64_t(rid[e < to ? e : to - 1]);
-    }
-    double sc[NR];
-    slot_scores<L, NR, T, M, ALIGNED>(qv, x, rows, dim, g, sc);
-    if (g == 0) {
-#pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        const int e = e0 + slot * NR + r;
-        if (e < to) { key[e] = score_key(sc[r]); }
+      for (int64_t j0 = 0; j0 < dim; j0 += 64 * U) {
+        load(e0, j0);
+        add(j0);
       }
     }
+    lanes::split_sums<L, N>(w);
+    double sc = w[0];
+    // levels off < P: partials of one lane, now in the lanes g ^ (L / 2), g ^ (L / 4), ...
+    if constexpr (P >= 4) { sc += lanes::exchange<L / 2>(sc); }
+    if constexpr (P >= 2) { sc += lanes::exchange<(P >= 4 ? L / 4 : L / 2)>(sc); }
+    if constexpr (M == metric_kind::inner) { sc = -sc; }
+    if constexpr (M == metric_kind::cosine) {
+      const double xx = lanes::exchange<DR / 2>(sc);  // the row's squares (s = 1)
+      sc              = -sc / sqrt(qq * xx);
+    }
+    const int e = e0 + slot * NR + my_r;
+    if (put && e < to) { key[e] = score_key(sc); }
+    if (e1 >= to) { break; }
+    e0 = e1;
   }
 }
 
-template <int L, typename T>
-__device__ __forceinline__ void score_rows_m(const double* qv, const T* x, int64_t dim, metric_kind metric,
-                                    const uint32_t* rid, uint64_t* key, int from, int to)
+template <int L, int NT, typename T>
+__device__ __forceinline__ void score_rows_m(const double* qv, double qq, const T* x, int64_t dim,
+                                    metric_kind metric, const uint32_t* rid, uint64_t* key, int from, int to)
 {
   constexpr int P    = 64 / L;
   const bool aligned = dim % P == 0;
   switch (metric) {
     case metric_kind::l2:
-      aligned ? score_rows_t<L, T, metric_kind::l2, true>(qv, x, dim, rid, key, from, to)
-              : score_rows_t<L, T, metric_kind::l2, false>(qv, x, dim, rid, key, from, to);
+      aligned ? score_rows_t<L, T, metric_kind::l2, true, NT>(qv, qq, x, dim, rid, key, from, to)
+              : score_rows_t<L, T, metric_kind::l2, false, NT>(qv, qq, x, dim, rid, key, from, to);
       break;
     case metric_kind::inner:
-      aligned ? score_rows_t<L, T, metric_kind::inner, true>(qv, x, dim, rid, key, from, to)
-              : score_rows_t<L, T, metric_kind::inner, false>(qv, x, dim, rid, key, from, to);
+      aligned ? score_rows_t<L, T, metric_kind::inner, true, NT>(qv, qq, x, dim, rid, key, from, to)
+              : score_rows_t<L, T, metric_kind::inner, false, NT>(qv, qq, x, dim, rid, key, from, to);
       break;
     default:
-      aligned ? score_rows_t<L, T, metric_kind::cosine, true>(qv, x, dim, rid, key, from, to)
-              : score_rows_t<L, T, metric_kind::cosine, false>(qv, x, dim, rid, key, from, to);
+      aligned ? score_rows_t<L, T, metric_kind::cosine, true, NT>(qv, qq, x, dim, rid, key, from, to)
+              : score_rows_t<L, T, metric_kind::cosine, false, NT>(qv, qq, x, dim, rid, key, from, to);
       break;
   }
 }
 
-/** Scores rid[from, to) into key[] (ordered keys) with slots of L lanes, NR rows per slot. */
-template <int L>
-__device__ __forceinline__ void score_rows_l(const double* qv, const void* vectors, elem t, int64_t dim,
+/** Scores rid[from, to) into key[] (ordered keys) by the NT threads of the block, with slots of L
+ *  lanes. */
+template <int L, int NT>
+__device__ __forceinline__ void score_rows_l(const double* qv, double qq, const void* vectors, elem t, int64_t dim,
                                     metric_kind metric, const uint32_t* rid, uint64_t* key,
                                     int from, int to)
 {
   if (t == elem::f32) {
-    score_rows_m<L>(qv, static_cast<const float*>(vectors), dim, metric, rid, key, from, to);
+    score_rows_m<L, NT>(qv, qq, static_cast<const float*>(vectors), dim, metric, rid, key, from, to);
   } else if (t == elem::bf16) {
-    score_rows_m<L>(qv, static_cast<const __bf16*>(vectors), dim, metric, rid, key, from, to);
+    score_rows_m<L, NT>(qv, qq, static_cast<const __bf16*>(vectors), dim, metric, rid, key, from, to);
   } else {
-    score_rows_m<L>(qv, static_cast<const _Float16*>(vectors), dim, metric, rid, key, from, to);
+    score_rows_m<L, NT>(qv, qq, static_cast<const _Float16*>(vectors), dim, metric, rid, key, from, to);
   }
+}
+
+/** sum q^2 of the query copy in LDS (n coordinates, a multiple of 64), in the canonical order:
+ *  lane p of every wave accumulates coordinates p, p + 64, ...; every thread gets the sum. */
+__device__ __forceinline__ double query_square(const double* qv, int64_t n)
+{
+  double s = 0;
+  for (int64_t j = threadIdx.x & 63; j < n; j += 64) { s = fma(qv[j], qv[j], s); }
+  return lanes::sum<64>(s);
 }
 
 /**
@@ -1172,43 +1179,14 @@ __global__ void certificate_bounds_kernel(threshold_f_args a, const uint32_t* co
   }
 }
 
-/** Inclusive prefix sum over the T threads of a block of T = 64 (one wave), kThreads or 1024. */
-template <int T>
-__device__ inline int scan_incl_t(int v, int* wave_tot)
-{
-  static_assert(T == 64 || T == kThreads || T == 1024, "block shapes of the selects");
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int incl = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int t = __shfl_up(incl, off);
-    if (lane >= off) { incl += t; }
-  }
-  if constexpr (T == 64) {
-    return incl;
-  } else {
-    if (lane == 63) { wave_tot[wave] = incl; }
-    __syncthreads();
-    int add = 0;
-    for (int w = 0; w < wave; ++w) { add += wave_tot[w]; }
-    __syncthreads();
-    return incl + add;
-  }
-}
-
 /** The minimum, the maximum and the sum of (lo, hi, n) over the T threads of a block; every
  *  thread gets them. red: 3 * 16 LDS words. */
 template <int T>
 __device__ inline void block_min_max_sum(uint32_t& lo, uint32_t& hi, int& n, uint32_t* red)
 {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const uint32_t l = __shfl_xor(lo, off), h = __shfl_xor(hi, off);
-    const int c      = __shfl_xor(n, off);
-    lo               = l < lo ? l : lo;
-    hi               = h > hi ? h : hi;
-    n += c;
-  }
+  lo = lanes::min<64>(lo);
+  hi = lanes::max<64>(hi);
+  n  = lanes::sum<64>(n);
   if constexpr (T > 64) {
     constexpr int W = T / 64;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1320,7 +1298,7 @@ __device__ int radix_pass(int64_t n, F key_of, radix_state& st, int* hist, int* 
   if (run_n > 0) { atomicAdd(&hist[cur], run_n); }
   __syncthreads();
   const int c    = hist[tid];
-  const int incl = block_scan_incl(c, wave_tot);
+  const int incl = scan_incl_t<kThreads>(c, wave_tot);
   if (incl - c < st.rank && st.rank <= incl) {
     *sel_digit = uint32_t(tid);
     *sel_rank  = st.rank - (incl - c);
@@ -1596,7 +1574,7 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
   extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];
   auto* key = reinterpret_cast<uint64_t*>(dyn);                 // [cap]
   auto* rid = reinterpret_cast<uint32_t*>(dyn + size_t(cap) * 8);  // [cap]
-  auto* qv  = reinterpret_cast<double*>(dyn + size_t(cap) * 12);  // [dim]
+  auto* qv  = reinterpret_cast<double*>(dyn + size_t(cap) * 12);  // [query_coords]
   __shared__ int hist[257];
   __shared__ int wave_tot[4];
   __shared__ uint32_t red[48];
@@ -1614,7 +1592,15 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
   const int tid   = threadIdx.x;
   const int k     = a.k;
   const int64_t qr = a.query_rows != nullptr ? int64_t(a.query_rows[q]) : q;
-  for (int64_t j = tid; j < a.dim; j += kThreads) { qv[j] = fcoord(a.queries, a.t, qr * a.dim + j); }
+  const int64_t qn = query_coords(L, a.dim);
+  for (int64_t j = tid; j < qn; j += kThreads) {
+    qv[j] = j < a.dim ? fcoord(a.queries, a.t, qr * a.dim + j) : 0.0;
+  }
+  double qq = 0;
+  if (a.metric == metric_kind::cosine) {
+    __syncthreads();
+    qq = query_square(qv, qn);
+  }
 
   const int64_t n_cand =
     a.all_rows ? a.n_rows : (a.cand_count[q] < a.cap ? int64_t(a.cand_count[q]) : a.cap);
@@ -1628,7 +1614,7 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
   int64_t n_scored = 0;
   auto score       = [&](int from, int to) {
     n_scored += to - from;
-    score_rows_l<L>(qv, a.vectors, a.t, a.dim, a.metric, rid, key, from, to);
+    score_rows_l<L, kThreads>(qv, qq, a.vectors, a.t, a.dim, a.metric, rid, key, from, to);
   };
   int have = 0;  // entries [0, have) of key / rid are scored
   // the k best so far move to [0, k) (unordered); the k-th key bounds the k-th score. With
@@ -1878,9 +1864,10 @@ void verify_topk_f(const verify_f_args& a, hipStream_t stream)
   int cap = (3 * a.k / 2 + 255) / 256 * 256;
   cap     = cap > pow2_ge(a.k) ? cap : pow2_ge(a.k);
   cap     = cap > 1024 ? (cap < kBuf ? cap : kBuf) : 1024;
-  const size_t bytes  = size_t(cap) * 12 + size_t(a.dim) * 8;
+  const int L         = score_lanes(a.dim);
+  const size_t bytes  = size_t(cap) * 12 + size_t(query_coords(L, a.dim)) * 8;
   const unsigned grid = unsigned(a.nq);
-  switch (score_lanes(a.dim)) {
+  switch (L) {
     case 16: launch_dyn(verify_topk_f_kernel<16>, grid, bytes, stream, a, cap); break;
     case 32: launch_dyn(verify_topk_f_kernel<32>, grid, bytes, stream, a, cap); break;
     default: launch_dyn(verify_topk_f_kernel<64>, grid, bytes, stream, a, cap); break;

@@ -72,6 +72,20 @@ def test_dims_and_ragged(gpu):
         check(X, Q, 17, "l2", D, I)
 
 
+@pytest.mark.parametrize("metric", ["l2", "ip", "cosine"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_scoring_slots(gpu, dtype, metric):
+    """Exact scores at the edges of the re-rank's row slots (16, 32 and 64 lanes; partials per lane
+    4, 2 and 1; 128 or 256 coordinates per load): equal to the oracle's, bit for bit."""
+    for d in (1, 2, 3, 63, 64, 65, 126, 127, 128, 129, 130, 192, 255, 256, 257, 320, 511, 513, 770):
+        X, Q = correlated(701, d, 9, seed=d, scale_norms=True)
+        Xt, Qt = torch.from_numpy(X).to(dtype), torch.from_numpy(Q).to(dtype)
+        idx = certex.Index(d, metric=metric)
+        idx.add(Xt.cuda())
+        D, I = idx.search(Qt.cuda(), k=37)
+        check(Xt.float().numpy(), Qt.float().numpy(), 37, metric, D.cpu().numpy(), I.cpu().numpy())
+
+
 def test_inner_product_unequal_norms(gpu):
     X, Q = correlated(20_000, 64, 500, scale_norms=True)
     D, I, _ = run(X, Q, 10, "ip")
