@@ -6,6 +6,9 @@
 // the screen is exact; the row term folds the norm (l2) or the shift correction (inner product).
 
 #include "../kernels.hpp"
+#include "lanes.hpp"
+
+#include <type_traits>
 
 namespace certex_amd {
 namespace {
@@ -16,74 +19,57 @@ inline unsigned blocks_for(int64_t n, int block = 256)
 }
 
 /**
- * One thread per 16-byte chunk of a stored row (row_bytes / 16 = 8 or 16 consecutive lanes per
- * row), so that the reads of the input rows and the writes of the codes are coalesced; the
- * chunks' partial norms and sums meet by shuffles within the row's lanes.
+ * Bytes [j0, j0 + 16) of a row of dim bytes as int8 codes (zero past dim) in four words. A whole
+ * chunk is one 16-byte load whatever the row's alignment (memory accesses of any alignment are
+ * enabled on these devices); only the chunk that crosses the row's end goes byte by byte.
  */
-__global__ void encode_rows_kernel(const uint8_t* x, int64_t n, int64_t dim, int row_bytes,
-                                   uint8_t flip, metric_kind metric, int8_t* codes, int32_t* rowc)
+__device__ __forceinline__ void code_chunk(const uint8_t* row, int64_t dim, int64_t j0, uint8_t flip,
+                                           int (&w)[4])
 {
-  const int cpr   = row_bytes / 16;  // a power of two that divides 64
-  const int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  const int64_t r = t / cpr;
-  const int c     = int(t % cpr);
-  int norm = 0, sum = 0;
-  if (r < n) {
-    uint8_t v[16];
-    const int64_t j0 = int64_t(c) * 16;
-    if (dim % 16 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && j0 < dim) {
-      *reinterpret_cast<int4*>(v) = *reinterpret_cast<const int4*>(x + r * dim + j0);
-    } else {
+  if (j0 + 16 <= dim) {
+    __builtin_memcpy(w, row + j0, 16);
+    const uint32_t f = uint32_t(flip) * 0x01010101u;
 #pragma unroll
-      for (int b = 0; b < 16; ++b) { v[b] = j0 + b < dim ? x[r * dim + j0 + b] : uint8_t(0); }
-    }
-    int8_t out[16];
+    for (int i = 0; i < 4; ++i) { w[i] = int(uint32_t(w[i]) ^ f); }
+    return;
+  }
+  uint8_t v[16];
 #pragma unroll
-    for (int b = 0; b < 16; ++b) {
-      const int code = j0 + b < dim ? int(int8_t(v[b] ^ flip)) : 0;
-      out[b]         = int8_t(code);
-      norm += code * code;
-      sum += code;
-    }
-    *reinterpret_cast<int4*>(codes + r * row_bytes + j0) = *reinterpret_cast<const int4*>(out);
-  }
-  for (int off = 1; off < cpr; off <<= 1) {
-    norm += __shfl_xor(norm, off);
-    sum += __shfl_xor(sum, off);
-  }
-  if (r < n && c == 0) {
-    rowc[r] = metric == metric_kind::l2 ? -(norm >> 1) : (flip ? 128 * sum : 0);
-  }
+  for (int b = 0; b < 16; ++b) { v[b] = j0 + b < dim ? uint8_t(row[j0 + b] ^ flip) : uint8_t(0); }
+  __builtin_memcpy(w, v, 16);
 }
 
 /**
- * The rows of more than 256 bytes (row_bytes a multiple of 256): one wave per row, lane l on the
- * 16-byte chunks l, l + 64, ...; the row's norm and sum meet by shuffles over the wave.
+ * Stored rows of integer vectors: CPR consecutive lanes per row, lane c on the 16-byte chunks c,
+ * c + CPR, ... of the row (CPR = 8 and 16: rows of 128 and 256 bytes, one chunk per lane; 16 also
+ * for wider rows, whose rows are multiples of 256 bytes). The row's norm and sum meet by a
+ * butterfly over its lanes. Memory-bound: 250,000 x 960 bytes (0.5 GB read and written) 290 -> 86
+ * us, 5.8 TB/s (a wave per row and byte loads before).
  */
-__global__ void encode_rows_wide_kernel(const uint8_t* x, int64_t n, int64_t dim, int row_bytes,
-                                        uint8_t flip, metric_kind metric, int8_t* codes, int32_t* rowc)
+template <int CPR>
+__global__ __launch_bounds__(256) void encode_rows_kernel(const uint8_t* x, int64_t n, int64_t dim, int row_bytes,
+                                                          uint8_t flip, metric_kind metric, int8_t* codes,
+                                                          int32_t* rowc)
 {
-  const int64_t r = (blockIdx.x * int64_t(blockDim.x) + threadIdx.x) >> 6;
-  const int lane  = threadIdx.x & 63;
-  if (r >= n) { return; }  // whole waves leave together (64 divides the block)
+  const int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  const int64_t r = t / CPR;
+  const int c     = int(t % CPR);
   int norm = 0, sum = 0;
-  for (int c = lane; c < row_bytes / 16; c += 64) {
-    const int64_t j0 = int64_t(c) * 16;
-    int8_t out[16];
+  if (r < n) {
+    for (int j = c; j < row_bytes / 16; j += CPR) {
+      int w[4];
+      code_chunk(x + r * dim, dim, int64_t(j) * 16, flip, w);
 #pragma unroll
-    for (int b = 0; b < 16; ++b) {
-      const int code = j0 + b < dim ? int(int8_t(x[r * dim + j0 + b] ^ flip)) : 0;
-      out[b]         = int8_t(code);
-      norm += code * code;
-      sum += code;
+      for (int i = 0; i < 4; ++i) {
+        norm = __builtin_amdgcn_sdot4(w[i], w[i], norm, false);
+        sum  = __builtin_amdgcn_sdot4(w[i], 0x01010101, sum, false);
+      }
+      *reinterpret_cast<int4*>(codes + r * row_bytes + int64_t(j) * 16) = int4{w[0], w[1], w[2], w[3]};
     }
-    *reinterpret_cast<int4*>(codes + r * row_bytes + j0) = *reinterpret_cast<const int4*>(out);
   }
-  for (int off = 1; off < 64; off <<= 1) {
-    norm += __shfl_xor(norm, off);
-    sum += __shfl_xor(sum, off);
-  }
-  if (lane == 0) { rowc[r] = metric == metric_kind::l2 ? -(norm >> 1) : (flip ? 128 * sum : 0); }
+  norm = lanes::sum<CPR>(norm);
+  sum  = lanes::sum<CPR>(sum);
+  if (r < n && c == 0) { rowc[r] = metric == metric_kind::l2 ? -(norm >> 1) : (flip ? 128 * sum : 0); }
 }
 
 __global__ void encode_queries_kernel(const uint8_t* q, const int32_t* rows, int64_t nq,
@@ -144,19 +130,11 @@ __device__ inline double coord(const void* p, elem t, int64_t i)
                         : double(static_cast<const _Float16*>(p)[i]);
 }
 
-/** Euclidean norm of row i (1 when zero) for unit normalisation, fp64 in coordinate order. */
-__device__ inline double row_norm(const void* x, elem t, int64_t i, int64_t dim)
-{
-  double s = 0;
-  for (int64_t j = 0; j < dim; ++j) {
-    const double v = coord(x, t, i * dim + j);
-    s              = fma(v, v, s);
-  }
-  return s > 0 ? sqrt(s) : 1.0;
-}
-
+/** *p = max(*p, v) for non-negative doubles: a plain atomic on one word takes about 10 ns of every
+ *  workgroup's turn, so a workgroup whose value cannot raise it only reads it. */
 __device__ inline void atomic_max_pos(double* p, double v)
 {
+  if (!(v > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) { return; }
   // non-negative doubles order like their bit patterns
   atomicMax(reinterpret_cast<unsigned long long*>(p), (unsigned long long)__double_as_longlong(v));
 }
@@ -165,23 +143,6 @@ __device__ inline void atomic_max_pos(double* p, double v)
 __device__ inline double sqrt_up(double s, int64_t terms)
 {
   return sqrt(s * (1.0 + 4e-16 * double(terms + 4))) * (1.0 + 4e-16);
-}
-
-__global__ void column_sums_kernel(const void* x, elem t, int64_t n, int64_t dim, bool normalize,
-                                   int64_t rows_per_block, double* sums)
-{
-  __shared__ double nrm[512];
-  const int64_t r0 = blockIdx.x * rows_per_block;
-  const int64_t r1 = r0 + rows_per_block < n ? r0 + rows_per_block : n;
-  for (int64_t i = r0 + threadIdx.x; i < r1; i += blockDim.x) {
-    nrm[i - r0] = normalize ? row_norm(x, t, i, dim) : 1.0;
-  }
-  __syncthreads();
-  for (int64_t j = threadIdx.x; j < dim; j += blockDim.x) {
-    double s = 0;
-    for (int64_t i = r0; i < r1; ++i) { s += coord(x, t, i * dim + j) / nrm[i - r0]; }
-    atomicAdd(sums + j, s);
-  }
 }
 
 constexpr double kF16Safe = 4096.0;  // |Z| above this: the row is always a candidate
@@ -194,12 +155,7 @@ __device__ inline _Float16 to_f16(double z)
 }
 
 /** Sum of v over the 64 lanes of a wave (xor butterfly: every lane gets the sum). */
-__device__ inline double wave_sum(double v)
-{
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) { v += __shfl_xor(v, off); }
-  return v;
-}
+__device__ inline double wave_sum(double v) { return lanes::sum<64>(v); }
 
 /** A lane's coordinates of one row loaded together: j = j0 + 64 u + lane, u < kLaneChunk. */
 constexpr int kLaneChunk = 16;
@@ -260,129 +216,315 @@ __device__ inline double wave_row_norm(const void* x, elem t, int64_t i, int64_t
 }
 
 /**
- * out[0] raised to the largest |x / |x| - center| (|x - center| without normalizing) over the n
- * rows, sqrt_up of the fp64 sum: rows by waves over a grid stride as encode_rows_f16_kernel takes
- * them, one atomic per workgroup.
+ * The kernels over the rows of a build or an addition (column_sums, max_norm, encode_rows_f16): G
+ * lanes per row, 64 / G rows per wave, lane g of a row on the coordinates 4 (u G + g) .. + 3, u < N
+ * (one vector load of 4 coordinates each, N of them in flight). (G, N) is sized so that one slice
+ * of 4 G N coordinates covers the row (dim up to 1,024); wider rows (MULTI) take slice after slice.
+ * Bound by memory, or for small builds by latency and the workgroups' atomics. A wave per row with
+ * 16 coordinates per lane loaded 1,024 coordinates of a row of 64. 131,072 fp16 rows of 64: encoding
+ * 229 -> 14 us, max_norm 117 -> 10 us; 60,000 x 300 float32, cosine: 163 -> 39 and 93 -> 24 us.
  */
-__global__ __launch_bounds__(256) void max_norm_kernel(const void* x, elem t, int64_t n,
-                                                       int64_t dim, bool normalize,
-                                                       const double* center, double* out)
+constexpr int kRowThreads = 1024;  // of max_norm and encode_rows_f16: few workgroups, few atomics
+
+template <typename T, int N>
+struct row_slice {
+  T v[N][4];
+};
+
+/** Coordinates of `row` from j0 on for lane g: a whole group of 4 is one load whatever the row's
+ *  alignment, the group that crosses the row's end goes one by one; zero past dim. */
+template <typename T, int G, int N>
+__device__ __forceinline__ row_slice<T, N> load_slice(const T* row, int64_t dim, int64_t j0, int g)
 {
-  __shared__ double wmax[4];
-  const int lane      = threadIdx.x & 63;
-  const int wave      = threadIdx.x >> 6;
-  const int64_t waves = int64_t(gridDim.x) * 4;
-  double m            = 0;
-  for (int64_t i = blockIdx.x * int64_t(4) + wave; i < n; i += waves) {
-    const double nrm = normalize ? wave_row_norm(x, t, i, dim, lane) : 1.0;
-    double s         = 0;
-    for (int64_t j0 = 0; j0 < dim; j0 += 64 * kLaneChunk) {
-      double v[kLaneChunk], c[kLaneChunk];
-      lane_coords(x, t, i, dim, j0, lane, v);
-      lane_center(center, dim, j0, lane, c);
+  row_slice<T, N> s;
 #pragma unroll
-      for (int u = 0; u < kLaneChunk; ++u) {
-        if (j0 + 64 * u + lane < dim) {
-          const double z = v[u] / nrm - c[u];
-          s              = fma(z, z, s);
-        }
-      }
+  for (int u = 0; u < N; ++u) {
+    const int64_t j = j0 + 4 * (u * G + g);
+    if (j + 4 <= dim) {
+      __builtin_memcpy(s.v[u], row + j, 4 * sizeof(T));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { s.v[u][e] = j + e < dim ? row[j + e] : T(0); }
     }
-    m = fmax(m, sqrt_up(wave_sum(s), dim));
   }
-  if (lane == 0) { wmax[wave] = m; }
-  __syncthreads();
-  if (threadIdx.x == 0) { atomic_max_pos(out, fmax(fmax(wmax[0], wmax[1]), fmax(wmax[2], wmax[3]))); }
+  return s;
+}
+
+/** The center's coordinates of a slice (any value past dim). */
+template <int G, int N>
+__device__ __forceinline__ void center_slice(const double* center, int64_t dim, int64_t j0, int g, double (&c)[N][4])
+{
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int64_t j = j0 + 4 * (u * G + g) + e;
+      c[u][e]         = center[j < dim ? j : dim - 1];
+    }
+  }
+}
+
+/** A row's norm and its reciprocal, for quotients. */
+struct unit_scale {
+  double nrm, inv;
+};
+
+/** v / |x|: the product with the reciprocal and one correction of its remainder, which rounds the
+ *  quotient as the division does but for rare last bits, at a fifth of its instructions. */
+__device__ __forceinline__ double unit_coord(double v, const unit_scale& s)
+{
+  const double q = v * s.inv;
+  const double r = fma(-q, s.nrm, v);
+  return fma(r, s.inv, q);
+}
+
+/** |x| of a row (1 when zero) over its G lanes, from its slice (or, MULTI, slice after slice). */
+template <typename T, int G, int N, bool MULTI>
+__device__ __forceinline__ unit_scale row_scale(const row_slice<T, N>& first, const T* row, int64_t dim, int g)
+{
+  double s2 = 0;
+  row_slice<T, N> x = first;
+  for (int64_t j0 = 0;;) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { s2 = fma(double(x.v[u][e]), double(x.v[u][e]), s2); }
+    }
+    j0 += 4 * G * N;
+    if (!MULTI || j0 >= dim) { break; }
+    x = load_slice<T, G, N>(row, dim, j0, g);
+  }
+  s2 = lanes::sum<G>(s2);
+  unit_scale k;
+  k.nrm = s2 > 0 ? sqrt(s2) : 1.0;
+  k.inv = 1.0 / k.nrm;
+  return k;
 }
 
 /**
- * Rows i = w, w + W, ... for wave w of W (a grid stride), each by one wave whose lanes take the
- * coordinates j = lane, lane + 64, ... (coalesced loads and stores): rows[i] = fp16(Z) with
- * Z = (x / |x| - center) / alpha (x / |x| when normalizing), subnormals set to 0, zero padded;
- * rowc[i] = -|Z|^2 / 2, raised so that it bounds the term's fp32 accumulation (0 for the inner
- * product); a row with |Z| above kF16Safe is stored as zeros with rowc = +inf (always a
- * candidate). maxima[0] and maxima[1] are raised to the largest |fp16(Z)| and |Z - fp16(Z)|
- * (sqrt_up of their sums), one atomic each per workgroup. The fp64 sums are per-lane partials
- * and a butterfly; they only enter bounds that carry their rounding slack.
+ * sums[j] += the column sums of the rows (of x / |x| when NORM): each wave keeps its lanes' columns
+ * in registers over its rows; the block's waves meet in LDS and add each column with one atomic.
+ * MULTI (dim above 1,024): the block's wave w takes the columns of slice w of every row of the block.
+ * 60,000 x 300 float32 rows, cosine: 845 -> 35 us (a thread per column and serial row norms before).
  */
-__global__ __launch_bounds__(256) void encode_rows_f16_kernel(const void* x, elem t, int64_t n,
-                                                              int64_t dim, int halves,
-                                                              bool normalize, const double* center,
-                                                              double inv_alpha, metric_kind metric,
-                                                              double gamma, uint16_t* rows,
-                                                              float* rowc, double* maxima)
+template <typename T, int G, int N, bool NORM, bool MULTI>
+__global__ __launch_bounds__(256) void column_sums_kernel(const T* x, int64_t n, int64_t dim, double* sums)
 {
-  __shared__ double wmax[2][4];
-  const int lane      = threadIdx.x & 63;
-  const int wave      = threadIdx.x >> 6;
-  const int64_t waves = int64_t(gridDim.x) * 4;
-  double mh = 0, me = 0;  // this wave's largest bounds of |fp16(Z)| and |Z - fp16(Z)|
-  for (int64_t i = blockIdx.x * int64_t(4) + wave; i < n; i += waves) {
-    _Float16* dst    = reinterpret_cast<_Float16*>(rows + i * halves);
-    const double nrm = normalize ? wave_row_norm(x, t, i, dim, lane) : 1.0;
-    double a         = 0;
-    for (int64_t j0 = 0; j0 < dim; j0 += 64 * kLaneChunk) {
-      double v[kLaneChunk], c[kLaneChunk];
-      lane_coords(x, t, i, dim, j0, lane, v);
-      lane_center(center, dim, j0, lane, c);
+  constexpr int RPW = 64 / G;
+  constexpr int C   = 4 * G * N;  // columns of a slice
+  __shared__ double part[MULTI ? 1 : 4 * C];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane % G, slot = lane / G;
+  const int64_t col0  = MULTI ? int64_t(wave) * C : 0;
+  const int64_t first = MULTI ? int64_t(blockIdx.x) : (blockIdx.x * int64_t(4) + wave) * RPW;
+  const int64_t step  = MULTI ? int64_t(gridDim.x) : int64_t(gridDim.x) * 4 * RPW;
+  double acc[N][4] = {};
+  if (col0 < dim) {
+    for (int64_t i0 = first; i0 < n; i0 += step) {
+      const int64_t i = i0 + slot;
+      const bool live = i < n;
+      const T* row    = x + (live ? i : n - 1) * dim;
+      const auto v    = load_slice<T, G, N>(row, dim, col0, g);
+      unit_scale k{1.0, 1.0};
+      if constexpr (NORM) {
+        k = row_scale<T, G, N, MULTI>(MULTI ? load_slice<T, G, N>(row, dim, 0, g) : v, row, dim, g);
+      }
 #pragma unroll
-      for (int u = 0; u < kLaneChunk; ++u) {
-        if (j0 + 64 * u + lane < dim) {
-          const double z = (v[u] / nrm - c[u]) * inv_alpha;
-          a              = fma(z, z, a);
+      for (int u = 0; u < N; ++u) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const double d = double(v.v[u][e]);
+          acc[u][e] += live ? (NORM ? unit_coord(d, k) : d) : 0.0;
         }
       }
     }
-    a = wave_sum(a);  // the same value in every lane: the branch below is uniform
-    if (!(sqrt(a) <= kF16Safe)) {
-      for (int64_t j = lane; j < halves; j += 64) { dst[j] = _Float16(0.0f); }
-      if (lane == 0) { rowc[i] = INFINITY; }
-      continue;
-    }
-    double nz = 0, ez = 0;
-    for (int64_t j0 = 0; j0 < dim; j0 += 64 * kLaneChunk) {
-      double v[kLaneChunk], c[kLaneChunk];
-      lane_coords(x, t, i, dim, j0, lane, v);
-      lane_center(center, dim, j0, lane, c);
+  }
 #pragma unroll
-      for (int u = 0; u < kLaneChunk; ++u) {
-        const int64_t j = j0 + 64 * u + lane;
-        if (j < dim) {
-          const double z   = (v[u] / nrm - c[u]) * inv_alpha;
-          const _Float16 h = to_f16(z);
-          const double e   = z - double(h);  // exact (Sterbenz, or h = 0)
-          dst[j]           = h;
-          nz               = fma(double(h), double(h), nz);
-          ez               = fma(e, e, ez);
-        }
-      }
-    }
-    for (int64_t j = dim + lane; j < halves; j += 64) { dst[j] = _Float16(0.0f); }
-    nz = wave_sum(nz);
-    ez = wave_sum(ez);
-    if (lane == 0) {
-      if (metric == metric_kind::inner) {
-        rowc[i] = 0.0f;
+  for (int u = 0; u < N; ++u) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int j = 4 * (u * G + g) + e;
+      if constexpr (MULTI) {
+        if (col0 + j < dim) { atomicAdd(sums + col0 + j, acc[u][e]); }
       } else {
-        // row term rounded up: the fp32 accumulation error of this term is folded in (factor
-        // 1 - 2g)
-        const double c = -(a * (1.0 - 1e-13) / 2.0) * (1.0 - 2.0 * gamma - 1e-10);
-        float f        = float(c);
-        if (double(f) < c) { f = nextafterf(f, INFINITY); }
+        double a = acc[u][e];
+        if constexpr (G <= 16) { a += lanes::exchange<16>(a); }
+        if constexpr (G <= 32) { a += lanes::exchange<32>(a); }
+        if (slot == 0) { part[wave * C + j] = a; }
+      }
+    }
+  }
+  if constexpr (!MULTI) {
+    __syncthreads();
+    for (int j = threadIdx.x; j < C && j < dim; j += 256) {
+      atomicAdd(sums + j, (part[j] + part[C + j]) + (part[2 * C + j] + part[3 * C + j]));
+    }
+  }
+}
+
+/**
+ * out[0] raised to the largest |x / |x| - center| (|x - center| without NORM) over the n rows,
+ * sqrt_up of the largest fp64 sum, one atomic per workgroup.
+ */
+template <typename T, int G, int N, bool NORM, bool MULTI>
+__global__ __launch_bounds__(kRowThreads) void max_norm_kernel(const T* x, int64_t n, int64_t dim,
+                                                       const double* center, double* out)
+{
+  constexpr int RPW = 64 / G;
+  constexpr int C   = 4 * G * N;
+  __shared__ double wmax[kRowThreads / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane % G, slot = lane / G;
+  double c[N][4];
+  if constexpr (!MULTI) { center_slice<G, N>(center, dim, 0, g, c); }
+  double m = 0;
+  for (int64_t i0 = (blockIdx.x * int64_t(kRowThreads / 64) + wave) * RPW; i0 < n;
+       i0 += int64_t(gridDim.x) * (kRowThreads / 64) * RPW) {
+    const int64_t i = i0 + slot < n ? i0 + slot : n - 1;
+    const T* row    = x + i * dim;
+    auto v          = load_slice<T, G, N>(row, dim, 0, g);
+    unit_scale k{1.0, 1.0};
+    if constexpr (NORM) { k = row_scale<T, G, N, MULTI>(v, row, dim, g); }
+    double s = 0;
+    for (int64_t j0 = 0;;) {
+      if constexpr (MULTI) { center_slice<G, N>(center, dim, j0, g, c); }
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const double d = double(v.v[u][e]);
+          const double z = (NORM ? unit_coord(d, k) : d) - c[u][e];
+          s              = j0 + 4 * (u * G + g) + e < dim ? fma(z, z, s) : s;
+        }
+      }
+      j0 += C;
+      if (!MULTI || j0 >= dim) { break; }
+      v = load_slice<T, G, N>(row, dim, j0, g);
+    }
+    m = fmax(m, lanes::sum<G>(s));
+  }
+  m = lanes::max<64>(m);
+  if (lane == 0) { wmax[wave] = m; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kRowThreads / 64; ++w) { m = fmax(m, wmax[w]); }
+    atomic_max_pos(out, sqrt_up(m, dim));
+  }
+}
+
+/**
+ * rows[i] = fp16(Z) with Z = (x / |x| - center) / alpha (x / |x| with NORM), subnormals set to 0,
+ * zero padded; rowc[i] = -|Z|^2 / 2, raised so that it bounds the term's fp32 accumulation (0 for
+ * the inner product); a row with |Z| above kF16Safe is stored as zeros with rowc = +inf (always a
+ * candidate). maxima[0] and maxima[1] are raised to the largest |fp16(Z)| and |Z - fp16(Z)|
+ * (sqrt_up of the largest sums), one atomic each per workgroup. The fp64 sums are per-lane partials
+ * and a butterfly; they only enter bounds that carry their rounding slack. A row that one slice
+ * covers is read once and encoded from registers; wider rows (MULTI) are read again for the sums
+ * before they are stored.
+ */
+template <typename T, int G, int N, bool NORM, bool MULTI>
+__global__ __launch_bounds__(kRowThreads) void encode_rows_f16_kernel(const T* x, int64_t n, int64_t dim, int halves,
+                                                              const double* center, double inv_alpha,
+                                                              metric_kind metric, double gamma,
+                                                              uint16_t* rows, float* rowc, double* maxima)
+{
+  constexpr int RPW = 64 / G;
+  constexpr int C   = 4 * G * N;
+  __shared__ double wmax[2][kRowThreads / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane % G, slot = lane / G;
+  double c[N][4];
+  if constexpr (!MULTI) { center_slice<G, N>(center, dim, 0, g, c); }
+  double mh = 0, me = 0;  // the largest sums of fp16(Z)^2 and (Z - fp16(Z))^2
+  for (int64_t i0 = (blockIdx.x * int64_t(kRowThreads / 64) + wave) * RPW; i0 < n;
+       i0 += int64_t(gridDim.x) * (kRowThreads / 64) * RPW) {
+    const int64_t i = i0 + slot;
+    const bool live = i < n;
+    const T* row    = x + (live ? i : n - 1) * dim;
+    auto v          = load_slice<T, G, N>(row, dim, 0, g);
+    unit_scale k{1.0, 1.0};
+    if constexpr (NORM) { k = row_scale<T, G, N, MULTI>(v, row, dim, g); }
+    double a = 0, nz = 0, ez = 0;
+    _Float16 h[N][4];
+    for (int64_t j0 = 0;;) {
+      if constexpr (MULTI) { center_slice<G, N>(center, dim, j0, g, c); }
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const bool in  = j0 + 4 * (u * G + g) + e < dim;
+          const double d = double(v.v[u][e]);
+          const double z = in ? ((NORM ? unit_coord(d, k) : d) - c[u][e]) * inv_alpha : 0.0;
+          h[u][e]        = to_f16(z);
+          const double r = z - double(h[u][e]);  // exact (Sterbenz, or h = 0)
+          a  = fma(z, z, a);
+          nz = fma(double(h[u][e]), double(h[u][e]), nz);
+          ez = fma(r, r, ez);
+        }
+      }
+      j0 += C;
+      if (!MULTI || j0 >= dim) { break; }
+      v = load_slice<T, G, N>(row, dim, j0, g);
+    }
+    a  = lanes::sum<G>(a);  // the same value in the lanes of a row
+    nz = lanes::sum<G>(nz);
+    ez = lanes::sum<G>(ez);
+    const bool safe = a <= kF16Safe * kF16Safe;  // false for a NaN too
+    if (safe) {
+      mh = fmax(mh, nz);
+      me = fmax(me, ez);
+    }
+    if (live) {
+      _Float16* dst = reinterpret_cast<_Float16*>(rows + i * halves);
+      for (int64_t j0 = 0;;) {
+        if constexpr (MULTI) {  // this slice again
+          v = load_slice<T, G, N>(row, dim, j0, g);
+          center_slice<G, N>(center, dim, j0, g, c);
+        }
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+          const int64_t j = j0 + 4 * (u * G + g);
+          if constexpr (MULTI) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const double d = double(v.v[u][e]);
+              h[u][e] = to_f16(j + e < dim ? ((NORM ? unit_coord(d, k) : d) - c[u][e]) * inv_alpha : 0.0);
+            }
+          }
+          _Float16 o[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { o[e] = safe ? h[u][e] : _Float16(0.0f); }
+          if (j < halves) { __builtin_memcpy(__builtin_assume_aligned(dst + j, 8), o, 8); }
+        }
+        j0 += C;
+        if (!MULTI || j0 >= halves) { break; }
+      }
+      if (g == 0) {
+        float f = INFINITY;
+        if (safe && metric == metric_kind::inner) {
+          f = 0.0f;
+        } else if (safe) {
+          // row term rounded up: the fp32 accumulation error of this term is folded in (factor
+          // 1 - 2g)
+          const double t = -(a * (1.0 - 1e-13) / 2.0) * (1.0 - 2.0 * gamma - 1e-10);
+          f              = float(t);
+          if (double(f) < t) { f = nextafterf(f, INFINITY); }
+        }
         rowc[i] = f;
       }
     }
-    mh = fmax(mh, sqrt_up(nz, dim));
-    me = fmax(me, sqrt_up(ez, dim));
   }
+  mh = lanes::max<64>(mh);
+  me = lanes::max<64>(me);
   if (lane == 0) {
     wmax[0][wave] = mh;
     wmax[1][wave] = me;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    atomic_max_pos(maxima + 0, fmax(fmax(wmax[0][0], wmax[0][1]), fmax(wmax[0][2], wmax[0][3])));
-    atomic_max_pos(maxima + 1, fmax(fmax(wmax[1][0], wmax[1][1]), fmax(wmax[1][2], wmax[1][3])));
+  if (threadIdx.x < 2) {  // thread 0: the rows' norms, thread 1: their rounding errors
+    double m = wmax[threadIdx.x][0];
+    for (int w = 1; w < kRowThreads / 64; ++w) { m = fmax(m, wmax[threadIdx.x][w]); }
+    atomic_max_pos(maxima + threadIdx.x, sqrt_up(m, dim));
   }
 }
 
@@ -486,21 +628,85 @@ __global__ void remove_f_kernel(const int64_t* ids, int64_t n, int64_t size, flo
 
 }  // namespace
 
+namespace {
+
+/**
+ * f(T{}, integral G, integral N, bool_constant NORM, bool_constant MULTI, rows per wave) for the
+ * row kernels: 16 lanes per row up to 64 coordinates, 32 up to 128, whole waves above, with as
+ * many groups of 4 per lane as cover the row (at most 4: 1,024 coordinates per slice).
+ */
+template <typename T, bool NORM, typename F>
+void with_shape(int64_t dim, F&& f)
+{
+  using std::integral_constant;
+  const auto go = [&](auto g, auto nn, auto multi) {
+    f(T{}, g, nn, std::bool_constant<NORM>{}, multi);
+  };
+  if (dim <= 64) {
+    go(integral_constant<int, 16>{}, integral_constant<int, 1>{}, std::false_type{});
+  } else if (dim <= 128) {
+    go(integral_constant<int, 32>{}, integral_constant<int, 1>{}, std::false_type{});
+  } else if (dim <= 256) {
+    go(integral_constant<int, 64>{}, integral_constant<int, 1>{}, std::false_type{});
+  } else if (dim <= 512) {
+    go(integral_constant<int, 64>{}, integral_constant<int, 2>{}, std::false_type{});
+  } else if (dim <= 768) {
+    go(integral_constant<int, 64>{}, integral_constant<int, 3>{}, std::false_type{});
+  } else if (dim <= 1024) {
+    go(integral_constant<int, 64>{}, integral_constant<int, 4>{}, std::false_type{});
+  } else {
+    go(integral_constant<int, 64>{}, integral_constant<int, 4>{}, std::true_type{});
+  }
+}
+
+template <typename F>
+void with_rows(elem t, bool normalize, int64_t dim, F&& f)
+{
+  if (t == elem::f32) {
+    normalize ? with_shape<float, true>(dim, f) : with_shape<float, false>(dim, f);
+  } else if (t == elem::bf16) {
+    normalize ? with_shape<__bf16, true>(dim, f) : with_shape<__bf16, false>(dim, f);
+  } else {
+    normalize ? with_shape<_Float16, true>(dim, f) : with_shape<_Float16, false>(dim, f);
+  }
+}
+
+/**
+ * Workgroups of a row kernel of `waves` waves with `rpw` rows each at a time: at most 512, which
+ * stride over the rest. Each ends with atomics on the same words: with 2,048 workgroups those took
+ * most of max_norm's 28 us over 131,072 rows of 64 fp16 (17 MB).
+ */
+unsigned row_blocks(int64_t n, int waves, int rpw)
+{
+  return unsigned(std::min<int64_t>((n + waves * rpw - 1) / (waves * rpw), 512));
+}
+
+}  // namespace
+
 void column_sums(const void* x, elem t, int64_t n, int64_t dim, bool normalize, double* sums,
                  hipStream_t stream)
 {
   if (n == 0) { return; }
-  const int64_t rows_per_block = 512;
-  const unsigned blocks        = unsigned((n + rows_per_block - 1) / rows_per_block);
-  column_sums_kernel<<<blocks, 128, 0, stream>>>(x, t, n, dim, normalize, rows_per_block, sums);
+  with_rows(t, normalize, dim, [&](auto v, auto g, auto nn, auto norm, auto multi) {
+    using T          = decltype(v);
+    constexpr int G  = decltype(g)::value, N = decltype(nn)::value;
+    constexpr bool Z = decltype(norm)::value, M = decltype(multi)::value;
+    const unsigned b = M ? unsigned(std::min<int64_t>(n, 512)) : row_blocks(n, 4, 64 / G);
+    column_sums_kernel<T, G, N, Z, M><<<b, 256, 0, stream>>>(static_cast<const T*>(x), n, dim, sums);
+  });
 }
 
 void max_norm(const void* x, elem t, int64_t n, int64_t dim, bool normalize, const double* center,
               double* out, hipStream_t stream)
 {
   if (n == 0) { return; }
-  const unsigned blocks = unsigned(std::min<int64_t>((n + 3) / 4, 4096));
-  max_norm_kernel<<<blocks, 256, 0, stream>>>(x, t, n, dim, normalize, center, out);
+  with_rows(t, normalize, dim, [&](auto v, auto g, auto nn, auto norm, auto multi) {
+    using T          = decltype(v);
+    constexpr int G  = decltype(g)::value, N = decltype(nn)::value;
+    constexpr bool Z = decltype(norm)::value, M = decltype(multi)::value;
+    max_norm_kernel<T, G, N, Z, M><<<row_blocks(n, kRowThreads / 64, 64 / G), kRowThreads, 0, stream>>>(static_cast<const T*>(x), n, dim,
+                                                                              center, out);
+  });
 }
 
 void encode_rows_f16(const void* x, elem t, int64_t n, int64_t dim, int halves, bool normalize,
@@ -508,10 +714,13 @@ void encode_rows_f16(const void* x, elem t, int64_t n, int64_t dim, int halves, 
                      uint16_t* rows, float* rowc, double* maxima, hipStream_t stream)
 {
   if (n == 0) { return; }
-  // four rows per workgroup at a time, at most 4,096 workgroups (16 per CU) striding over the rest
-  const unsigned blocks = unsigned(std::min<int64_t>((n + 3) / 4, 4096));
-  encode_rows_f16_kernel<<<blocks, 256, 0, stream>>>(x, t, n, dim, halves, normalize, center,
-                                                     inv_alpha, metric, gamma, rows, rowc, maxima);
+  with_rows(t, normalize, dim, [&](auto v, auto g, auto nn, auto norm, auto multi) {
+    using T          = decltype(v);
+    constexpr int G  = decltype(g)::value, N = decltype(nn)::value;
+    constexpr bool Z = decltype(norm)::value, M = decltype(multi)::value;
+    encode_rows_f16_kernel<T, G, N, Z, M><<<row_blocks(n, kRowThreads / 64, 64 / G), kRowThreads, 0, stream>>>(
+      static_cast<const T*>(x), n, dim, halves, center, inv_alpha, metric, gamma, rows, rowc, maxima);
+  });
 }
 
 void encode_queries_f16(const void* q, elem t, int64_t nq, int64_t nq_pad, int64_t dim,
@@ -548,13 +757,11 @@ void encode_rows_i8(const uint8_t* x, int64_t n, int64_t dim, int row_bytes, uin
                     metric_kind metric, int8_t* codes, int32_t* rowc, hipStream_t stream)
 {
   if (n == 0) { return; }
-  if (row_bytes > 256) {
-    encode_rows_wide_kernel<<<blocks_for(n * 64), 256, 0, stream>>>(x, n, dim, row_bytes, flip,
-                                                                   metric, codes, rowc);
-    return;
+  if (row_bytes == 128) {
+    encode_rows_kernel<8><<<blocks_for(n * 8), 256, 0, stream>>>(x, n, dim, row_bytes, flip, metric, codes, rowc);
+  } else {
+    encode_rows_kernel<16><<<blocks_for(n * 16), 256, 0, stream>>>(x, n, dim, row_bytes, flip, metric, codes, rowc);
   }
-  encode_rows_kernel<<<blocks_for(n * (row_bytes / 16)), 256, 0, stream>>>(x, n, dim, row_bytes,
-                                                                          flip, metric, codes, rowc);
 }
 
 void encode_queries_i8(const uint8_t* q, int64_t nq, int64_t nq_pad, int64_t dim, int row_bytes,

@@ -333,3 +333,56 @@ def test_fp16_certificate(gpu, kind, d, metric, k):
           f"gamma bound / accumulation error {WORST['accumulation']:.3g}, "
           f"(score - lb) / |score| {WORST['lower']:.3g}, (ub - score) / |score| {WORST['upper']:.3g}, "
           f"(U - kth) / |kth| {WORST['U']:.3g}")
+
+
+# --- the encoding of the rows at the edges of its kernels' shapes ---------------------------------
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.int8])
+@pytest.mark.parametrize("d", [1, 15, 16, 17, 127, 129, 255, 257, 301, 513, 1000, 4095])
+def test_int_row_encoding(gpu, dtype, d):
+    """Rows of any length and alignment (16-byte chunks that cross the row's end, the padding)."""
+    n = 1_003
+    X = data.uniform_int(n, d, seed=d, dtype=dtype)
+    idx = certex.Index(d, metric="l2")
+    idx.add(torch.from_numpy(X).cuda())
+    get = captured(lambda: idx.search(torch.from_numpy(X[:5]).cuda(), k=3))
+    codes = get("codes", np.int8, (n, int(get("row_bytes")))).astype(np.int64)
+    want = (X.view(np.uint8) ^ (0x80 if dtype == np.uint8 else 0)).view(np.int8).astype(np.int64)
+    assert np.array_equal(codes[:, :d], want) and not codes[:, d:].any()
+    assert np.array_equal(get("rowc", np.int32), -((want * want).sum(1) // 2))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("metric", ["l2", "ip", "cosine"])
+def test_float_row_encoding(gpu, dtype, metric):
+    """fp16 rows, row terms and their bounds against fp64 numpy, at the edges of the slices that the
+    row kernels take (64, 128, 256, ... 1,024 coordinates, and slice after slice above)."""
+    n = 1_003
+    for d in (1, 3, 4, 5, 63, 64, 65, 127, 129, 255, 257, 511, 513, 767, 769, 1023, 1025, 2101):
+        rng = np.random.default_rng(d)
+        Xt = torch.from_numpy(rng.standard_normal((n, d)).astype(np.float32) + np.float32(0.5)).to(dtype)
+        X = Xt.double().numpy()
+        if metric == "cosine":
+            X = X / np.sqrt((X * X).sum(1, keepdims=True))
+        idx = certex.Index(d, metric=metric)
+        idx.add(Xt.cuda())
+        get = captured(lambda: idx.search(Xt[:5].cuda(), k=3))
+        halves = int(get("halves"))
+        rows = get("codes", np.float16, (n, halves)).astype(np.float64)
+        rowc = get("rowc", np.float32).astype(np.float64)
+        nz, ez = get("maxima", np.float64)
+        alpha, gamma = np.sqrt(float(get("alpha2", np.float64)[0])), float(get("gamma", np.float64)[0])
+        c = np.zeros(d) if metric == "ip" else X.mean(0)
+        assert alpha == pytest.approx(np.sqrt(((X - c) ** 2).sum(1)).max() / 64, rel=1e-9)
+        Z = (X - c) / alpha
+        assert not rows[:, d:].any()
+        # fp16's rounding (2^-11 relative; values below its smallest normal become 0) and fp64's
+        assert (np.abs(rows[:, :d] - Z) <= 2.0**-11 * np.abs(Z) + 2.0**-14 + 1e-9).all()
+        assert np.sqrt((rows**2).sum(1)).max() <= nz * (1 + 1e-12)
+        assert np.sqrt(((rows[:, :d] - Z) ** 2).sum(1)).max() <= ez * (1 + 1e-9) + 1e-9
+        if metric == "ip":
+            assert not rowc.any()
+        else:
+            t = -(Z * Z).sum(1) / 2
+            assert (rowc >= t * (1 - 2 * gamma)).all() and (rowc <= t * (1 - 2 * gamma - 1e-6) + 1e-9).all()
