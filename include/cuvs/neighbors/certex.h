@@ -227,6 +227,14 @@ CUVS_EXPORT cuvsError_t cuvsCertexTimingEnd(double* ms, int64_t* launches);
 CUVS_EXPORT cuvsError_t cuvsCertexTimingShaderClock(double* mhz);
 
 /**
+ * Filter words of a boolean mask: entry e of `mask` (a dense uint8 device tensor of 1 or 2
+ * dimensions, entries in row-major order, any non-zero byte set) becomes bit e % 32 of word e / 32
+ * of `words` (a uint32 device vector of ceil(entries / 32)); the last word is zero past the mask.
+ * The packing that the reference's Python package does in torch (certex/index.py:99-104).
+ */
+CUVS_EXPORT cuvsError_t cuvsCertexPackMask(cuvsResources_t res, DLManagedTensor* mask, DLManagedTensor* words);
+
+/**
  * Free the scratch memory that searches on `res` have grown (device buffers and pinned host
  * staging), after waiting for its stream; later searches grow it again. The counterpart of the
  * reference's Python trim_pool (certex/index.py:165-169), which returns the unused memory of the

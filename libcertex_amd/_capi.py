@@ -161,6 +161,7 @@ def lib():
                     "cuvsCertexIndexGetLists": [P(IndexHandle), P(i32), P(i64)],
                     "cuvsCertexReserve": [ctypes.c_size_t, i64, P(IndexHandle)],
                     "cuvsCertexIndexListOrder": [ctypes.c_size_t, P(IndexHandle), P(DLManagedTensor)],
+                    "cuvsCertexPackMask": [ctypes.c_size_t, P(DLManagedTensor), P(DLManagedTensor)],
                     "cuvsCertexStatsBegin": [],
                     "cuvsCertexStatsEnd": [P(i64), P(i64), P(i64)],
                     "cuvsCertexTimingShaderClock": [P(ctypes.c_double)],

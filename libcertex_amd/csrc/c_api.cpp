@@ -636,6 +636,23 @@ cuvsError_t cuvsCertexIndexListOrder(cuvsResources_t res,
   });
 }
 
+cuvsError_t cuvsCertexPackMask(cuvsResources_t res, DLManagedTensor* mask, DLManagedTensor* words)
+{
+  return translate([=] {
+    auto& r = res_of(res);
+    certex::expects(mask != nullptr, "certex: a tensor argument is NULL");
+    const int ndim = mask->dl_tensor.ndim;
+    certex::expects(ndim == 1 || ndim == 2, "certex: a mask has one or two dimensions");
+    const auto* m = device_data<uint8_t>(mask, ndim, "the mask");
+    auto* w       = device_data<uint32_t>(words, 1, "the filter words");
+    int64_t n     = mask->dl_tensor.shape[0];
+    if (ndim == 2) { n *= mask->dl_tensor.shape[1]; }
+    certex::expects(words->dl_tensor.shape[0] == (n + 31) / 32,
+                    "certex: the filter words of n mask entries are ceil(n / 32) words");
+    certex_amd::pack_bits(m, n, w, static_cast<hipStream_t>(r.stream()));
+  });
+}
+
 cuvsError_t cuvsCertexStatsBegin(void)
 {
   return translate([] { certex::stats_begin(); });

@@ -133,6 +133,9 @@ struct row_places {
 void remove_rows_i8(const int64_t* ids, int64_t n, int64_t size, int32_t* rowc,
                     unsigned long long* newly_removed, const row_places& at, hipStream_t stream);
 
+/** Filter words of n boolean bytes: entry e is bit e % 32 of words[e / 32], zeros past n. */
+void pack_bits(const uint8_t* mask, int64_t n, uint32_t* words, hipStream_t stream);
+
 void fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t stream);
 void fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t stream);
 /** p[i] = first + i for i < n. */

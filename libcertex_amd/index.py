@@ -87,19 +87,21 @@ def _cast(t, dtype):
     return y
 
 
-_BIT_WEIGHTS = {}
-
-
 def _pack(mask):
     """A boolean mask, flattened row-major, as 32-bit filter words on the mask's device: entry e is
-    bit e % 32 of word e // 32 (the reference's layout, certex/index.py:99-104). Eight entries
-    become one byte by a weighted sum, and four consecutive bytes are read as one little-endian
-    word; the returned words are int32."""
+    bit e % 32 of word e // 32 (the reference's layout, certex/index.py:99-104), as int32 words. A
+    mask on the GPU is packed by the library; one on the host by tensor operations (eight entries
+    become one byte by a weighted sum, four bytes are read as one little-endian word)."""
+    if mask.is_cuda:
+        m = mask.to(torch.bool).contiguous()
+        words = torch.empty((m.numel() + 31) // 32, dtype=torch.int32, device=m.device)
+        if words.numel():
+            b, w = C.Borrowed(m, dtype_override=(C.kDLUInt, 8)), C.Borrowed(words, dtype_override=(C.kDLUInt, 32))
+            C.check(C.lib().cuvsCertexPackMask(C.resources(), b.ptr, w.ptr))
+        return words
     flat = mask.reshape(-1).to(torch.uint8)
     flat = torch.nn.functional.pad(flat, (0, (-flat.numel()) % 32))
-    w = _BIT_WEIGHTS.get(flat.device)
-    if w is None:
-        w = _BIT_WEIGHTS[flat.device] = torch.tensor([1 << b for b in range(8)], dtype=torch.int32, device=flat.device)
+    w = torch.tensor([1 << b for b in range(8)], dtype=torch.int32)
     octets = (flat.view(-1, 8).to(torch.int32) * w).sum(1).to(torch.uint8)
     return octets.contiguous().view(torch.int32)
 

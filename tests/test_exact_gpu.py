@@ -220,3 +220,22 @@ def test_small_and_large_buckets(gpu, k):
     Q = np.concatenate([near, far])[rng.permutation(64)]
     D, I, _ = run(X, Q, k)
     check(X, Q, k, "l2", D, I)
+
+
+@pytest.mark.parametrize("shape", [(1,), (15,), (16,), (17,), (31,), (32,), (33,), (1000,), (3, 37), (5, 64), (0, 9)])
+def test_filter_words_packed_on_the_gpu(gpu, shape):
+    """Entry e is bit e % 32 of word e / 32 and the last word is zero past the mask, for masks at
+    any alignment, for views, and for boolean bytes other than 1."""
+    from libcertex_amd.index import _pack
+
+    n = int(np.prod(shape))
+    m = np.random.default_rng(n).random(n + 1) < 0.5
+    want = np.packbits(m[1:], bitorder="little")
+    want = np.pad(want, (0, (-want.size) % 4)).view(np.uint32)
+    base = torch.from_numpy(m.astype(np.uint8) * 3).cuda().view(torch.bool)
+    got = _pack(base[1:].reshape(shape))
+    np.testing.assert_array_equal(got.cpu().numpy().view(np.uint32), want)
+    row = torch.from_numpy(m[1:]).cuda()
+    both = np.packbits(np.concatenate([m[1:], m[1:]]), bitorder="little")
+    np.testing.assert_array_equal(_pack(row.expand(2, n)).cpu().numpy().view(np.uint32),
+                                  np.pad(both, (0, (-both.size) % 4)).view(np.uint32))
