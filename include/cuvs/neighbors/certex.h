@@ -236,7 +236,8 @@ CUVS_EXPORT cuvsError_t cuvsCertexPackMask(cuvsResources_t res, DLManagedTensor*
 
 /**
  * Free the scratch memory that searches on `res` have grown (device buffers and pinned host
- * staging), after waiting for its stream; later searches grow it again. The counterpart of the
+ * staging), after waiting for its stream, and the pool of device memory that dropped indexes and
+ * scratch left on its device (at most 4 GiB); later calls allocate again. The counterpart of the
  * reference's Python trim_pool (certex/index.py:165-169), which returns the unused memory of the
  * device's stream-ordered pool.
  */

@@ -39,8 +39,8 @@ class resources {
   [[nodiscard]] auto device() const -> int;
   void sync() const;
   /** Free the scratch memory that the searches on these resources have grown (device slots and
-   *  pinned host staging), after waiting for the stream; later searches grow it again. The
-   *  counterpart of the reference's trim_pool (certex/index.py:165-169). */
+   *  pinned host staging), after waiting for the stream, and the device's pool of freed memory;
+   *  later calls allocate again. The counterpart of the reference's trim_pool (certex/index.py:165-169). */
   void trim() const;
   /** Testing only (no counterpart in the reference): a scratch request above `bytes` fails as an
    *  allocation failure would, so that the search's batch halving can be exercised; 0 = no cap. */

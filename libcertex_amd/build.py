@@ -26,6 +26,7 @@ SOURCES = [
     "kernels/encode.hip",
     "kernels/partition.hip",
     "kernels/lists.hip",
+    "device_memory.cpp",
     "certex.cpp",
     "c_api.cpp",
 ]

@@ -72,6 +72,7 @@ void resources::trim() const
   }
   CERTEX_HIP_TRY(hipStreamSynchronize(s_->stream));
   for (auto& b : s_->slots) { b.release(); }
+  detail::device_trim(s_->device);
   if (s_->host_stage != nullptr) {
     CERTEX_HIP_TRY(hipHostFree(s_->host_stage));
     s_->host_stage       = nullptr;

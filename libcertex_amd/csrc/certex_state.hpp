@@ -12,6 +12,7 @@
 #include <string>
 #include <vector>
 
+#include "device_memory.hpp"
 #include "kernels.hpp"
 
 #define CERTEX_HIP_TRY(call)                                                              \
@@ -40,18 +41,21 @@ inline void expects(bool ok, const char* message)
 namespace cuvs::detail {
 
 /**
- * Owned memory that kernels read: device memory, or (host = true) pinned host memory mapped into
- * the device's address space (hipHostMalloc), which kernels read over PCIe.
+ * Owned memory that kernels read: device memory (device_allocate), or (host = true) pinned host
+ * memory mapped into the device's address space (hipHostMalloc), which kernels read over PCIe.
  */
 struct device_buffer {
-  void* p      = nullptr;
-  size_t bytes = 0;
-  bool host    = false;
+  void* p         = nullptr;
+  size_t bytes    = 0;
+  bool host       = false;
+  size_t capacity = 0;  // of the device block, and its device
+  int device      = 0;
   device_buffer() = default;
   explicit device_buffer(size_t n, bool in_host = false) : host(in_host) { resize_discard(n); }
   device_buffer(device_buffer const&)            = delete;
   device_buffer& operator=(device_buffer const&) = delete;
-  device_buffer(device_buffer&& o) noexcept : p(o.p), bytes(o.bytes), host(o.host)
+  device_buffer(device_buffer&& o) noexcept
+    : p(o.p), bytes(o.bytes), host(o.host), capacity(o.capacity), device(o.device)
   {
     o.p     = nullptr;
     o.bytes = 0;
@@ -61,12 +65,18 @@ struct device_buffer {
     std::swap(p, o.p);
     std::swap(bytes, o.bytes);
     std::swap(host, o.host);
+    std::swap(capacity, o.capacity);
+    std::swap(device, o.device);
     return *this;
   }
   ~device_buffer() { release(); }
   void release()
   {
-    if (p != nullptr) { (void)(host ? hipHostFree(p) : hipFree(p)); }
+    if (p != nullptr && host) {
+      (void)hipHostFree(p);
+    } else if (p != nullptr) {
+      device_release(p, capacity, device);
+    }
     p     = nullptr;
     bytes = 0;
   }
@@ -75,12 +85,13 @@ struct device_buffer {
   {
     release();
     if (n > 0) {
-      const hipError_t e = host ? hipHostMalloc(&p, n, hipHostMallocMapped) : hipMalloc(&p, n);
-      if (e != hipSuccess) {
+      if (!host) {
+        p = device_allocate(n, &capacity, &device);
+      } else if (hipHostMalloc(&p, n, hipHostMallocMapped) != hipSuccess) {
         (void)hipGetLastError();
         p = nullptr;
-        throw std::bad_alloc();
       }
+      if (p == nullptr) { throw std::bad_alloc(); }
       bytes = n;
     }
   }
@@ -241,6 +252,7 @@ struct row_partition {
 };
 
 struct index_state {
+  cuvs::detail::device_idle idle;  // before the buffers: the destructor waits for the device once
   int device                            = 0;
   vtype type                            = vtype::f32;
   cuvs::distance::DistanceType dmetric  = cuvs::distance::DistanceType::L2Expanded;
@@ -305,6 +317,7 @@ struct index_state {
   index_state() { CERTEX_HIP_TRY(hipEventCreateWithFlags(&updated, hipEventDisableTiming)); }
   ~index_state()
   {
+    idle.enter(device);
     if (updated != nullptr) { (void)hipEventDestroy(updated); }
   }
   index_state(index_state const&)            = delete;

@@ -1,0 +1,141 @@
+#include "device_memory.hpp"
+
+#include <hip/hip_runtime.h>
+
+#include <map>
+#include <mutex>
+#include <new>
+#include <unordered_map>
+
+namespace cuvs::detail {
+
+namespace {
+
+struct pool {
+  std::multimap<size_t, void*> blocks;
+  size_t held = 0;
+};
+
+std::mutex g_mutex;
+/** Never destroyed: at the process's end the driver takes the memory back. */
+auto pools() -> std::unordered_map<int, pool>&
+{
+  static auto* p = new std::unordered_map<int, pool>();
+  return *p;
+}
+
+/** The device that a device_idle of this thread covers (-1: none). */
+thread_local int t_idle = -1;
+
+/** hipSetDevice(device) for a scope, when it is not the current one. */
+struct on_device {
+  int before = -1;
+  explicit on_device(int device)
+  {
+    int now = -1;
+    if (hipGetDevice(&now) == hipSuccess && now != device && hipSetDevice(device) == hipSuccess) { before = now; }
+  }
+  ~on_device()
+  {
+    if (before >= 0) { (void)hipSetDevice(before); }
+  }
+};
+
+/** Sizes that allocations are rounded up to: 2 MiB pages from 1 MiB on, else 4 KiB. */
+auto rounded(size_t bytes) -> size_t
+{
+  const size_t unit = bytes >= (size_t(1) << 20) ? size_t(2) << 20 : size_t(4) << 10;
+  return (bytes + unit - 1) / unit * unit;
+}
+
+}  // namespace
+
+void* device_allocate(size_t bytes, size_t* capacity, int* device)
+{
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) { return nullptr; }
+  const size_t n = rounded(bytes);
+  {
+    std::lock_guard lk(g_mutex);
+    pool& p = pools()[dev];
+    auto it = p.blocks.lower_bound(n);
+    if (it != p.blocks.end() && it->first - it->first / 4 <= n) {
+      void* ptr = it->second;
+      *capacity = it->first;
+      *device   = dev;
+      p.held -= it->first;
+      p.blocks.erase(it);
+      return ptr;
+    }
+  }
+  void* ptr = nullptr;
+  if (hipMalloc(&ptr, n) != hipSuccess) {
+    (void)hipGetLastError();
+    device_trim(dev);
+    if (hipMalloc(&ptr, n) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+  }
+  *capacity = n;
+  *device   = dev;
+  return ptr;
+}
+
+void device_release(void* p, size_t capacity, int device) noexcept
+{
+  if (p == nullptr) { return; }
+  on_device at(device);
+  if (capacity <= kPoolBytes && (t_idle == device || hipDeviceSynchronize() == hipSuccess)) {
+    try {
+      std::lock_guard lk(g_mutex);
+      pool& q = pools()[device];
+      if (q.held + capacity <= kPoolBytes) {
+        q.blocks.emplace(capacity, p);
+        q.held += capacity;
+        return;
+      }
+    } catch (std::bad_alloc const&) {  // no host memory for the entry: the block goes back
+    }
+  }
+  (void)hipGetLastError();
+  (void)hipFree(p);
+}
+
+void device_trim(int device) noexcept
+{
+  std::multimap<size_t, void*> blocks;
+  {
+    std::lock_guard lk(g_mutex);
+    pool& p = pools()[device];
+    blocks.swap(p.blocks);
+    p.held = 0;
+  }
+  on_device at(device);
+  for (auto const& b : blocks) { (void)hipFree(b.second); }
+}
+
+size_t device_pooled(int device)
+{
+  std::lock_guard lk(g_mutex);
+  return pools()[device].held;
+}
+
+void device_idle::enter(int device) noexcept
+{
+  on_device at(device);
+  if (entered_ || hipDeviceSynchronize() != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  outer_   = t_idle;
+  t_idle   = device;
+  entered_ = true;
+}
+
+device_idle::~device_idle()
+{
+  if (entered_) { t_idle = outer_; }
+}
+
+}  // namespace cuvs::detail

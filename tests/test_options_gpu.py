@@ -117,3 +117,63 @@ def test_trim_pool(gpu):
     D1, I1 = idx.search(Q, k=100, batch=4_000)
     assert torch.equal(I0, I1) and torch.equal(D0, D1)
     check(X, Q[:50].cpu().numpy(), 100, "l2", D1[:50], I1[:50])
+
+
+def test_dropped_indexes_leave_a_bounded_pool(gpu):
+    """The memory of a dropped index serves the next one of its size and goes back to the driver by
+    trim_pool; a block larger than the pool's bound never stays."""
+    def made(n):
+        idx = certex.Index(128)
+        idx.add(torch.zeros((n, 128), dtype=torch.uint8, device="cuda"))
+        del idx
+
+    def used():
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    certex.trim_pool()
+    start = used()
+    made(1_000_000)
+    once = used()
+    assert once - start >= 128_000_000  # the codes wait in the pool
+    for _ in range(5):
+        made(1_000_000)
+    assert used() - once <= 64 << 20
+    made(36_000_000)  # 4.6 GB of codes: past the bound
+    assert used() - start <= (4 << 30) + (256 << 20)
+    certex.trim_pool()
+    assert used() - start <= 64 << 20
+
+
+def test_pooled_memory_across_threads_and_streams(gpu):
+    """Indexes built, searched and dropped at once on streams of four threads, their blocks passing
+    from one to another: every result is the exhaustive one."""
+    import threading
+
+    X = data.mixture_u8(60_000, seed=3)
+    Q = data.mixture_u8(64, seed=4)
+    want = {}
+    for t in range(4):
+        want[t] = oracle.knn(X[t * 10_000:][: 20_000 + 1_000 * t], Q, 5, "l2")[1]
+    Xg, Qg = torch.from_numpy(X).cuda(), torch.from_numpy(Q).cuda()
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(t):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(15):
+                idx = certex.Index(128)
+                idx.add(Xg[t * 10_000:][: 20_000 + 1_000 * t])
+                D, I = idx.search(Qg, k=5)
+                del idx
+                if not np.array_equal(I.cpu().numpy(), want[t]):
+                    bad.append(t)
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not bad
