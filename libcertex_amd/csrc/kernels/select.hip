@@ -209,51 +209,124 @@ __device__ inline bool keeps(const filter_args& f, int64_t q, uint32_t row)
 typedef int v4i_t __attribute__((ext_vector_type(4)));
 
 /**
- * Exact score of stored integer row `xrow` (row_bytes bytes, 16-byte aligned) against the query
- * codes in LDS, in int32. The codes are int8 (uint8 coordinates shifted by -128, bias = 128) and
- * zero past dim in both. For 8-bit data every fp64 partial sum of the oracle is an exact integer,
- * so this exact integer converts to the same double:
- *   l2:    sum (q - x)^2 = |q|^2 + |x|^2 - 2 <q, x>            (at most 255^2 * 256 < 2^31)
+ * Exact scores of stored integer rows, in int32. The codes are int8 (uint8 coordinates shifted by
+ * -128, bias = 128) and zero past dim. For 8-bit data every fp64 partial sum of the oracle is an
+ * exact integer, so this exact integer converts to the same double:
+ *   l2:    sum (q - x)^2 = |q|^2 + |x|^2 - 2 <q, x>            (at most 255^2 * 4096 < 2^31)
  *   inner: -sum (q + bias)(x + bias) = -(<q, x> + bias (sum q + sum x) + bias^2 dim)
- * qq = |q|^2 and qs = sum q of the query codes. Each 16-byte load feeds twelve v_dot4_i32_i8.
+ *
+ * A wave scores 64 candidates, one per lane, G lanes per row at a time (8 for rows of 128 bytes, 16
+ * for 256, 64 for wider ones): a row's 16-byte chunks are read by neighbouring lanes, so a load asks
+ * for whole lines, and 8 rows per slot are in flight. Slot s (lanes s G ..) takes the candidates of
+ * its own G lanes, one per round, and the rounds' sums are split over the slot's lanes
+ * (lanes::split_sums) so that lane e ends with the sum of candidate e. A lane per row read 16 bytes
+ * of 64 rows per load, each row's line again for every chunk. With it and several waves per query
+ * (verify_i8): one query over 128-byte rows 15.7 -> 5.5 us, 1,000 queries 20.8 -> 11 us, 10,000
+ * queries 61 -> 37 us; 100 queries over 960-byte rows 48 -> 16.6 us.
  */
-__device__ inline double int_score(const int8_t* qv, const int8_t* base, int64_t r, bool paired,
-                                   int row_bytes, int64_t dim, int bias, int qq, int qs,
-                                   metric_kind metric)
-{
-  int qx = 0, xx = 0, xs = 0;
-  // row r of `base`: contiguous, or in the paired layout (a wide label partition), where each
-  // 16-byte chunk lies whole inside one 64-byte piece
-  const int8_t* xrow = base + (paired ? (r >> 1) * 2 * int64_t(row_bytes) + (r & 1) * 64 : r * int64_t(row_bytes));
-  for (int j = 0; j < row_bytes; j += 16) {
-    const int jo   = paired ? (j >> 6) * 128 + (j & 63) : j;
-    const v4i_t x  = *reinterpret_cast<const v4i_t*>(xrow + jo);
-    const v4i_t qw = *reinterpret_cast<const v4i_t*>(qv + j);
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      qx = __builtin_amdgcn_sdot4(qw[b], x[b], qx, false);
-      xx = __builtin_amdgcn_sdot4(x[b], x[b], xx, false);
-      xs = __builtin_amdgcn_sdot4(x[b], 0x01010101, xs, false);
-    }
-  }
-  if (metric == metric_kind::l2) { return double(qq + xx - 2 * qx); }
-  return -double(int64_t(qx) + int64_t(bias) * (qs + xs) + int64_t(bias) * bias * dim);
-}
+template <int G>
+struct row_slots {
+  static constexpr int NCH = G == 64 ? 4 : 1;  // 16-byte chunks of a row per lane (rows up to 4,096)
+  v4i_t q[NCH];  // the query's chunks of this lane
+  int base;      // the score's part that does not depend on the row
+  bool l2;
+  int bias;
 
-/** |q|^2 and sum q of the query codes in LDS (row_bytes bytes, zero past dim). */
-__device__ inline void query_sums(const int8_t* qv, int row_bytes, int& qq, int& qs)
-{
-  qq = 0;
-  qs = 0;
-  for (int j = 0; j < row_bytes; j += 16) {
-    const v4i_t qw = *reinterpret_cast<const v4i_t*>(qv + j);
+  /** The chunks of query row `qrow` (row_bytes codes, zero past dim); every lane calls it. */
+  __device__ __forceinline__ void load_query(const int8_t* qrow, int row_bytes, int64_t dim, int b, bool is_l2)
+  {
+    l2       = is_l2;
+    bias     = b;
+    int part = 0;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      qq = __builtin_amdgcn_sdot4(qw[b], qw[b], qq, false);
-      qs = __builtin_amdgcn_sdot4(qw[b], 0x01010101, qs, false);
+    for (int t = 0; t < NCH; ++t) {
+      const int off = int(threadIdx.x % G) * 16 + 1024 * t;
+      q[t]          = v4i_t{0, 0, 0, 0};
+      if (off < row_bytes) { q[t] = *reinterpret_cast<const v4i_t*>(qrow + off); }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) { part = __builtin_amdgcn_sdot4(q[t][i], l2 ? q[t][i] : 0x01010101, part, false); }
     }
+    part = lanes::sum<G>(part);
+    base = l2 ? part : bias * part + int(int64_t(bias) * bias * dim);
   }
-}
+
+  /**
+   * The score (smaller is better) of this lane's candidate, a row at `row` (bit 0 set: in the paired
+   * layout, whose 16-byte chunks lie whole inside one 64-byte piece). Lanes at or past n (n >= 1)
+   * get some value. Every lane of the wave calls it with the same n.
+   */
+  __device__ __forceinline__ int score(uint64_t row, int n, int row_bytes) const
+  {
+    const int lane  = threadIdx.x & 63;
+    const int chunk = (lane % G) * 16;
+    if (lane >= n) { row = 0; }
+    const int first = __builtin_amdgcn_readfirstlane(int(uint32_t(row)));
+    const int firsh = __builtin_amdgcn_readfirstlane(int(row >> 32));
+    if (lane >= n) { row = (uint64_t(uint32_t(firsh)) << 32) | uint32_t(first); }  // in bounds, unused
+    constexpr int R = G < 16 ? G : 8;  // rows of a slot in flight
+    // sums of R rows of the slot: candidates j0 .. j0 + R - 1 of its lanes
+    const auto sums = [&](int j0, int* w) {
+      const int8_t* p[R];
+      bool paired[R];
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        uint32_t lo, hi;
+        if constexpr (G == 64) {
+          lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(row)), j0 + j));
+          hi = uint32_t(__builtin_amdgcn_readlane(int(row >> 32), j0 + j));
+        } else {
+          const int src = 4 * ((lane & ~(G - 1)) + j0 + j);
+          lo = uint32_t(__builtin_amdgcn_ds_bpermute(src, int(uint32_t(row))));
+          hi = uint32_t(__builtin_amdgcn_ds_bpermute(src, int(row >> 32)));
+        }
+        const uint64_t r = (uint64_t(hi) << 32) | lo;
+        paired[j]        = (r & 1) != 0;
+        p[j]             = reinterpret_cast<const int8_t*>(r & ~uint64_t(1));
+      }
+      int s1[R] = {}, s2[R] = {};
+#pragma unroll
+      for (int t = 0; t < NCH; ++t) {
+        const int off = chunk + 1024 * t;
+        if (NCH > 1 && t > 0 && 1024 * t >= row_bytes) { break; }  // uniform
+        const bool in = off < row_bytes;
+        v4i_t x[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          const int o = in ? off : 0;
+          x[j] = *reinterpret_cast<const v4i_t*>(p[j] + (paired[j] ? (o >> 6) * 128 + (o & 63) : o));
+        }
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int xi = in ? x[j][i] : 0;
+            s1[j] = __builtin_amdgcn_sdot4(xi, l2 ? xi : 0x01010101, s1[j], false);
+            s2[j] = __builtin_amdgcn_sdot4(q[t][i], xi, s2[j], false);
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < R; ++j) { w[j] = l2 ? s1[j] - 2 * s2[j] : s2[j] + bias * s1[j]; }
+    };
+    int mine = 0;
+    if constexpr (G <= 16) {
+      int w[G];
+#pragma unroll
+      for (int j0 = 0; j0 < G; j0 += R) { sums(j0, w + j0); }
+      lanes::split_sums<G, G>(w);
+      mine = w[0];
+    } else {
+      for (int j0 = 0; j0 < n; j0 += R) {
+        int w[R];
+        sums(j0, w);
+        lanes::split_sums<64, R>(w);  // sum j in the lanes 8 j .. 8 j + 7
+        const int v = __builtin_amdgcn_ds_bpermute(4 * 8 * (lane & 7), w[0]);
+        mine        = (lane & ~7) == j0 ? v : mine;
+      }
+    }
+    return l2 ? base + mine : -(base + mine);
+  }
+};
 
 constexpr int kBuf = 4096;  // LDS candidates per query (keys 32 KB + rows 16 KB)
 
@@ -579,12 +652,31 @@ __device__ inline uint64_t keep_k_best(uint64_t* key, uint32_t* row, int n, int 
   return K;
 }
 
+/** A candidate's codes (their address; bit 0: paired) and its id: a partition row, or a stored row. */
+struct code_row {
+  uint64_t at;
+  uint32_t id;
+};
+__device__ __forceinline__ code_row find_row(const verify_args& a, uint32_t r)
+{
+  code_row c;
+  const bool part = a.part_ids != nullptr && r < a.n_part;
+  const bool prd  = part && a.part_paired;
+  const auto* b   = part ? a.part_codes : a.codes;
+  const auto* row = b + (prd ? int64_t(r >> 1) * 2 * a.row_bytes + (r & 1) * 64 : int64_t(r) * a.row_bytes);
+  c.at            = reinterpret_cast<uint64_t>(row) | (prd ? 1u : 0u);
+  c.id            = part ? uint32_t(a.part_ids[r]) : listed_id(a.filter, r);
+  return c;
+}
+
+/** The integer re-rank of large buckets, large k or every row: one block per query, the candidates
+ *  scored by waves (row_slots) into an LDS buffer that is cut back to the k best when it fills. */
+template <int G>
 __global__ __launch_bounds__(kThreads) void verify_topk_i8_kernel(verify_args a, int cap)
 {
   extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];
   auto* key = reinterpret_cast<uint64_t*>(dyn);                    // [cap]
   auto* rid = reinterpret_cast<uint32_t*>(dyn + size_t(cap) * 8);  // [cap]
-  auto* qv  = reinterpret_cast<int8_t*>(dyn + size_t(cap) * 12);   // [row_bytes]
   __shared__ int fill;
   __shared__ int hist[256];
   __shared__ int wave_tot[4];
@@ -593,17 +685,14 @@ __global__ __launch_bounds__(kThreads) void verify_topk_i8_kernel(verify_args a,
 
   const int64_t q = blockIdx.x;
   const int tid   = threadIdx.x;
+  const int lane  = tid & 63;
   const int k     = a.k;
-  for (int j = tid; j < a.row_bytes; j += kThreads) { qv[j] = a.qcodes[q * a.row_bytes + j]; }
-  const int bias = a.flip ? 128 : 0;
-  __syncthreads();  // the query codes are in LDS
-  int qq, qs;
-  query_sums(qv, a.row_bytes, qq, qs);
-
   const int64_t n_cand =
     a.all_rows ? a.n_rows : (a.cand_count[q] < a.cap ? int64_t(a.cand_count[q]) : a.cap);
   if (!a.all_rows && n_cand <= a.small_max) { return; }  // the one-wave kernel's query
   const uint32_t* cand = a.cand_rows + q * a.cap;
+  row_slots<G> slots;
+  slots.load_query(a.qcodes + q * a.row_bytes, a.row_bytes, a.dim, a.flip ? 128 : 0, a.metric == metric_kind::l2);
 
   int have = 0;  // entries [0, have) of the buffer hold the best candidates so far
   if (tid == 0) { fill = 0; }
@@ -612,33 +701,20 @@ __global__ __launch_bounds__(kThreads) void verify_topk_i8_kernel(verify_args a,
     // fill the buffer beyond `have` with the next candidates (compacted by an LDS counter)
     const int room  = cap - have;
     const int64_t m = n_cand - c0 < room ? n_cand - c0 : room;
-    for (int64_t e = tid; e < m; e += kThreads) {
-      // the candidate's stored row (or partition row), then its id
-      uint32_t r;
-      bool live;
-      const int8_t* base = a.codes;
-      if (a.all_rows) {
-        r    = uint32_t(c0 + e);
-        live = a.rowc[r] != kDeadRow && keeps(a.filter, q, r);
-      } else {
-        r    = cand[c0 + e];
-        live = true;
-      }
-      uint32_t id;
-      bool paired = false;
-      if (!a.all_rows && a.part_ids != nullptr && r < a.n_part) {
-        base   = a.part_codes;
-        paired = a.part_paired;
-        id     = uint32_t(a.part_ids[r]);
-      } else {
-        id = listed_id(a.filter, r);
-      }
+    for (int64_t e0 = tid & ~63; e0 < m; e0 += kThreads) {
+      const int n      = m - e0 < 64 ? int(m - e0) : 64;
+      const int64_t e  = c0 + e0 + (lane < n ? lane : 0);
+      const uint32_t r = a.all_rows ? uint32_t(e) : cand[e];
+      const bool live =
+        lane < n && (!a.all_rows || (a.rowc[r] != kDeadRow && keeps(a.filter, q, r)));
+      const code_row c = a.all_rows ? code_row{reinterpret_cast<uint64_t>(a.codes + int64_t(r) * a.row_bytes),
+                                               listed_id(a.filter, r)}
+                                    : find_row(a, r);
+      const int v      = slots.score(c.at, n, a.row_bytes);
+      const int slot   = have + wave_append(live, &fill);
       if (live) {
-        const double s =
-          int_score(qv, base, r, paired, a.row_bytes, a.dim, bias, qq, qs, a.metric);
-        const int slot = have + atomicAdd(&fill, 1);
-        key[slot]      = score_key(s);
-        rid[slot]      = id;
+        key[slot] = score_key(double(v));
+        rid[slot] = c.id;
       }
     }
     c0 += m;
@@ -669,99 +745,95 @@ __global__ __launch_bounds__(kThreads) void verify_topk_i8_kernel(verify_args a,
   }
 }
 
+/** One compare-exchange stage of a bitonic sort over the 64 lanes; `up`: the lane's block of SIZE
+ *  lanes ends ascending. */
+template <int STRIDE>
+__device__ __forceinline__ uint64_t wave_stage(uint64_t k, bool up)
+{
+  const uint64_t o = lanes::exchange<STRIDE>(k);
+  const bool lower = (threadIdx.x & STRIDE) == 0;
+  return (lower == up) == (o < k) ? o : k;  // the lower lane keeps the smaller one going up
+}
+template <int SIZE, int STRIDE>
+__device__ __forceinline__ uint64_t wave_strides(uint64_t k, bool up)
+{
+  k = wave_stage<STRIDE>(k, up);
+  if constexpr (STRIDE > 1) { k = wave_strides<SIZE, STRIDE / 2>(k, up); }
+  return k;
+}
+template <int SIZE>
+__device__ __forceinline__ uint64_t wave_sizes(uint64_t k, bool descending)
+{
+  const bool up = ((threadIdx.x & SIZE & 63) == 0) != descending;
+  k             = wave_strides<SIZE, SIZE / 2>(k, up);
+  if constexpr (SIZE < 64) { k = wave_sizes<SIZE * 2>(k, descending); }
+  return k;
+}
 
 /** Candidates per query up to which the integer re-rank runs one wave per query. */
 constexpr int kSmallBucket = 512;
 
 /**
- * The integer re-rank for small buckets (at most kSmallBucket candidates, k <= 64): one wave per
- * query. Each lane scores up to kSmallBucket / 64 candidates into registers; then k rounds of a
- * wave minimum over (score key, id) emit the k best in order, with no LDS buffer and no barrier.
- * The output is the block kernel's: the k smallest (key, id) pairs, ascending, then +inf / -1.
- * Queries with larger buckets are left to the block kernel.
+ * The integer re-rank for small buckets (at most kSmallBucket candidates, k <= 64): W waves per
+ * query, each on every W-th run of CH candidates. Scores are whole numbers of 32 bits, so a
+ * candidate is one 64-bit key (score, id); a run's keys are sorted over the lanes (21
+ * compare-exchange stages on the VALU) and merged with the wave's 64 best so far (6 more), unless
+ * none of them beats the k-th best; then the waves' lists are merged. The output is the block
+ * kernel's: the k smallest (score, id) pairs, ascending, then +inf / -1. Queries with larger buckets
+ * are left to the block kernel.
  */
-__global__ __launch_bounds__(kThreads) void verify_topk_i8_small_kernel(verify_args a)
+template <int G, int W, int CH>
+__global__ __launch_bounds__(W == 1 ? kThreads : 64 * W) void verify_topk_i8_small_kernel(verify_args a)
 {
-  // dynamic LDS: the query codes of the block's waves [kThreads / 64][row_bytes]
-  extern __shared__ __attribute__((aligned(16))) int8_t qlds[];
-  const int lane    = threadIdx.x & 63;
-  const int wave    = threadIdx.x >> 6;
-  const int64_t q   = int64_t(blockIdx.x) * (kThreads / 64) + wave;
-  const bool live_q = q < a.nq;
-  int8_t* qv        = qlds + wave * a.row_bytes;
-  if (live_q) {
-    for (int j = lane; j < a.row_bytes; j += 64) { qv[j] = a.qcodes[q * a.row_bytes + j]; }
-  }
-  __syncthreads();  // the query codes are in LDS (the block's only barrier)
-  if (!live_q) { return; }
-  int qq, qs;
-  query_sums(qv, a.row_bytes, qq, qs);
-  const int bias       = a.flip ? 128 : 0;
-  const int64_t n_cand = a.cand_count[q] < a.cap ? int64_t(a.cand_count[q]) : a.cap;
+  __shared__ uint64_t lists[W > 1 ? (W - 1) * 64 : 1];
+  const int lane  = threadIdx.x & 63;
+  const int wave  = threadIdx.x >> 6;
+  const int64_t q = W > 1 ? int64_t(blockIdx.x) : int64_t(blockIdx.x) * (kThreads / 64) + wave;
+  if (q >= a.nq) { return; }  // whole waves leave (W > 1: whole blocks)
+  const int n_cand = int(a.cand_count[q] < a.cap ? int64_t(a.cand_count[q]) : a.cap);
   if (n_cand > kSmallBucket) { return; }
   const uint32_t* cand = a.cand_rows + q * a.cap;
-  constexpr int NPL    = kSmallBucket / 64;  // candidates per lane
-  uint64_t key[NPL];
-  uint32_t rid[NPL];
-#pragma unroll
-  for (int i = 0; i < NPL; ++i) {
-    const int64_t e = lane + 64 * i;
-    key[i]          = ~0ull;
-    rid[i]          = ~0u;
-    if (e < n_cand) {
-      const uint32_t r   = cand[e];
-      const int8_t* base = a.codes;
-      uint32_t id;
-      bool paired = false;
-      if (a.part_ids != nullptr && r < a.n_part) {
-        base   = a.part_codes;
-        paired = a.part_paired;
-        id     = uint32_t(a.part_ids[r]);
+  uint64_t best = ~0ull;  // lane j: the j-th best so far
+  uint64_t kth  = ~0ull;
+  const int c1  = W > 1 ? wave * CH : 0;
+  if (c1 < n_cand) {
+    row_slots<G> slots;
+    slots.load_query(a.qcodes + q * a.row_bytes, a.row_bytes, a.dim, a.flip ? 128 : 0, a.metric == metric_kind::l2);
+    for (int c0 = c1; c0 < n_cand; c0 += W * CH) {
+      const int n      = n_cand - c0 < CH ? n_cand - c0 : CH;
+      const code_row c = find_row(a, cand[c0 + (lane < n ? lane : 0)]);
+      const int v      = slots.score(c.at, n, a.row_bytes);
+      uint64_t key     = (uint64_t(uint32_t(v) ^ 0x80000000u) << 32) | c.id;
+      key              = lane < n ? key : ~0ull;
+      if (!__any(key < kth)) { continue; }
+      if (c0 == c1) {
+        best = wave_sizes<2>(key, false);
       } else {
-        id = listed_id(a.filter, r);
+        key  = wave_sizes<2>(key, true);
+        best = key < best ? key : best;  // the 64 smallest of both, a bitonic sequence
+        best = wave_strides<64, 32>(best, true);
       }
-      key[i] = score_key(int_score(qv, base, r, paired, a.row_bytes, a.dim, bias,
-                                   qq, qs, a.metric));
-      rid[i] = id;
+      const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(best)), a.k - 1));
+      const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(best >> 32), a.k - 1));
+      kth               = (uint64_t(hi) << 32) | lo;
     }
   }
-  double my_s   = INFINITY;
-  int64_t my_r  = -1;
-  for (int j = 0; j < a.k; ++j) {
-    uint64_t bk = key[0];
-    uint32_t br = rid[0];
-#pragma unroll
-    for (int i = 1; i < NPL; ++i) {
-      if (key[i] < bk || (key[i] == bk && rid[i] < br)) {
-        bk = key[i];
-        br = rid[i];
-      }
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      const uint32_t lo = uint32_t(__shfl_xor(int(uint32_t(bk)), off));
-      const uint32_t hi = uint32_t(__shfl_xor(int(uint32_t(bk >> 32)), off));
-      const uint64_t ok = (uint64_t(hi) << 32) | lo;
-      const uint32_t orr = uint32_t(__shfl_xor(int(br), off));
-      if (ok < bk || (ok == bk && orr < br)) {
-        bk = ok;
-        br = orr;
-      }
-    }
-    if (bk == ~0ull) { break; }  // every lane holds the same pair: fewer than k candidates
-#pragma unroll
-    for (int i = 0; i < NPL; ++i) {
-      if (key[i] == bk && rid[i] == br) {
-        key[i] = ~0ull;
-        rid[i] = ~0u;
-      }
-    }
-    if (lane == j) {
-      my_s = key_score(bk);
-      my_r = int64_t(br);
+  if constexpr (W > 1) {
+    if (wave > 0) { lists[(wave - 1) * 64 + 63 - lane] = best; }  // descending, for the merge
+    __syncthreads();
+    if (wave > 0) { return; }
+    for (int w = 1; w < W && w * CH < n_cand; ++w) {
+      const uint64_t key = lists[(w - 1) * 64 + lane];
+      if (!__any(key < best)) { continue; }
+      best = key < best ? key : best;
+      best = wave_strides<64, 32>(best, true);
     }
   }
-  if (lane < a.k) { put_result(a, q, lane, my_s, my_r); }
+  if (lane < a.k) {
+    const bool has = best != ~0ull;
+    put_result(a, q, lane, has ? double(int(uint32_t(best >> 32) ^ 0x80000000u)) : 0.0,
+               has ? int64_t(uint32_t(best)) : -1);
+  }
 }
 
 // ---- float vectors ---------------------------------------------------------------------------
@@ -1806,16 +1878,26 @@ void sum_u32(const uint32_t* count, int64_t n, int64_t cap, unsigned long long* 
   if (blocks > 0) { sum_kernel<<<unsigned(blocks), 256, 0, stream>>>(count, n, cap, out); }
 }
 
-void verify_topk_i8(const verify_args& a, hipStream_t stream)
+namespace {
+
+template <int G>
+void verify_i8(const verify_args& a, hipStream_t stream)
 {
-  if (a.nq == 0) { return; }
   verify_args b = a;
   b.small_max   = -1;
   if (!a.all_rows && a.k <= 64) {
     // buckets of up to kSmallBucket candidates: one wave per query; the block kernel then takes
     // only the larger buckets (launched when the host saw one)
-    verify_topk_i8_small_kernel<<<unsigned((a.nq + 3) / 4), kThreads,
-                                  size_t(kThreads / 64) * size_t(a.row_bytes), stream>>>(a);
+    // fewer queries than fill the chip with waves: several waves per query, whose runs of
+    // candidates then wait for memory at the same time (wide rows take shorter runs: a run is a row
+    // after the other there)
+    if (a.nq <= 512) {
+      verify_topk_i8_small_kernel<G, 8, G == 64 ? 16 : 64><<<unsigned(a.nq), 512, 0, stream>>>(a);
+    } else if (a.nq <= 2048) {
+      verify_topk_i8_small_kernel<G, 4, G == 64 ? 16 : 64><<<unsigned(a.nq), 256, 0, stream>>>(a);
+    } else {
+      verify_topk_i8_small_kernel<G, 1, 64><<<unsigned((a.nq + 3) / 4), kThreads, 0, stream>>>(a);
+    }
     if (a.max_cand >= 0 && a.max_cand <= kSmallBucket) { return; }
     b.small_max = kSmallBucket;
   }
@@ -1823,8 +1905,19 @@ void verify_topk_i8(const verify_args& a, hipStream_t stream)
   // blocks share a CU
   int cap = pow2_ge(2 * a.k);
   cap     = cap > 1024 ? (cap < kBuf ? cap : kBuf) : 1024;
-  const size_t bytes = size_t(cap) * 12 + size_t(a.row_bytes);
-  verify_topk_i8_kernel<<<unsigned(a.nq), kThreads, bytes, stream>>>(b, cap);
+  verify_topk_i8_kernel<G><<<unsigned(a.nq), kThreads, size_t(cap) * 12, stream>>>(b, cap);
+}
+
+}  // namespace
+
+void verify_topk_i8(const verify_args& a, hipStream_t stream)
+{
+  if (a.nq == 0) { return; }
+  switch (a.row_bytes) {
+    case 128: verify_i8<8>(a, stream); break;
+    case 256: verify_i8<16>(a, stream); break;
+    default: verify_i8<64>(a, stream); break;
+  }
 }
 
 /** Launches a kernel with `bytes` of dynamic LDS (raising the kernel's limit when needed). */

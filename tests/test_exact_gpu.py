@@ -239,3 +239,20 @@ def test_filter_words_packed_on_the_gpu(gpu, shape):
     both = np.packbits(np.concatenate([m[1:], m[1:]]), bitorder="little")
     np.testing.assert_array_equal(_pack(row.expand(2, n)).cpu().numpy().view(np.uint32),
                                   np.pad(both, (0, (-both.size) % 4)).view(np.uint32))
+
+
+@pytest.mark.parametrize("d", [128, 200, 300, 1100])  # 8, 16 and 64 lanes per scored row
+@pytest.mark.parametrize("nq", [1, 512, 513, 2048, 2049])  # 8, 4 and 1 waves per query
+def test_integer_rerank_waves(gpu, d, nq):
+    """The one-wave-group re-rank of small buckets next to the block re-rank of large ones (k = 64
+    leaves more than 512 survivors on some queries), ties to the lower id, both metrics."""
+    X = data.uniform_int(9_001, d, seed=d, dtype=np.int8)
+    X[4_000:4_500] = X[:500]  # ties
+    Q = np.concatenate([X[:40], data.uniform_int(2_009, d, seed=d + 1, dtype=np.int8)])[:nq]
+    for metric, k in (("l2", 1), ("l2", 13), ("ip", 64)):
+        idx = certex.Index(d, metric=metric)
+        idx.add(torch.from_numpy(X).cuda())
+        D, I = idx.search(torch.from_numpy(Q).cuda(), k=k, batch=4096)
+        s, i = oracle.knn(X, Q, k, metric)
+        np.testing.assert_array_equal(I.cpu().numpy(), i)
+        np.testing.assert_array_equal(D.cpu().numpy(), oracle.distances(s, i, metric))
