@@ -11,9 +11,14 @@ namespace cuvs::detail {
 
 namespace {
 
+struct block {
+  void* p;
+  unsigned long long age;  // the pool's count when it came in
+};
 struct pool {
-  std::multimap<size_t, void*> blocks;
-  size_t held = 0;
+  std::multimap<size_t, block> blocks;
+  size_t held             = 0;
+  unsigned long long ages = 0;
 };
 
 std::mutex g_mutex;
@@ -60,7 +65,7 @@ void* device_allocate(size_t bytes, size_t* capacity, int* device)
     pool& p = pools()[dev];
     auto it = p.blocks.lower_bound(n);
     if (it != p.blocks.end() && it->first - it->first / 4 <= n) {
-      void* ptr = it->second;
+      void* ptr = it->second.p;
       *capacity = it->first;
       *device   = dev;
       p.held -= it->first;
@@ -87,15 +92,29 @@ void device_release(void* p, size_t capacity, int device) noexcept
   if (p == nullptr) { return; }
   on_device at(device);
   if (capacity <= kPoolBytes && (t_idle == device || hipDeviceSynchronize() == hipSuccess)) {
-    try {
-      std::lock_guard lk(g_mutex);
-      pool& q = pools()[device];
-      if (q.held + capacity <= kPoolBytes) {
-        q.blocks.emplace(capacity, p);
-        q.held += capacity;
-        return;
+    // the newest block stays, the oldest ones make room: what was freed last is what a program
+    // that builds and drops alike indexes asks for next
+    while (true) {
+      void* oldest = nullptr;
+      try {
+        std::lock_guard lk(g_mutex);
+        pool& q = pools()[device];
+        if (q.held + capacity <= kPoolBytes) {
+          q.blocks.emplace(capacity, block{p, q.ages++});
+          q.held += capacity;
+          return;
+        }
+        auto it = q.blocks.begin();
+        for (auto b = q.blocks.begin(); b != q.blocks.end(); ++b) {
+          if (b->second.age < it->second.age) { it = b; }
+        }
+        oldest = it->second.p;
+        q.held -= it->first;
+        q.blocks.erase(it);
+      } catch (std::bad_alloc const&) {  // no host memory for the entry: the block goes back
+        break;
       }
-    } catch (std::bad_alloc const&) {  // no host memory for the entry: the block goes back
+      (void)hipFree(oldest);
     }
   }
   (void)hipGetLastError();
@@ -104,7 +123,7 @@ void device_release(void* p, size_t capacity, int device) noexcept
 
 void device_trim(int device) noexcept
 {
-  std::multimap<size_t, void*> blocks;
+  std::multimap<size_t, block> blocks;
   {
     std::lock_guard lk(g_mutex);
     pool& p = pools()[device];
@@ -112,7 +131,7 @@ void device_trim(int device) noexcept
     p.held = 0;
   }
   on_device at(device);
-  for (auto const& b : blocks) { (void)hipFree(b.second); }
+  for (auto const& b : blocks) { (void)hipFree(b.second.p); }
 }
 
 size_t device_pooled(int device)

@@ -12,8 +12,9 @@ namespace cuvs::detail {
  * - a block enters the pool only when the device is idle of every use of it: device_release waits
  *   for the device, as hipFree does, or the caller has (device_idle). Any thread and any stream
  *   may then take it;
- * - the pool of a device holds at most kPoolBytes; a block that does not fit goes back to the
- *   driver, and an allocation the driver refuses empties the pool and is tried again;
+ * - the pool of a device holds at most kPoolBytes: its oldest blocks go back to the driver to make
+ *   room, a larger block at once, and an allocation the driver refuses empties the pool and is tried
+ *   again;
  * - device_trim gives the pool of a device back to the driver (cuvsCertexTrimPool).
  * A block serves requests of at least three quarters of its size, so that little of it is unused.
  */

@@ -143,6 +143,12 @@ def test_dropped_indexes_leave_a_bounded_pool(gpu):
     assert used() - once <= 64 << 20
     made(36_000_000)  # 4.6 GB of codes: past the bound
     assert used() - start <= (4 << 30) + (256 << 20)
+    for n in (20_000_000, 12_000_000, 9_000_000):  # 2.6, 1.5 and 1.2 GB: the oldest make room
+        made(n)
+        assert used() - start <= (4 << 30) + (256 << 20)
+    kept = used()
+    made(9_000_000)
+    assert abs(used() - kept) <= 64 << 20
     certex.trim_pool()
     assert used() - start <= 64 << 20
 
