@@ -31,8 +31,9 @@ resources::resources(void* stream) : s_(std::make_unique<detail::resources_state
     CERTEX_HIP_TRY(hipStreamCreateWithFlags(&s_->stream, hipStreamNonBlocking));
     s_->owns_stream = true;
   }
-  CERTEX_HIP_TRY(hipHostMalloc(&s_->host_small, 64, hipHostMallocDefault));
-  CERTEX_HIP_TRY(hipEventCreateWithFlags(&s_->read_back, hipEventDisableTiming));
+  // written by kernels while they run (publish_args): coherent
+  CERTEX_HIP_TRY(hipHostMalloc(&s_->host_small, 64, hipHostMallocMapped | hipHostMallocCoherent));
+  std::memset(s_->host_small, 0, 64);
   CERTEX_HIP_TRY(hipEventCreateWithFlags(&s_->staged, hipEventDisableTiming));
 }
 
@@ -42,7 +43,6 @@ resources::~resources()
     (void)hipStreamSynchronize(s_->stream);
     for (auto& b : s_->slots) { b.release(); }
     if (s_->host_small) { (void)hipHostFree(s_->host_small); }
-    if (s_->read_back) { (void)hipEventDestroy(s_->read_back); }
     if (s_->staged) { (void)hipEventDestroy(s_->staged); }
     if (s_->host_stage) { (void)hipHostFree(s_->host_stage); }
     if (s_->owns_stream) { (void)hipStreamDestroy(s_->stream); }
@@ -504,34 +504,41 @@ auto screen_pass(index_state const& st, route_plan const* route, F&& launch)
   };
 }
 
-/** No work launched behind the screen before its bucket check (see screen_into_buckets). */
-struct no_speculation {
-  void operator()() const {}
+/** The buckets' counts [nq_pad] and the two words that the screen leaves for the host (the largest
+ *  count past a limit, and past the LDS lists); the threshold kernels clear both. */
+struct bucket_counts {
+  uint32_t* count;
+  uint32_t* small;
 };
+auto get_counts(cuvs::resources const& res, int64_t nq_pad) -> bucket_counts
+{
+  auto& rs = res.state();
+  return {static_cast<uint32_t*>(rs.get(cuvs::detail::ws_count, size_t(nq_pad) * 4)),
+          static_cast<uint32_t*>(rs.get(cuvs::detail::ws_small, 64))};
+}
 
 /**
  * Screen pass into per-query buckets, re-run with larger buckets while one overflows (the
  * reference re-runs on segment overflow, certex.cu:1208-1269). Returns false when some query
  * keeps so many rows that scoring every row is cheaper (all_rows).
  * `speculate` launches the work that reads the buckets (the exact re-rank) right behind the
- * screen, before the host has read back the largest bucket: the host then waits for that read-back
- * only (an event), not for the re-rank. When the check fails (a re-run, or all_rows) the
- * speculative work has read clipped buckets, and what the caller launches next overwrites its
- * results in stream order.
+ * screen, before the host knows the largest bucket, with a publication that its first kernel makes
+ * as it starts: the host then waits for the screen, not for the re-rank. When the check fails (a
+ * re-run, or all_rows) the speculative work has read clipped buckets, and what the caller launches
+ * next overwrites its results in stream order. Without it (false) a kernel of its own publishes.
+ * *past (if given): whether some bucket holds more than `limit` rows.
  */
-template <typename F, typename V = no_speculation>
-bool screen_into_buckets(cuvs::resources const& res, int64_t B, int64_t nq_pad, int64_t size,
-                         certex_amd::screen_args& sa, F&& screen, uint32_t*& count,
-                         uint32_t*& rows, int64_t& cap, float** vals = nullptr,
-                         int64_t* worst_out = nullptr, V&& speculate = V{})
+template <typename F, typename V>
+bool screen_into_buckets(cuvs::resources const& res, int64_t nq_pad, int64_t size,
+                         certex_amd::screen_args& sa, F&& screen, bucket_counts const& bc,
+                         uint32_t*& rows, int64_t& cap, float** vals, int64_t limit, bool* past,
+                         V&& speculate)
 {
   auto& rs           = res.state();
   hipStream_t stream = rs.stream;
-  auto* small        = static_cast<uint32_t*>(rs.get(cuvs::detail::ws_small, 64));
-  count              = static_cast<uint32_t*>(rs.get(cuvs::detail::ws_count, size_t(nq_pad) * 4));
   cap                = rs.bucket_cap;
   const int64_t all_rows_above = std::max<int64_t>(1 << 16, size / 8);
-  while (true) {
+  for (bool cleared = true;; cleared = false) {
     if (size_t(nq_pad) * size_t(cap) * 4 > (size_t(1) << 32)) { throw batch_too_large(); }
     rows = static_cast<uint32_t*>(
       rs.get(cuvs::detail::ws_rows, size_t(nq_pad) * size_t(cap) * 4));
@@ -549,25 +556,27 @@ bool screen_into_buckets(cuvs::resources const& res, int64_t B, int64_t nq_pad, 
       sa.spill       = static_cast<uint32_t*>(rs.get(cuvs::detail::ws_spill, e * 4 * w));
       sa.spill_pool  = int64_t(e);
     }
-    certex_amd::fill_u32(count, nq_pad, 0, stream);
-    certex_amd::fill_u32(small, 2, 0, stream);
-    sa.spill_need  = small + 1;
+    if (!cleared) {  // a re-run: the threshold kernel cleared them for the first
+      certex_amd::fill_u32(bc.count, nq_pad, 0, stream);
+      certex_amd::fill_u32(bc.small, 2, 0, stream);
+    }
+    sa.most        = bc.small;
+    sa.most_above  = uint32_t(std::min(cap, limit));
+    sa.spill_need  = bc.small + 1;
     sa.n_scan      = size;
     sa.row_stride  = 1;
-    sa.cand_count  = count;
+    sa.cand_count  = bc.count;
     sa.cand_rows   = rows;
     sa.cap         = cap;
     sa.clock = t_timing.on ? t_timing.clock : nullptr;
     timed(2, stream, [&] { screen(sa, stream); });
     sa.clock = nullptr;
-    certex_amd::max_u32(count, B, small, stream);
-    CERTEX_HIP_TRY(hipMemcpyAsync(rs.host_small, small, 8, hipMemcpyDeviceToHost, stream));
-    CERTEX_HIP_TRY(hipEventRecord(rs.read_back, stream));
-    speculate();
-    CERTEX_HIP_TRY(hipEventSynchronize(rs.read_back));
-    const int64_t worst = static_cast<uint32_t*>(rs.host_small)[0];
-    if (static_cast<uint32_t*>(rs.host_small)[1] > 0) { rs.spill_pool = true; }
-    if (worst_out != nullptr) { *worst_out = worst; }
+    const auto pub = rs.next_publication(bc.small);
+    if (!speculate(pub)) { certex_amd::publish(pub, stream); }
+    const uint32_t* words = rs.published();
+    const int64_t worst   = words[0];
+    if (words[1] > 0) { rs.spill_pool = true; }
+    if (past != nullptr) { *past = worst > limit; }
     if (worst <= cap) { return true; }
     if (worst > all_rows_above) { return false; }
     int64_t c = 1024;
@@ -987,24 +996,67 @@ void search_batch_int(cuvs::resources const& res, index_state const& st, const v
 
   auto* theta   = static_cast<int32_t*>(rs.get(cuvs::detail::ws_theta, size_t(nq_pad) * 4));
   bool all_rows = tp.n_groups < k;
+  bucket_counts bc{};
   if (!all_rows) {
+    bc         = get_counts(res, nq_pad);
     auto* gmax = static_cast<int32_t*>(
       rs.get(cuvs::detail::ws_gmax, size_t(nq_pad) * size_t(tp.n_groups) * 4));
     certex_amd::screen_args aa = sa;
     aa.gmax                    = gmax;
     timed(0, stream, [&] { table_pass(res, st, aa, tp, route, certex_amd::anchors_i8); });
-    timed(1, stream,
-          [&] { certex_amd::threshold_i8(gmax, tp.n_groups, B, nq_pad, k, theta, stream); });
+    timed(1, stream, [&] {
+      certex_amd::threshold_i8(gmax, tp.n_groups, B, nq_pad, k, theta, bc.count, bc.small, stream);
+    });
   }
 
-  uint32_t *count = nullptr, *rows = nullptr;
-  int64_t cap = 0, worst = -1;
+  uint32_t* rows = nullptr;
+  int64_t cap    = 0;
+  certex_amd::verify_args va{};
+  va.n_rows     = size;
+  va.codes      = st.codes.as<int8_t>();
+  va.rowc       = st.rowc.as<int32_t>();
+  va.row_bytes  = st.row_bytes;
+  va.dim        = st.dim;
+  va.flip       = flip;
+  va.qcodes     = qcodes;
+  va.metric     = st.metric;
+  va.filter     = fa;
+  va.nq         = B;
+  va.k          = k;
+  if (route != nullptr) {
+    va.part_ids   = st.label_part.ids.as<int32_t>();
+    va.n_part     = st.label_part.n;
+    va.part_codes  = st.label_part.codes.as<int8_t>();
+    va.part_paired = st.label_part.paired;
+  }
+  va.distances = distances;
+  va.neighbors = neighbors;
+  va.out_rows  = qmap;
+  // the exact re-rank over the buckets as they are (some part of it), or over every row (all_rows)
+  auto verify = [&](bool every_row, int part, certex_amd::publish_args pub) {
+    va.cand_count = bc.count;
+    va.cand_rows  = rows;
+    va.cap        = cap;
+    va.all_rows   = every_row;
+    va.part       = part;
+    va.publish    = pub;
+    timed(3, stream, [&] { certex_amd::verify_topk_i8(va, stream); });
+  };
+  const bool capture = t_capture.on;
+  const bool waves   = k <= 64;  // part 1 of the re-rank covers buckets of up to kSmallBucket
+  bool verified = false, large = true;
   if (!all_rows) {
     sa.theta = theta;
-    all_rows = !screen_into_buckets(res, B, nq_pad, size, sa,
-                                    screen_pass(st, route, certex_amd::screen_i8), count, rows,
-                                    cap, nullptr, &worst);
+    all_rows = !screen_into_buckets(
+      res, nq_pad, size, sa, screen_pass(st, route, certex_amd::screen_i8), bc, rows, cap, nullptr,
+      waves ? certex_amd::kSmallBucket : INT32_MAX, &large, [&](certex_amd::publish_args pub) {
+        if (!capture) { verify(false, waves ? 1 : 0, pub); }
+        return !capture;
+      });
+    verified = !all_rows && !capture;
+    if (verified && waves && large) { verify(false, 2, {}); }
   }
+  uint32_t* count = bc.count;
   count_stats(res, st, B, all_rows, count, cap);
   if (t_capture.on) {
     capture_common(st, tp, B, nq_pad, k, all_rows, cap, route, stream);
@@ -1026,33 +1078,7 @@ void search_batch_int(cuvs::resources const& res, index_state const& st, const v
     t_capture.on = false;
   }
 
-  certex_amd::verify_args va{};
-  va.cand_count = count;
-  va.cand_rows  = rows;
-  va.cap        = cap;
-  va.all_rows   = all_rows;
-  va.max_cand   = all_rows ? -1 : worst;
-  va.n_rows     = size;
-  va.codes      = st.codes.as<int8_t>();
-  va.rowc       = st.rowc.as<int32_t>();
-  va.row_bytes  = st.row_bytes;
-  va.dim        = st.dim;
-  va.flip       = flip;
-  va.qcodes     = qcodes;
-  va.metric     = st.metric;
-  va.filter     = fa;
-  va.nq         = B;
-  va.k          = k;
-  if (route != nullptr) {
-    va.part_ids   = st.label_part.ids.as<int32_t>();
-    va.n_part     = st.label_part.n;
-    va.part_codes  = st.label_part.codes.as<int8_t>();
-    va.part_paired = st.label_part.paired;
-  }
-  va.distances = distances;
-  va.neighbors = neighbors;
-  va.out_rows  = qmap;
-  timed(3, stream, [&] { certex_amd::verify_topk_i8(va, stream); });
+  if (!verified) { verify(all_rows, 0, {}); }
 }
 
 /** One batch of queries of a float index (the caller holds the shared lock). */
@@ -1099,7 +1125,9 @@ void search_batch_float(cuvs::resources const& res, index_state const& st, const
   bool all_rows = tp.n_groups < k;
   certex_amd::threshold_f_args ta{};
   std::unique_ptr<capture_buffer<double>> ub_q;  // testing: U per query
+  bucket_counts bc{};
   if (!all_rows) {
+    bc = get_counts(res, nq_pad);
     auto* gmax = static_cast<float*>(
       rs.get(cuvs::detail::ws_gmax, size_t(nq_pad) * size_t(tp.n_groups) * 4));
     certex_amd::screen_args aa = sa;
@@ -1120,6 +1148,8 @@ void search_batch_float(cuvs::resources const& res, index_state const& st, const
     ta.alpha2   = st.alpha * st.alpha;
     ta.gamma    = st.gamma;
     ta.theta    = theta;
+    ta.count    = bc.count;
+    ta.small    = bc.small;
     if (t_capture.on) {
       ub_q = std::make_unique<capture_buffer<double>>(size_t(nq_pad));
       ta.ub = ub_q->p;
@@ -1128,7 +1158,7 @@ void search_batch_float(cuvs::resources const& res, index_state const& st, const
     ta.ub = nullptr;
   }
 
-  uint32_t *count = nullptr, *rows = nullptr;
+  uint32_t *count = bc.count, *rows = nullptr;
   float* vals = nullptr;
   int64_t cap = 0;
   unsigned long long* scored = nullptr;
@@ -1161,12 +1191,13 @@ void search_batch_float(cuvs::resources const& res, index_state const& st, const
     va.n_part   = st.label_part.n;
   }
   // the exact re-rank over the buckets as they are, or over every row (all_rows)
-  auto verify = [&](bool every_row) {
+  auto verify = [&](bool every_row, certex_amd::publish_args pub) {
     va.cand_count = count;
     va.cand_rows  = rows;
     va.cand_vals  = vals;
     va.cap        = cap;
     va.all_rows   = every_row;
+    va.publish    = pub;
     if (scored != nullptr) { certex_amd::fill_u32(reinterpret_cast<uint32_t*>(scored), 2, 0, stream); }
     timed(3, stream, [&] { certex_amd::verify_topk_f(va, stream); });
   };
@@ -1176,10 +1207,11 @@ void search_batch_float(cuvs::resources const& res, index_state const& st, const
   if (!all_rows) {
     sa.theta = theta;
     all_rows = !screen_into_buckets(
-      res, B, nq_pad, size, sa,
-      screen_pass(st, route, wide ? certex_amd::screen_f16_tile : certex_amd::screen_f16), count,
-      rows, cap, &vals, nullptr, [&] {
-        if (!capture) { verify(false); }
+      res, nq_pad, size, sa,
+      screen_pass(st, route, wide ? certex_amd::screen_f16_tile : certex_amd::screen_f16), bc, rows,
+      cap, &vals, INT32_MAX, nullptr, [&](certex_amd::publish_args pub) {
+        if (!capture) { verify(false, pub); }
+        return !capture;
       });
     verified = !all_rows && !capture;
   }
@@ -1212,11 +1244,11 @@ void search_batch_float(cuvs::resources const& res, index_state const& st, const
     CERTEX_HIP_TRY(hipStreamSynchronize(stream));
     t_capture.on = false;
     if (!all_rows) {
-      verify(false);
+      verify(false, {});
       verified = true;
     }
   }
-  if (!verified) { verify(true); }
+  if (!verified) { verify(true, {}); }
   count_stats(res, st, B, all_rows, count, cap, true);
   if (scored != nullptr) {
     CERTEX_HIP_TRY(hipMemcpyAsync(rs.host_small, scored, 8, hipMemcpyDeviceToHost, stream));

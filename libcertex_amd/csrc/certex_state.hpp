@@ -10,6 +10,7 @@
 #include <shared_mutex>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "device_memory.hpp"
@@ -133,7 +134,7 @@ struct resources_state {
   bool spill_pool     = false;  // a screen's LDS survivor lists overflowed: provide a spill pool
   device_buffer slots[ws_n_slots];
   void* host_small    = nullptr;  // pinned host words for counters read back by the host
-  hipEvent_t read_back = nullptr;  // recorded behind a read-back into host_small
+  uint32_t ticket      = 0;  // of the latest publication into host_small (publish_args)
   void* host_stage    = nullptr;  // pinned host staging of the routing tables (grow-only)
   size_t host_stage_bytes = 0;
   hipEvent_t staged   = nullptr;  // recorded behind the last copy out of host_stage
@@ -151,6 +152,33 @@ struct resources_state {
   size_t arena_used  = 0;
   void* carved[ws_n_slots]        = {};
   size_t carved_bytes[ws_n_slots] = {};
+
+  /** The next publication of the two words `words` into host_small. */
+  auto next_publication(const uint32_t* words) -> certex_amd::publish_args
+  {
+    return {words, static_cast<uint32_t*>(host_small) + kPublished, ++ticket};
+  }
+  static constexpr int kPublished = 8;  // host_small's words 8, 9 and 10 (the ticket)
+
+  /** Waits until the latest publication has arrived; its two words. */
+  auto published() -> const uint32_t*
+  {
+    uint32_t* w = static_cast<uint32_t*>(host_small) + kPublished;
+    for (uint32_t spin = 1; __atomic_load_n(w + 2, __ATOMIC_ACQUIRE) != ticket; ++spin) {
+      // every so often: is the stream still at it?
+      if (spin % 4096 != 0) { continue; }
+      const hipError_t e = hipStreamQuery(stream);
+      if (e == hipErrorNotReady) {
+        std::this_thread::yield();
+      } else {
+        CERTEX_HIP_TRY(e);
+        if (__atomic_load_n(w + 2, __ATOMIC_ACQUIRE) != ticket) {
+          throw std::runtime_error("certex: a search's kernels ended without their counts");
+        }
+      }
+    }
+    return w;
+  }
 
   /** Forget every carved slot: the next batch carves from the start of the arena. */
   void arena_reset()

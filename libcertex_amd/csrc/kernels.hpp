@@ -209,6 +209,10 @@ struct screen_args {
   uint32_t* cand_rows  = nullptr;  // [nq_pad, cap]
   float* cand_vals     = nullptr;  // [nq_pad, cap] screen values (fp16 rows only)
   int64_t cap          = 0;
+  // *most: at least the largest bucket count past cap (exactly where flushes alone fill the
+  // bucket), else some count past most_above when a bucket passes that, else as it was
+  uint32_t* most      = nullptr;
+  uint32_t most_above = 0;
   // screen: survivors past a workgroup's LDS list go to the workgroup's own region of a pool of
   // spill_pool entries, with plain stores; the launcher splits the pool evenly among its
   // workgroups (spill_cap each), and the workgroup's flush moves its region into the buckets.
@@ -317,13 +321,25 @@ int tile_block_queries();
 
 /**
  * theta[q] = the k-th largest of gmax[q, 0 .. n_groups) (kKeepAll when n_groups < k, and never
- * below kKeepAll); padding queries q >= nq get kKeepNone.
+ * below kKeepAll); padding queries q >= nq get kKeepNone. Also clears count[q] for every q < nq_pad
+ * and the two words of `small`: the screen behind it counts into them.
  */
 void threshold_i8(const int32_t* gmax, int64_t n_groups, int64_t nq, int64_t nq_pad, int k,
-                  int32_t* theta, hipStream_t stream);
+                  int32_t* theta, uint32_t* count, uint32_t* small, hipStream_t stream);
 
-/** *out = max(count[0 .. n)). */
-void max_u32(const uint32_t* count, int64_t n, uint32_t* out, hipStream_t stream);
+/**
+ * Two device words that the host waits for, written to pinned host memory (words[0], words[1] to
+ * host[0], host[1], then ticket to host[2]) as a kernel starts: what the kernels before it left
+ * reaches the host while it runs, with no copy or event of its own. Null host: nothing.
+ */
+struct publish_args {
+  const uint32_t* words = nullptr;
+  uint32_t* host        = nullptr;
+  uint32_t ticket       = 0;
+};
+/** The publication by a kernel of its own. */
+void publish(const publish_args& a, hipStream_t stream);
+
 /** *out += sum(min(count[i], cap)) over i < n (64-bit). */
 void sum_u32(const uint32_t* count, int64_t n, int64_t cap, unsigned long long* out,
              hipStream_t stream);
@@ -336,7 +352,10 @@ struct verify_args {
   const uint32_t* cand_rows;
   int64_t cap;
   bool all_rows;
-  int64_t max_cand  = -1;  // the largest bucket count when the host knows it (else -1)
+  // part 1: buckets of at most kSmallBucket candidates (k <= 64), part 2: the others, 0: both. A
+  // caller that does not know the bucket counts yet launches part 1 and, if some count turns out
+  // larger, part 2
+  int part = 0;
   int64_t small_max = -1;  // set by the launcher: buckets up to this size take the one-wave path
   int64_t n_rows;         // rows of the index (all_rows)
   // vectors: integer codes (int path)
@@ -362,7 +381,11 @@ struct verify_args {
   float* distances;
   int64_t* neighbors;
   const int32_t* out_rows = nullptr;
+  publish_args publish;  // by the first kernel launched
 };
+
+/** Candidates per query up to which the integer re-rank runs without the block kernel (k <= 64). */
+constexpr int kSmallBucket = 512;
 
 /** fp64 exact scores of the candidates of every query and their k best by (score, row). */
 void verify_topk_i8(const verify_args& a, hipStream_t stream);
@@ -438,6 +461,8 @@ struct threshold_f_args {
   // testing only (null in searches): U per live query, the certified bound of its k-th
   // neighbour's score that theta is derived from (+inf when fewer than k groups count)
   double* ub = nullptr;
+  uint32_t* count = nullptr;  // cleared for every query (threshold_i8)
+  uint32_t* small = nullptr;  // two words, cleared
 };
 /**
  * theta[q] for fp16 rows, certified from the anchor pass alone: the k-th largest finite group
@@ -484,6 +509,7 @@ struct verify_f_args {
   float* distances;    // as in verify_args
   int64_t* neighbors;
   const int32_t* out_rows = nullptr;  // as in verify_args
+  publish_args publish;
 };
 /**
  * fp64 exact scores (the canonical order of the oracle) and top-k by (score, row); with screen

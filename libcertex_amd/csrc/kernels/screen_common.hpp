@@ -283,6 +283,28 @@ __device__ __forceinline__ void spill_put(const screen_args& a, int64_t e, uint3
 }
 
 /**
+ * Notes that a query's bucket count went from `old` to `now` (screen_args::most): the host reads
+ * one word instead of a kernel reading every count. Only counts past a limit get here to the
+ * atomic, and only those that raise the word: a word that every workgroup's atomic hits costs each
+ * about 10 ns of all others' time.
+ */
+__device__ __forceinline__ void note_count(const screen_args& a, uint32_t old, uint32_t now)
+{
+  if (now <= a.most_above) { return; }
+  if ((old <= a.most_above || now > a.cap) &&
+      __hip_atomic_load(a.most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < now) {
+    atomicMax(a.most, now);
+  }
+}
+
+/** A survivor counted by an atomic of its own, at slot `at`: every 64th of them past the bucket is
+ *  noted, and the ones that pass a limit. */
+__device__ __forceinline__ void note_slot(const screen_args& a, uint32_t at)
+{
+  if (at == a.most_above || at == a.cap || ((at & 63u) == 63u && at >= a.cap)) { note_count(a, at, at + 1); }
+}
+
+/**
  * LDS survivor list of a workgroup: hit_q / hit_row / hit_val (the screen values, when the rows
  * carry them) of `cap` entries (kHitCap, or what the K-loop screen's LDS leaves) and the count
  * n_hits, passed as separate pointers (a struct of LDS addresses can end up as a constant
@@ -393,6 +415,7 @@ __device__ __forceinline__ void push_hits(uint32_t bits, uint32_t qloc, int64_t 
     } else {
       const int64_t q   = q0 + qloc;
       const uint32_t at = atomicAdd(a.cand_count + q, 1u);
+      note_slot(a, at);
       if (at < a.cap) {
         a.cand_rows[q * a.cap + at] = uint32_t(row0) + d;
         if constexpr (VALS) { a.cand_vals[q * a.cap + at] = val; }
@@ -465,7 +488,12 @@ __device__ inline void flush_hits(int64_t q0, int64_t rbase, int qb, const scree
     __syncthreads();
   }
   for (int e = threadIdx.x; e < qb; e += blockDim.x) {
-    if (cnt[e] != 0) { cnt[e] = atomicAdd(a.cand_count + q0 + e, cnt[e]); }
+    if (cnt[e] != 0) {
+      const uint32_t n   = cnt[e];
+      const uint32_t old = atomicAdd(a.cand_count + q0 + e, n);
+      note_count(a, old, old + n);
+      cnt[e] = old;
+    }
   }
   __syncthreads();
   for (uint32_t e = threadIdx.x; e < nh; e += blockDim.x) {

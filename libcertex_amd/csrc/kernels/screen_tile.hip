@@ -441,6 +441,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void screen_tile_kernel(screen_
       } else {
         const int64_t q   = w.q0 + qloc;
         const uint32_t at = atomicAdd(a.cand_count + q, 1u);
+        note_slot(a, at);
         if (at < a.cap) {
           a.cand_rows[q * a.cap + at] = row;
           if constexpr (R::kValues) { a.cand_vals[q * a.cap + at] = val; }

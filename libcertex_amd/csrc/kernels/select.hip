@@ -23,6 +23,28 @@ namespace {
 
 constexpr int kThreads = 256;
 
+/** publish_args by thread 0 of block 0: the words, then the ticket that says they are there. */
+__device__ __forceinline__ void publish_words(const publish_args& p)
+{
+  if (p.host != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
+    __hip_atomic_store(p.host, p.words[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(p.host + 1, p.words[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(p.host + 2, p.ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+__global__ void publish_kernel(publish_args p) { publish_words(p); }
+
+/** The threshold kernels' second task (threshold_i8): query q's bucket count, and block 0 the two
+ *  words, cleared by one thread. */
+__device__ __forceinline__ void clear_counts(uint32_t* count, uint32_t* small, int64_t q)
+{
+  if (threadIdx.x == 0 && count != nullptr) {
+    count[q] = 0;
+    if (q == 0) { small[0] = small[1] = 0; }
+  }
+}
+
 /** Inclusive prefix sum over the T threads of a block of T = 64 (one wave), kThreads or 1024. */
 template <int T>
 __device__ inline int scan_incl_t(int v, int* wave_tot)
@@ -97,8 +119,9 @@ __device__ uint32_t radix_select_collect(int64_t n, int rank, F key_of, uint32_t
                                          int* sel_rank, uint32_t* list, int* n_list);
 
 __global__ __launch_bounds__(kThreads) void threshold_kernel(
-  const int32_t* gmax, int64_t n_groups, int64_t nq, int k, int32_t* theta)
+  const int32_t* gmax, int64_t n_groups, int64_t nq, int k, int32_t* theta, uint32_t* count, uint32_t* small)
 {
+  clear_counts(count, small, blockIdx.x);
   __shared__ int hist[257];
   __shared__ int wave_tot[4];
   __shared__ uint32_t red[48];
@@ -129,17 +152,6 @@ __global__ __launch_bounds__(kThreads) void threshold_kernel(
     const int32_t t = desc_value(key);
     theta[q]        = t > kKeepAll ? t : kKeepAll;
   }
-}
-
-__global__ void max_kernel(const uint32_t* c, int64_t n, uint32_t* out)
-{
-  uint32_t m = 0;
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * blockDim.x) {
-    m = max(m, c[i]);
-  }
-  m = lanes::max<64>(m);
-  if ((threadIdx.x & 63) == 0) { atomicMax(out, m); }
 }
 
 __global__ void sum_kernel(const uint32_t* c, int64_t n, int64_t cap, unsigned long long* out)
@@ -674,6 +686,7 @@ __device__ __forceinline__ code_row find_row(const verify_args& a, uint32_t r)
 template <int G>
 __global__ __launch_bounds__(kThreads) void verify_topk_i8_kernel(verify_args a, int cap)
 {
+  publish_words(a.publish);
   extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];
   auto* key = reinterpret_cast<uint64_t*>(dyn);                    // [cap]
   auto* rid = reinterpret_cast<uint32_t*>(dyn + size_t(cap) * 8);  // [cap]
@@ -770,9 +783,6 @@ __device__ __forceinline__ uint64_t wave_sizes(uint64_t k, bool descending)
   return k;
 }
 
-/** Candidates per query up to which the integer re-rank runs one wave per query. */
-constexpr int kSmallBucket = 512;
-
 /**
  * The integer re-rank for small buckets (at most kSmallBucket candidates, k <= 64): W waves per
  * query, each on every W-th run of CH candidates. Scores are whole numbers of 32 bits, so a
@@ -785,6 +795,7 @@ constexpr int kSmallBucket = 512;
 template <int G, int W, int CH>
 __global__ __launch_bounds__(W == 1 ? kThreads : 64 * W) void verify_topk_i8_small_kernel(verify_args a)
 {
+  publish_words(a.publish);
   __shared__ uint64_t lists[W > 1 ? (W - 1) * 64 : 1];
   const int lane  = threadIdx.x & 63;
   const int wave  = threadIdx.x >> 6;
@@ -1172,6 +1183,7 @@ __device__ inline double screen_upper_bound(float vf, const threshold_f_args& a,
  */
 __global__ __launch_bounds__(kThreads) void threshold_f16_cert_kernel(threshold_f_args a)
 {
+  clear_counts(a.count, a.small, blockIdx.x);
   __shared__ int hist[257];
   __shared__ int wave_tot[4];
   __shared__ uint32_t red[48];
@@ -1532,8 +1544,10 @@ __device__ uint32_t radix_select_regs(const uint32_t (&kk)[VPT], int rank, int* 
 /** threshold_kernel with the query's group maxima read once into registers (n_groups <= T VPT). */
 template <int T, int VPT>
 __global__ __launch_bounds__(T) void threshold_regs_kernel(const int32_t* gmax, int64_t n_groups,
-                                                           int64_t nq, int k, int32_t* theta)
+                                                           int64_t nq, int k, int32_t* theta,
+                                                           uint32_t* count, uint32_t* small)
 {
+  clear_counts(count, small, blockIdx.x);
   __shared__ int hist[256];
   __shared__ int wave_tot[16];
   __shared__ uint32_t red[48];
@@ -1568,6 +1582,7 @@ __global__ __launch_bounds__(T) void threshold_regs_kernel(const int32_t* gmax, 
 template <int T, int VPT>
 __global__ __launch_bounds__(T) void threshold_f16_cert_regs_kernel(threshold_f_args a)
 {
+  clear_counts(a.count, a.small, blockIdx.x);
   __shared__ int hist[256];
   __shared__ int wave_tot[16];
   __shared__ uint32_t red[48];
@@ -1616,9 +1631,9 @@ bool launch_select_regs(int64_t n, unsigned blocks, hipStream_t stream, Args... 
 template <int T, int VPT>
 struct threshold_regs_launch {
   static void go(unsigned blocks, hipStream_t stream, const int32_t* gmax, int64_t n_groups,
-                 int64_t nq, int k, int32_t* theta)
+                 int64_t nq, int k, int32_t* theta, uint32_t* count, uint32_t* small)
   {
-    threshold_regs_kernel<T, VPT><<<blocks, T, 0, stream>>>(gmax, n_groups, nq, k, theta);
+    threshold_regs_kernel<T, VPT><<<blocks, T, 0, stream>>>(gmax, n_groups, nq, k, theta, count, small);
   }
 };
 
@@ -1643,6 +1658,7 @@ template <int L>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(L == 64 ? 8 : 4)))
 void verify_topk_f_kernel(verify_f_args a, int cap)
 {
+  publish_words(a.publish);
   extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];
   auto* key = reinterpret_cast<uint64_t*>(dyn);                 // [cap]
   auto* rid = reinterpret_cast<uint32_t*>(dyn + size_t(cap) * 8);  // [cap]
@@ -1855,21 +1871,17 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
 }  // namespace
 
 void threshold_i8(const int32_t* gmax, int64_t n_groups, int64_t nq, int64_t nq_pad, int k,
-                  int32_t* theta, hipStream_t stream)
+                  int32_t* theta, uint32_t* count, uint32_t* small, hipStream_t stream)
 {
   if (nq_pad == 0) { return; }
   if (launch_select_regs<threshold_regs_launch>(n_groups, unsigned(nq_pad), stream, gmax, n_groups,
-                                                nq, k, theta)) {
+                                                nq, k, theta, count, small)) {
     return;
   }
-  threshold_kernel<<<unsigned(nq_pad), kThreads, 0, stream>>>(gmax, n_groups, nq, k, theta);
+  threshold_kernel<<<unsigned(nq_pad), kThreads, 0, stream>>>(gmax, n_groups, nq, k, theta, count, small);
 }
 
-void max_u32(const uint32_t* count, int64_t n, uint32_t* out, hipStream_t stream)
-{
-  const int64_t blocks = (n + 255) / 256 < 1024 ? (n + 255) / 256 : 1024;
-  if (blocks > 0) { max_kernel<<<unsigned(blocks), 256, 0, stream>>>(count, n, out); }
-}
+void publish(const publish_args& a, hipStream_t stream) { publish_kernel<<<1, 64, 0, stream>>>(a); }
 
 void sum_u32(const uint32_t* count, int64_t n, int64_t cap, unsigned long long* out,
              hipStream_t stream)
@@ -1886,20 +1898,22 @@ void verify_i8(const verify_args& a, hipStream_t stream)
   verify_args b = a;
   b.small_max   = -1;
   if (!a.all_rows && a.k <= 64) {
-    // buckets of up to kSmallBucket candidates: one wave per query; the block kernel then takes
-    // only the larger buckets (launched when the host saw one)
+    // buckets of up to kSmallBucket candidates by waves; the block kernel then takes only the
+    // larger buckets (part 2)
+    b.small_max = kSmallBucket;
     // fewer queries than fill the chip with waves: several waves per query, whose runs of
     // candidates then wait for memory at the same time (wide rows take shorter runs: a run is a row
     // after the other there)
-    if (a.nq <= 512) {
+    if (a.part == 2) {
+    } else if (a.nq <= 512) {
       verify_topk_i8_small_kernel<G, 8, G == 64 ? 16 : 64><<<unsigned(a.nq), 512, 0, stream>>>(a);
     } else if (a.nq <= 2048) {
       verify_topk_i8_small_kernel<G, 4, G == 64 ? 16 : 64><<<unsigned(a.nq), 256, 0, stream>>>(a);
     } else {
       verify_topk_i8_small_kernel<G, 1, 64><<<unsigned((a.nq + 3) / 4), kThreads, 0, stream>>>(a);
     }
-    if (a.max_cand >= 0 && a.max_cand <= kSmallBucket) { return; }
-    b.small_max = kSmallBucket;
+    if (a.part == 1) { return; }
+    b.publish = {};
   }
   // room for 2 k candidates (at least 1,024): small k keeps the block's LDS small, so that many
   // blocks share a CU
