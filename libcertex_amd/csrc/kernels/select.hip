@@ -17,6 +17,7 @@
 #include <cfloat>
 #include <climits>
 #include <cmath>
+#include <type_traits>
 
 namespace certex_amd {
 namespace {
@@ -65,15 +66,16 @@ __device__ inline int scan_incl_t(int v, int* wave_tot)
 }
 
 /** The largest of key[0, n) over the block (every thread gets it); scratch: 4 LDS words x 2. */
+template <int NT>
 __device__ inline uint64_t block_max_key(const uint64_t* key, int n, uint64_t* wave_max)
 {
   uint64_t m = 0;
-  for (int e = threadIdx.x; e < n; e += kThreads) { m = key[e] > m ? key[e] : m; }
+  for (int e = threadIdx.x; e < n; e += NT) { m = key[e] > m ? key[e] : m; }
   m = lanes::max<64>(m);
   if ((threadIdx.x & 63) == 0) { wave_max[threadIdx.x >> 6] = m; }
   __syncthreads();
   uint64_t r = wave_max[0];
-  for (int w = 1; w < kThreads / 64; ++w) { r = wave_max[w] > r ? wave_max[w] : r; }
+  for (int w = 1; w < NT / 64; ++w) { r = wave_max[w] > r ? wave_max[w] : r; }
   __syncthreads();
   return r;
 }
@@ -103,17 +105,17 @@ constexpr int kBatch = 8;
 __device__ inline uint32_t desc_key(int32_t v) { return ~(uint32_t(v) ^ 0x80000000u); }
 __device__ inline int32_t desc_value(uint32_t key) { return int32_t(~key ^ 0x80000000u); }
 
-template <typename F>
+template <int NT, typename F>
 __device__ uint32_t radix_select(int64_t n, int rank, F key_of, uint32_t lo, uint32_t hi, int* hist,
                                  int* wave_tot, uint32_t* sel_digit, int* sel_rank);
 
-template <typename F>
+template <int NT, typename F>
 __device__ void key_range(int64_t n, F key_of, uint32_t& lo, uint32_t& hi, int& below,
                           uint32_t* red);
 
 constexpr int kCollect = 2048;  // keys of the selected first digit copied into LDS, at most
 
-template <typename F>
+template <int NT, typename F>
 __device__ uint32_t radix_select_collect(int64_t n, int rank, F key_of, uint32_t lo, uint32_t hi,
                                          int* hist, int* wave_tot, uint32_t* sel_digit,
                                          int* sel_rank, uint32_t* list, int* n_list);
@@ -141,12 +143,12 @@ __global__ __launch_bounds__(kThreads) void threshold_kernel(
   auto key_of      = [&](int64_t e) { return desc_key(v[e]); };
   uint32_t lo, hi;
   int below;
-  key_range(n_groups, key_of, lo, hi, below, red);
+  key_range<kThreads>(n_groups, key_of, lo, hi, below, red);
   // the k-th largest value: the k-th smallest descending key (0xffffffff is the lowest value)
   __shared__ uint32_t list[kCollect];
   __shared__ int n_list;
   const uint32_t key = k > below ? 0xffffffffu
-                                 : radix_select_collect(n_groups, k, key_of, lo, hi, hist, wave_tot,
+                                 : radix_select_collect<kThreads>(n_groups, k, key_of, lo, hi, hist, wave_tot,
                                                         &sel_digit, &sel_rank, list, &n_list);
   if (tid == 0) {
     const int32_t t = desc_value(key);
@@ -343,11 +345,12 @@ struct row_slots {
 constexpr int kBuf = 4096;  // LDS candidates per query (keys 32 KB + rows 16 KB)
 
 /** Bitonic sort of key/row pairs [0, P) in LDS by (key, row); P a power of two. */
+template <int NT>
 __device__ inline void bitonic_sort(uint64_t* key, uint32_t* row, int P)
 {
   for (int size = 2; size <= P; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = threadIdx.x; i < (P >> 1); i += kThreads) {
+      for (int i = threadIdx.x; i < (P >> 1); i += NT) {
         const int lo  = 2 * i - (i & (stride - 1));
         const int hi  = lo + stride;
         const bool up = (lo & size) == 0;
@@ -373,7 +376,7 @@ __device__ __forceinline__ bool pair_less(uint64_t ka, uint32_t ra, uint64_t kb,
 }
 
 /**
- * One compare-exchange stage (SIZE, STRIDE) of bitonic_sort over kThreads E pairs held E per
+ * One compare-exchange stage (SIZE, STRIDE) of bitonic_sort over the block's pairs held E per
  * thread in registers, thread t holding positions t E .. t E + E - 1: within the thread for
  * STRIDE < E, by a cross-lane exchange for partners in the same wave (STRIDE < 64 E), else
  * through LDS (key / row, two barriers).
@@ -441,20 +444,20 @@ __device__ __forceinline__ void bitonic_strides_regs(uint64_t (&k)[E], uint32_t 
   if constexpr (STRIDE > 1) { bitonic_strides_regs<E, SIZE, STRIDE / 2>(k, r, key, row); }
 }
 
-template <int E, int SIZE>
+template <int NT, int E, int SIZE>
 __device__ __forceinline__ void bitonic_sizes_regs(uint64_t (&k)[E], uint32_t (&r)[E],
                                                    uint64_t* key, uint32_t* row)
 {
   bitonic_strides_regs<E, SIZE, SIZE / 2>(k, r, key, row);
-  if constexpr (SIZE < kThreads * E) { bitonic_sizes_regs<E, 2 * SIZE>(k, r, key, row); }
+  if constexpr (SIZE < NT * E) { bitonic_sizes_regs<NT, E, 2 * SIZE>(k, r, key, row); }
 }
 
 /**
- * bitonic_sort of exactly kThreads E pairs (the same network, the same result), the pairs held E
- * per thread in registers: of the 66 stages of 2,048 pairs only the 3 whose partners sit in
+ * bitonic_sort of exactly NT E pairs (the same network, the same result), the pairs held E per
+ * thread in registers: of the 66 stages of 2,048 pairs (NT = 256) only the 3 whose partners sit in
  * another wave go through LDS and barriers (every stage of the LDS sort takes a barrier).
  */
-template <int E>
+template <int NT, int E>
 __device__ void bitonic_sort_regs(uint64_t* key, uint32_t* row)
 {
   const int t = threadIdx.x;
@@ -466,7 +469,7 @@ __device__ void bitonic_sort_regs(uint64_t* key, uint32_t* row)
     r[e] = row[t * E + e];
   }
   __syncthreads();  // every pair is read before the cross-wave stages write
-  bitonic_sizes_regs<E, 2>(k, r, key, row);
+  bitonic_sizes_regs<NT, E, 2>(k, r, key, row);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     key[t * E + e] = k[e];
@@ -475,22 +478,22 @@ __device__ void bitonic_sort_regs(uint64_t* key, uint32_t* row)
   __syncthreads();
 }
 
-/** bitonic_sort; with REGS, the register form for 1,024 and 2,048 pairs (it takes about 130
+/** bitonic_sort; with REGS, the register form for 1,024 and 2,048 pairs (8 per thread take about 130
  *  VGPRs, which a kernel pays at every phase). */
-template <bool REGS>
+template <bool REGS, int NT>
 __device__ inline void sort_pairs(uint64_t* key, uint32_t* row, int P)
 {
   if constexpr (REGS) {
-    if (P == 8 * kThreads) {
-      bitonic_sort_regs<8>(key, row);
+    if (P == 2048) {
+      bitonic_sort_regs<NT, 2048 / NT>(key, row);
       return;
     }
-    if (P == 4 * kThreads) {
-      bitonic_sort_regs<4>(key, row);
+    if (P == 1024) {
+      bitonic_sort_regs<NT, 1024 / NT>(key, row);
       return;
     }
   }
-  bitonic_sort(key, row, P);
+  bitonic_sort<NT>(key, row, P);
 }
 
 __device__ inline int pow2_at_least(int v)
@@ -507,6 +510,7 @@ __device__ inline int pow2_at_least(int v)
  * thread of the block calls it and gets the same pair. Scratch: hist[256], wave_tot[4], and three
  * LDS words.
  */
+template <int NT>
 __device__ inline void select_pair(const uint64_t* key, const uint32_t* row, int n, int rank,
                                    bool with_row, int* hist, int* wave_tot, uint32_t* sel_digit,
                                    int* sel_rank, int* sel_count, uint64_t* out_key,
@@ -516,9 +520,9 @@ __device__ inline void select_pair(const uint64_t* key, const uint32_t* row, int
   // the keys' range: the bits that the smallest and the largest share are shared by every key (the
   // best scores of a query lie close together) and need no pass, whose counts would all go to one
   // histogram bin; the select runs 8 bits at a time from the first differing bit down
-  __shared__ uint64_t rng[2 * (kThreads / 64)];
+  __shared__ uint64_t rng[2 * (NT / 64)];
   uint64_t lo = ~0ull, hi = 0;
-  for (int e = tid; e < n; e += kThreads) {
+  for (int e = tid; e < n; e += NT) {
     const uint64_t kk = key[e];
     lo                = kk < lo ? kk : lo;
     hi                = kk > hi ? kk : hi;
@@ -527,14 +531,14 @@ __device__ inline void select_pair(const uint64_t* key, const uint32_t* row, int
   hi = lanes::max<64>(hi);
   if ((tid & 63) == 0) {
     rng[tid >> 6]                 = lo;
-    rng[kThreads / 64 + (tid >> 6)] = hi;
+    rng[NT / 64 + (tid >> 6)] = hi;
   }
   __syncthreads();
   lo = rng[0];
-  hi = rng[kThreads / 64];
-  for (int w = 1; w < kThreads / 64; ++w) {
+  hi = rng[NT / 64];
+  for (int w = 1; w < NT / 64; ++w) {
     lo = rng[w] < lo ? rng[w] : lo;
-    hi = rng[kThreads / 64 + w] > hi ? rng[kThreads / 64 + w] : hi;
+    hi = rng[NT / 64 + w] > hi ? rng[NT / 64 + w] : hi;
   }
   __syncthreads();
   int r           = lo == hi ? 0 : 64 - __builtin_clzll(lo ^ hi);  // bits below the common prefix
@@ -545,15 +549,15 @@ __device__ inline void select_pair(const uint64_t* key, const uint32_t* row, int
     const int w       = r < 8 ? r : 8;
     const int shift   = r - w;
     const uint64_t dm = (uint64_t(1) << w) - 1;
-    hist[tid] = 0;
+    if (tid < 256) { hist[tid] = 0; }
     __syncthreads();
-    for (int e = tid; e < n; e += kThreads) {
+    for (int e = tid; e < n; e += NT) {
       const uint64_t kk = key[e];
       if ((kk & mask) == prefix) { atomicAdd(&hist[int((kk >> shift) & dm)], 1); }
     }
     __syncthreads();
-    const int c    = hist[tid];
-    const int incl = scan_incl_t<kThreads>(c, wave_tot);
+    const int c    = tid < 256 ? hist[tid] : 0;
+    const int incl = scan_incl_t<NT>(c, wave_tot);
     if (incl - c < rank && rank <= incl) {
       *sel_digit = uint32_t(tid);
       *sel_rank  = rank - (incl - c);
@@ -572,7 +576,7 @@ __device__ inline void select_pair(const uint64_t* key, const uint32_t* row, int
   const int same = *sel_count;  // pairs whose key is the selected one
   uint32_t rp = 0, rm = 0;
   if (same == 1) {
-    for (int e = tid; e < n; e += kThreads) {
+    for (int e = tid; e < n; e += NT) {
       if (key[e] == prefix) { *sel_digit = row[e]; }
     }
     __syncthreads();
@@ -580,15 +584,15 @@ __device__ inline void select_pair(const uint64_t* key, const uint32_t* row, int
     __syncthreads();
   } else {
     for (int shift = 24; shift >= 0; shift -= 8) {
-      hist[tid] = 0;
+      if (tid < 256) { hist[tid] = 0; }
       __syncthreads();
-      for (int e = tid; e < n; e += kThreads) {
+      for (int e = tid; e < n; e += NT) {
         const uint32_t rr = row[e];
         if (key[e] == prefix && (rr & rm) == rp) { atomicAdd(&hist[(rr >> shift) & 255], 1); }
       }
       __syncthreads();
-      const int c    = hist[tid];
-      const int incl = scan_incl_t<kThreads>(c, wave_tot);
+      const int c    = tid < 256 ? hist[tid] : 0;
+      const int incl = scan_incl_t<NT>(c, wave_tot);
       if (incl - c < rank && rank <= incl) {
         *sel_digit = uint32_t(tid);
         *sel_rank  = rank - (incl - c);
@@ -613,23 +617,24 @@ constexpr int kSortBelow = 512;
  * pairs per thread at a time (all pairs of a thread in registers had taken 48 VGPRs, which bounded
  * the verify kernels' occupancy).
  */
+template <int NT>
 __device__ inline uint64_t keep_k_best(uint64_t* key, uint32_t* row, int n, int k, int* hist,
                                        int* wave_tot, uint32_t* sel_digit, int* sel_rank,
                                        int* sel_count, int* fill)
 {
   if (n <= kSortBelow) {  // few pairs: one bitonic sort costs fewer barriers than the select
     const int P = pow2_at_least(n);
-    for (int j = n + threadIdx.x; j < P; j += kThreads) {
+    for (int j = n + threadIdx.x; j < P; j += NT) {
       key[j] = ~0ull;
       row[j] = ~0u;
     }
     __syncthreads();
-    bitonic_sort(key, row, P);
+    bitonic_sort<NT>(key, row, P);
     return key[k - 1];
   }
   __shared__ uint64_t kth_key;
   __shared__ uint32_t kth_row;
-  select_pair(key, row, n, k, n > k, hist, wave_tot, sel_digit, sel_rank, sel_count, &kth_key,
+  select_pair<NT>(key, row, n, k, n > k, hist, wave_tot, sel_digit, sel_rank, sel_count, &kth_key,
               &kth_row);
   const uint64_t K = kth_key;
   if (n == k) { return K; }
@@ -639,19 +644,19 @@ __device__ inline uint64_t keep_k_best(uint64_t* key, uint32_t* row, int n, int 
   constexpr int kPer = 4;
   if (threadIdx.x == 0) { *fill = 0; }
   __syncthreads();
-  for (int c0 = 0; c0 < n; c0 += kThreads * kPer) {
+  for (int c0 = 0; c0 < n; c0 += NT * kPer) {
     uint64_t kk[kPer];
     uint32_t rr[kPer];
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int e = c0 + threadIdx.x + i * kThreads;
+      const int e = c0 + threadIdx.x + i * NT;
       kk[i]       = e < n ? key[e] : ~0ull;
       rr[i]       = e < n ? row[e] : ~0u;
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      const int e   = c0 + threadIdx.x + i * kThreads;
+      const int e   = c0 + threadIdx.x + i * NT;
       const bool in = e < n && (kk[i] < K || (kk[i] == K && rr[i] <= R));
       const int s   = wave_append(in, fill);
       if (in) {
@@ -736,14 +741,14 @@ __global__ __launch_bounds__(kThreads) void verify_topk_i8_kernel(verify_args a,
     __syncthreads();
     if (tid == 0) { fill = 0; }
     if (c0 < n_cand && have > k) {  // keep the k best, drop the rest
-      (void)keep_k_best(key, rid, have, k, hist, wave_tot, &sel_digit, &sel_rank, &sel_count,
+      (void)keep_k_best<kThreads>(key, rid, have, k, hist, wave_tot, &sel_digit, &sel_rank, &sel_count,
                         &kept);
       have = k;
     }
     __syncthreads();
   }
   if (have > k) {
-    (void)keep_k_best(key, rid, have, k, hist, wave_tot, &sel_digit, &sel_rank, &sel_count, &kept);
+    (void)keep_k_best<kThreads>(key, rid, have, k, hist, wave_tot, &sel_digit, &sel_rank, &sel_count, &kept);
     have = k;
   }
   const int P = pow2_at_least(have > 1 ? have : 1);
@@ -752,7 +757,7 @@ __global__ __launch_bounds__(kThreads) void verify_topk_i8_kernel(verify_args a,
     rid[j] = ~0u;
   }
   __syncthreads();
-  sort_pairs<false>(key, rid, P);
+  sort_pairs<false, kThreads>(key, rid, P);
   for (int j = tid; j < k; j += kThreads) {
     put_result(a, q, j, j < have ? key_score(key[j]) : 0.0, j < have ? int64_t(rid[j]) : -1);
   }
@@ -1204,7 +1209,7 @@ __global__ __launch_bounds__(kThreads) void threshold_f16_cert_kernel(threshold_
   };
   uint32_t lo, hi;
   int finite;
-  key_range(a.n_groups, key_of, lo, hi, finite, red);
+  key_range<kThreads>(a.n_groups, key_of, lo, hi, finite, red);
   if (finite < a.k) {
     // keep every live row: removed rows (screen value -inf) still fail
     if (tid == 0) {
@@ -1215,7 +1220,7 @@ __global__ __launch_bounds__(kThreads) void threshold_f16_cert_kernel(threshold_
   }
   __shared__ uint32_t list[kCollect];
   __shared__ int n_list;
-  const uint32_t key = radix_select_collect(a.n_groups, a.k, key_of, lo, hi, hist, wave_tot,
+  const uint32_t key = radix_select_collect<kThreads>(a.n_groups, a.k, key_of, lo, hi, hist, wave_tot,
                                             &sel_digit, &sel_rank, list, &n_list);
   if (tid == 0) {
     const double U = screen_upper_bound(key_value(~key), a, q);
@@ -1296,22 +1301,22 @@ __device__ inline void block_min_max_sum(uint32_t& lo, uint32_t& hi, int& n, uin
  * The smallest key lo, the largest key hi below 0xffffffff and the number of keys below
  * 0xffffffff among key_of(e), e < n, over the block (every thread gets them); red: 48 LDS words.
  */
-template <typename F>
+template <int NT, typename F>
 __device__ void key_range(int64_t n, F key_of, uint32_t& lo, uint32_t& hi, int& below, uint32_t* red)
 {
   lo    = 0xffffffffu;
   hi    = 0;
   below = 0;
-  for (int64_t e0 = 0; e0 < n; e0 += int64_t(kThreads) * kBatch) {
+  for (int64_t e0 = 0; e0 < n; e0 += int64_t(NT) * kBatch) {
     uint32_t kk[kBatch];
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      const int64_t e = e0 + i * kThreads + threadIdx.x;
+      const int64_t e = e0 + i * NT + threadIdx.x;
       kk[i]           = key_of(e < n ? e : n - 1);
     }
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      if (e0 + i * kThreads + threadIdx.x < n) {
+      if (e0 + i * NT + threadIdx.x < n) {
         lo = kk[i] < lo ? kk[i] : lo;
         if (kk[i] != 0xffffffffu) {
           hi = kk[i] > hi ? kk[i] : hi;
@@ -1320,7 +1325,7 @@ __device__ void key_range(int64_t n, F key_of, uint32_t& lo, uint32_t& hi, int& 
       }
     }
   }
-  block_min_max_sum<kThreads>(lo, hi, below, red);
+  block_min_max_sum<NT>(lo, hi, below, red);
 }
 
 /** The state of an LDS radix select: the bits fixed so far (prefix under mask), the bits below
@@ -1347,7 +1352,7 @@ __device__ inline radix_state radix_start(uint32_t lo, uint32_t hi, int rank)
  * that digit over the keys key_of(e), e < n, that share the prefix, and the digit that holds the
  * rank. Returns how many keys share the longer prefix. Every thread of the block calls it.
  */
-template <typename F>
+template <int NT, typename F>
 __device__ int radix_pass(int64_t n, F key_of, radix_state& st, int* hist, int* wave_tot,
                           uint32_t* sel_digit, int* sel_rank)
 {
@@ -1355,19 +1360,19 @@ __device__ int radix_pass(int64_t n, F key_of, radix_state& st, int* hist, int* 
   const int w       = st.r < 8 ? st.r : 8;
   const int shift   = st.r - w;
   const uint32_t dm = (1u << w) - 1u;
-  hist[tid]         = 0;
+  if (tid < 256) { hist[tid] = 0; }
   __syncthreads();
   int cur = -1, run_n = 0;  // a run of keys in one bin adds up before one atomic
-  for (int64_t e0 = 0; e0 < n; e0 += int64_t(kThreads) * kBatch) {
+  for (int64_t e0 = 0; e0 < n; e0 += int64_t(NT) * kBatch) {
     uint32_t kk[kBatch];  // loads first (from clamped positions), then the counts
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      const int64_t e = e0 + i * kThreads + tid;
+      const int64_t e = e0 + i * NT + tid;
       kk[i]           = key_of(e < n ? e : n - 1);
     }
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      if (e0 + i * kThreads + tid < n && (kk[i] & st.mask) == st.prefix) {
+      if (e0 + i * NT + tid < n && (kk[i] & st.mask) == st.prefix) {
         const int d = int((kk[i] >> shift) & dm);
         if (d == cur) {
           ++run_n;
@@ -1381,8 +1386,8 @@ __device__ int radix_pass(int64_t n, F key_of, radix_state& st, int* hist, int* 
   }
   if (run_n > 0) { atomicAdd(&hist[cur], run_n); }
   __syncthreads();
-  const int c    = hist[tid];
-  const int incl = scan_incl_t<kThreads>(c, wave_tot);
+  const int c    = tid < 256 ? hist[tid] : 0;
+  const int incl = scan_incl_t<NT>(c, wave_tot);
   if (incl - c < st.rank && st.rank <= incl) {
     *sel_digit = uint32_t(tid);
     *sel_rank  = st.rank - (incl - c);
@@ -1406,12 +1411,12 @@ __device__ int radix_pass(int64_t n, F key_of, radix_state& st, int* hist, int* 
  * sorts last and leaves the rank-th unchanged). Every thread of the block calls it and gets the
  * same key. hist holds 257 words.
  */
-template <typename F>
+template <int NT, typename F>
 __device__ uint32_t radix_select(int64_t n, int rank, F key_of, uint32_t lo, uint32_t hi, int* hist,
                                  int* wave_tot, uint32_t* sel_digit, int* sel_rank)
 {
   radix_state st = radix_start(lo, hi, rank);
-  while (st.r > 0) { (void)radix_pass(n, key_of, st, hist, wave_tot, sel_digit, sel_rank); }
+  while (st.r > 0) { (void)radix_pass<NT>(n, key_of, st, hist, wave_tot, sel_digit, sel_rank); }
   return st.prefix;
 }
 
@@ -1421,31 +1426,31 @@ __device__ uint32_t radix_select(int64_t n, int rank, F key_of, uint32_t lo, uin
  * other digits read them there instead of all n keys, which saves the row's reads of the digits
  * after it. The same key as radix_select.
  */
-template <typename F>
+template <int NT, typename F>
 __device__ uint32_t radix_select_collect(int64_t n, int rank, F key_of, uint32_t lo, uint32_t hi,
                                          int* hist, int* wave_tot, uint32_t* sel_digit,
                                          int* sel_rank, uint32_t* list, int* n_list)
 {
   radix_state st = radix_start(lo, hi, rank);
   if (st.r == 0) { return st.prefix; }
-  int count = radix_pass(n, key_of, st, hist, wave_tot, sel_digit, sel_rank);
+  int count = radix_pass<NT>(n, key_of, st, hist, wave_tot, sel_digit, sel_rank);
   while (st.r > 0 && count > kCollect) {
-    count = radix_pass(n, key_of, st, hist, wave_tot, sel_digit, sel_rank);
+    count = radix_pass<NT>(n, key_of, st, hist, wave_tot, sel_digit, sel_rank);
   }
   if (st.r > 0) {
     const int tid = threadIdx.x;
     if (tid == 0) { *n_list = 0; }
     __syncthreads();
-    for (int64_t e0 = 0; e0 < n; e0 += int64_t(kThreads) * kBatch) {
+    for (int64_t e0 = 0; e0 < n; e0 += int64_t(NT) * kBatch) {
       uint32_t kk[kBatch];
 #pragma unroll
       for (int i = 0; i < kBatch; ++i) {
-        const int64_t e = e0 + i * kThreads + tid;
+        const int64_t e = e0 + i * NT + tid;
         kk[i]           = key_of(e < n ? e : n - 1);
       }
 #pragma unroll
       for (int i = 0; i < kBatch; ++i) {
-        const bool take = e0 + i * kThreads + tid < n && (kk[i] & st.mask) == st.prefix;
+        const bool take = e0 + i * NT + tid < n && (kk[i] & st.mask) == st.prefix;
         const int slot  = wave_append(take, n_list);
         if (take) { list[slot] = kk[i]; }
       }
@@ -1453,7 +1458,7 @@ __device__ uint32_t radix_select_collect(int64_t n, int rank, F key_of, uint32_t
     __syncthreads();
     const int nl = *n_list;  // = count
     auto key_at  = [&](int64_t e) { return list[e]; };
-    while (st.r > 0) { (void)radix_pass(nl, key_at, st, hist, wave_tot, sel_digit, sel_rank); }
+    while (st.r > 0) { (void)radix_pass<NT>(nl, key_at, st, hist, wave_tot, sel_digit, sel_rank); }
   }
   return st.prefix;
 }
@@ -1615,6 +1620,13 @@ __global__ __launch_bounds__(T) void threshold_f16_cert_regs_kernel(threshold_f_
   }
 }
 
+/**
+ * Queries up to which the float re-rank gives each a block of 1,024 threads (one block per CU, by
+ * its registers) instead of 256 (four): a block works alone on its query there, and most of its
+ * phases wait for memory or barriers.
+ */
+constexpr int64_t kBigBlockQueries = 256;
+
 /** Launches K<T, VPT> for the smallest register shape holding n keys per query, one block per
  *  query; false when n exceeds the largest shape (the streaming kernel then runs). */
 template <template <int, int> class L, typename... Args>
@@ -1624,6 +1636,11 @@ bool launch_select_regs(int64_t n, unsigned blocks, hipStream_t stream, Args... 
   if (n <= 64 * 16) { L<64, 16>::go(blocks, stream, args...); return true; }
   if (n <= kThreads * 8) { L<kThreads, 8>::go(blocks, stream, args...); return true; }
   if (n <= kThreads * 16) { L<kThreads, 16>::go(blocks, stream, args...); return true; }
+  if (blocks <= kBigBlockQueries) {  // one block per CU: more threads, fewer values each
+    if (n <= 1024 * 8) { L<1024, 8>::go(blocks, stream, args...); return true; }
+    if (n <= 1024 * 18) { L<1024, 18>::go(blocks, stream, args...); return true; }
+  }
+  if (n <= kThreads * 32) { L<kThreads, 32>::go(blocks, stream, args...); return true; }
   if (n <= kThreads * 72) { L<kThreads, 72>::go(blocks, stream, args...); return true; }
   return false;  // larger tables: the streaming kernels
 }
@@ -1654,8 +1671,8 @@ struct threshold_f_regs_launch {
  * stay in LDS. With 64-lane slots (d above 256) eight waves per SIMD, as many blocks as the LDS of a
  * CU holds at config 3 (18 spilled registers; against six waves per SIMD, verify 0.82 -> 0.79 ms).
  */
-template <int L>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(L == 64 ? 8 : 4)))
+template <int L, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(L == 64 && NT == kThreads ? 8 : 4)))
 void verify_topk_f_kernel(verify_f_args a, int cap)
 {
   publish_words(a.publish);
@@ -1664,7 +1681,7 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
   auto* rid = reinterpret_cast<uint32_t*>(dyn + size_t(cap) * 8);  // [cap]
   auto* qv  = reinterpret_cast<double*>(dyn + size_t(cap) * 12);  // [query_coords]
   __shared__ int hist[257];
-  __shared__ int wave_tot[4];
+  __shared__ int wave_tot[16];
   __shared__ uint32_t red[48];
   __shared__ uint32_t sel_digit;
   __shared__ int sel_rank;
@@ -1673,15 +1690,15 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
   // survivors whose screen values phase A selects in registers, 24 per thread; not with 64-lane
   // slots (d above 256), whose waves leave no registers to spare (16 per thread at six waves per
   // SIMD measured 4% slower than the streaming select, config 3)
-  constexpr bool REGS = L != 64;
-  constexpr int RV    = 24;
+  constexpr bool REGS = L != 64 || NT == 1024;
+  constexpr int RV    = NT == 1024 ? 8 : 24;
 
   const int64_t q = blockIdx.x;
   const int tid   = threadIdx.x;
   const int k     = a.k;
   const int64_t qr = a.query_rows != nullptr ? int64_t(a.query_rows[q]) : q;
   const int64_t qn = query_coords(L, a.dim);
-  for (int64_t j = tid; j < qn; j += kThreads) {
+  for (int64_t j = tid; j < qn; j += NT) {
     qv[j] = j < a.dim ? fcoord(a.queries, a.t, qr * a.dim + j) : 0.0;
   }
   double qq = 0;
@@ -1702,17 +1719,17 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
   int64_t n_scored = 0;
   auto score       = [&](int from, int to) {
     n_scored += to - from;
-    score_rows_l<L, kThreads>(qv, qq, a.vectors, a.t, a.dim, a.metric, rid, key, from, to);
+    score_rows_l<L, NT>(qv, qq, a.vectors, a.t, a.dim, a.metric, rid, key, from, to);
   };
   int have = 0;  // entries [0, have) of key / rid are scored
   // the k best so far move to [0, k) (unordered); the k-th key bounds the k-th score. With
   // exactly k entries the k-th key is their largest, and nothing moves
-  __shared__ uint64_t wave_max[kThreads / 64];
+  __shared__ uint64_t wave_max[NT / 64];
   uint64_t kth = ~0ull;
   auto keep_best = [&]() {
     if (have < k) { return; }
-    kth  = have == k ? block_max_key(key, k, wave_max)
-                     : keep_k_best(key, rid, have, k, hist, wave_tot, &sel_digit, &sel_rank,
+    kth  = have == k ? block_max_key<NT>(key, k, wave_max)
+                     : keep_k_best<NT>(key, rid, have, k, hist, wave_tot, &sel_digit, &sel_rank,
                                    &sel_count, &fill);
     have = k;
   };
@@ -1721,21 +1738,21 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
   bool ordered = vals != nullptr && n_cand > k;
   uint32_t tk  = 0;
   double U = INFINITY, aq = 0, C = 0;
-  if (REGS && ordered && n_cand <= int64_t(kThreads) * RV) {
+  if (REGS && ordered && n_cand <= int64_t(NT) * RV) {
     // the survivors' screen values read once into registers (RV per thread; 0xffffffff past the
     // bucket sorts last), selected there, and the k best collected from the same registers
     uint32_t kk[RV];
 #pragma unroll
     for (int i = 0; i < RV; ++i) {
-      const int64_t e = int64_t(i) * kThreads + tid;
+      const int64_t e = int64_t(i) * NT + tid;
       kk[i]           = e < n_cand ? ~fkey(vals[e]) : 0xffffffffu;
     }
-    tk = radix_select_regs<kThreads, RV>(kk, k, hist, wave_tot, red, &sel_digit, &sel_rank);
+    tk = radix_select_regs<NT, RV>(kk, k, hist, wave_tot, red, &sel_digit, &sel_rank);
     if (tid == 0) { fill = 0; }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < RV; ++i) {
-      const int64_t e = int64_t(i) * kThreads + tid;
+      const int64_t e = int64_t(i) * NT + tid;
       const bool take = e < n_cand && kk[i] <= tk;
       const int slot  = wave_append(take, &fill);
       if (take && slot < cap) { rid[slot] = to_id(cand[e]); }
@@ -1747,21 +1764,21 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
     auto key_of = [&](int64_t e) { return ~fkey(vals[e]); };
     uint32_t lo, hi;
     int below;
-    key_range(n_cand, key_of, lo, hi, below, reinterpret_cast<uint32_t*>(hist));
-    tk = k <= below ? radix_select(n_cand, k, key_of, lo, hi, hist, wave_tot, &sel_digit, &sel_rank)
-                    : radix_select(n_cand, k, key_of, 0u, 0xfffffffeu, hist, wave_tot, &sel_digit, &sel_rank);
+    key_range<NT>(n_cand, key_of, lo, hi, below, red);
+    tk = k <= below ? radix_select<NT>(n_cand, k, key_of, lo, hi, hist, wave_tot, &sel_digit, &sel_rank)
+                    : radix_select<NT>(n_cand, k, key_of, 0u, 0xfffffffeu, hist, wave_tot, &sel_digit, &sel_rank);
     if (tid == 0) { fill = 0; }
     __syncthreads();
-    for (int64_t e0 = 0; e0 < n_cand; e0 += int64_t(kThreads) * kBatch) {
+    for (int64_t e0 = 0; e0 < n_cand; e0 += int64_t(NT) * kBatch) {
       float v[kBatch];
 #pragma unroll
       for (int i = 0; i < kBatch; ++i) {
-        const int64_t e = e0 + i * kThreads + tid;
+        const int64_t e = e0 + i * NT + tid;
         v[i]            = vals[e < n_cand ? e : n_cand - 1];
       }
 #pragma unroll
       for (int i = 0; i < kBatch; ++i) {
-        const int64_t e = e0 + i * kThreads + tid;
+        const int64_t e = e0 + i * NT + tid;
         const bool take = e < n_cand && ~fkey(v[i]) <= tk;
         const int slot  = wave_append(take, &fill);
         if (take && slot < cap) { rid[slot] = to_id(cand[e]); }
@@ -1802,11 +1819,11 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
     const int64_t m = wide || n_cand - c0 < room ? n_cand - c0 : room;
     if (tid == 0) { fill = 0; }
     __syncthreads();
-    for (int64_t e0 = 0; e0 < m; e0 += int64_t(kThreads) * kBatch) {
+    for (int64_t e0 = 0; e0 < m; e0 += int64_t(NT) * kBatch) {
       bool take[kBatch];
 #pragma unroll
       for (int i = 0; i < kBatch; ++i) {
-        const int64_t e   = e0 + i * kThreads + tid;
+        const int64_t e   = e0 + i * NT + tid;
         const int64_t idx = c0 + (e < m ? e : m - 1);  // loads from clamped positions
         if (a.all_rows) {
           take[i] = a.rowc[idx] != -INFINITY && keeps(a.filter, q, uint32_t(idx));
@@ -1822,7 +1839,7 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
       for (int i = 0; i < kBatch; ++i) {
         const int slot = wave_append(take[i], &fill);
         if (take[i] && slot < room) {
-          const int64_t idx = c0 + e0 + i * kThreads + tid;
+          const int64_t idx = c0 + e0 + i * NT + tid;
           rid[have + slot]  = a.all_rows ? listed_id(a.filter, uint32_t(idx)) : to_id(cand[idx]);
         }
       }
@@ -1853,15 +1870,15 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
      // k come first), else a cut back to the k best and a sort of those
     if (have > kSortBelow) { keep_best(); }
     const int P = pow2_at_least(have > 1 ? have : 1);
-    for (int j = have + tid; j < P; j += kThreads) {
+    for (int j = have + tid; j < P; j += NT) {
       key[j] = ~0ull;
       rid[j] = ~0u;
     }
     __syncthreads();
-    sort_pairs<L == 16>(key, rid, P);
+    sort_pairs<L == 16 || NT == 1024, NT>(key, rid, P);
     have = have < k ? have : k;
   }
-  for (int j = tid; j < k; j += kThreads) {
+  for (int j = tid; j < k; j += NT) {
     put_result(a, q, j, j < have ? key_score(key[j]) : 0.0, j < have ? int64_t(rid[j]) : -1);
   }
   if (a.scored != nullptr && tid == 0) { atomicAdd(a.scored, (unsigned long long)n_scored); }
@@ -1935,7 +1952,7 @@ void verify_topk_i8(const verify_args& a, hipStream_t stream)
 }
 
 /** Launches a kernel with `bytes` of dynamic LDS (raising the kernel's limit when needed). */
-template <typename K, typename... Args>
+template <int NT, typename K, typename... Args>
 void launch_dyn(K kernel, unsigned blocks, size_t bytes, hipStream_t stream, Args... args)
 {
   if (bytes > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -1943,7 +1960,7 @@ void launch_dyn(K kernel, unsigned blocks, size_t bytes, hipStream_t stream, Arg
                                            int(bytes)) != hipSuccess) {
     (void)hipGetLastError();
   }
-  kernel<<<blocks, kThreads, bytes, stream>>>(args...);
+  kernel<<<blocks, NT, bytes, stream>>>(args...);
 }
 
 void threshold_f16(const threshold_f_args& a, hipStream_t stream)
@@ -1971,13 +1988,22 @@ void verify_topk_f(const verify_f_args& a, hipStream_t stream)
   int cap = (3 * a.k / 2 + 255) / 256 * 256;
   cap     = cap > pow2_ge(a.k) ? cap : pow2_ge(a.k);
   cap     = cap > 1024 ? (cap < kBuf ? cap : kBuf) : 1024;
+  const bool big      = a.nq <= kBigBlockQueries;
   const int L         = score_lanes(a.dim);
   const size_t bytes  = size_t(cap) * 12 + size_t(query_coords(L, a.dim)) * 8;
   const unsigned grid = unsigned(a.nq);
+  const auto go = [&](auto lanes) {
+    constexpr int N = decltype(lanes)::value;
+    if (big) {
+      launch_dyn<1024>(verify_topk_f_kernel<N, 1024>, grid, bytes, stream, a, cap);
+    } else {
+      launch_dyn<kThreads>(verify_topk_f_kernel<N, kThreads>, grid, bytes, stream, a, cap);
+    }
+  };
   switch (L) {
-    case 16: launch_dyn(verify_topk_f_kernel<16>, grid, bytes, stream, a, cap); break;
-    case 32: launch_dyn(verify_topk_f_kernel<32>, grid, bytes, stream, a, cap); break;
-    default: launch_dyn(verify_topk_f_kernel<64>, grid, bytes, stream, a, cap); break;
+    case 16: go(std::integral_constant<int, 16>{}); break;
+    case 32: go(std::integral_constant<int, 32>{}); break;
+    default: go(std::integral_constant<int, 64>{}); break;
   }
 }
 
