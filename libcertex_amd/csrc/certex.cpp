@@ -1191,29 +1191,36 @@ void search_batch_float(cuvs::resources const& res, index_state const& st, const
     va.n_part   = st.label_part.n;
   }
   // the exact re-rank over the buckets as they are, or over every row (all_rows)
-  auto verify = [&](bool every_row, certex_amd::publish_args pub) {
+  auto verify = [&](bool every_row, int part, certex_amd::publish_args pub) {
+    va.part       = part;
     va.cand_count = count;
     va.cand_rows  = rows;
     va.cand_vals  = vals;
     va.cap        = cap;
     va.all_rows   = every_row;
     va.publish    = pub;
-    if (scored != nullptr) { certex_amd::fill_u32(reinterpret_cast<uint32_t*>(scored), 2, 0, stream); }
+    if (scored != nullptr && part != 2) {
+      certex_amd::fill_u32(reinterpret_cast<uint32_t*>(scored), 2, 0, stream);
+    }
     timed(3, stream, [&] { certex_amd::verify_topk_f(va, stream); });
   };
   bool verified = false;
   // a capture reads the buckets before the verification (which compacts them in place)
   const bool capture = t_capture.on;
+  const bool waves   = k <= 64;  // part 1 of the re-rank covers buckets of up to small_bucket_f
+  bool large         = true;
   if (!all_rows) {
     sa.theta = theta;
     all_rows = !screen_into_buckets(
       res, nq_pad, size, sa,
       screen_pass(st, route, wide ? certex_amd::screen_f16_tile : certex_amd::screen_f16), bc, rows,
-      cap, &vals, INT32_MAX, nullptr, [&](certex_amd::publish_args pub) {
-        if (!capture) { verify(false, pub); }
+      cap, &vals, waves ? certex_amd::small_bucket_f(B) : INT32_MAX, &large,
+      [&](certex_amd::publish_args pub) {
+        if (!capture) { verify(false, waves ? 1 : 0, pub); }
         return !capture;
       });
     verified = !all_rows && !capture;
+    if (verified && waves && large) { verify(false, 2, {}); }
   }
   if (capture) {
     capture_common(st, tp, B, nq_pad, k, all_rows, cap, route, stream);
@@ -1244,11 +1251,11 @@ void search_batch_float(cuvs::resources const& res, index_state const& st, const
     CERTEX_HIP_TRY(hipStreamSynchronize(stream));
     t_capture.on = false;
     if (!all_rows) {
-      verify(false, {});
+      verify(false, 0, {});
       verified = true;
     }
   }
-  if (!verified) { verify(true, {}); }
+  if (!verified) { verify(true, 0, {}); }
   count_stats(res, st, B, all_rows, count, cap, true);
   if (scored != nullptr) {
     CERTEX_HIP_TRY(hipMemcpyAsync(rs.host_small, scored, 8, hipMemcpyDeviceToHost, stream));

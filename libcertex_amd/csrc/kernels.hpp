@@ -510,7 +510,14 @@ struct verify_f_args {
   int64_t* neighbors;
   const int32_t* out_rows = nullptr;  // as in verify_args
   publish_args publish;
+  int part          = 0;   // as in verify_args, buckets of at most small_bucket_f candidates
+  int64_t small_max = -1;  // set by the launcher: buckets up to this size are the small kernel's
 };
+
+/** Candidates per query up to which the float re-rank of nq queries takes the small kernel (k <=
+ *  64): 1,024, what 64 neighbours leave on average at an anchor stride of 16; twice that for few
+ *  queries, which get twice the waves. */
+int64_t small_bucket_f(int64_t nq);
 /**
  * fp64 exact scores (the canonical order of the oracle) and top-k by (score, row); with screen
  * values, only the candidates whose certified lower bound can reach the top k are scored.

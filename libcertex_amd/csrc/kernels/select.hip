@@ -46,11 +46,11 @@ __device__ __forceinline__ void clear_counts(uint32_t* count, uint32_t* small, i
   }
 }
 
-/** Inclusive prefix sum over the T threads of a block of T = 64 (one wave), kThreads or 1024. */
+/** Inclusive prefix sum over the T threads of a block. */
 template <int T>
 __device__ inline int scan_incl_t(int v, int* wave_tot)
 {
-  static_assert(T == 64 || T == kThreads || T == 1024, "block shapes of the selects");
+  static_assert(T % 64 == 0 && T <= 1024, "whole waves");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int incl = lanes::scan_incl(v);
   if constexpr (T == 64) {
@@ -840,7 +840,7 @@ __global__ __launch_bounds__(W == 1 ? kThreads : 64 * W) void verify_topk_i8_sma
     if (wave > 0) { return; }
     for (int w = 1; w < W && w * CH < n_cand; ++w) {
       const uint64_t key = lists[(w - 1) * 64 + lane];
-      if (!__any(key < best)) { continue; }
+      if (!__any(key < best)) { continue; }  // key descends: none of it is among the 64 smallest
       best = key < best ? key : best;
       best = wave_strides<64, 32>(best, true);
     }
@@ -1696,6 +1696,7 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
   const int64_t q = blockIdx.x;
   const int tid   = threadIdx.x;
   const int k     = a.k;
+  if (!a.all_rows && a.cand_count[q] <= a.small_max) { return; }  // the small kernel's query
   const int64_t qr = a.query_rows != nullptr ? int64_t(a.query_rows[q]) : q;
   const int64_t qn = query_coords(L, a.dim);
   for (int64_t j = tid; j < qn; j += NT) {
@@ -1885,6 +1886,179 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
 }
 
 
+/** The bitonic sort of 64 (key, id) pairs, one per lane, ascending by (key, id). */
+template <int SIZE, int STRIDE>
+__device__ __forceinline__ void wave_pair_strides(uint64_t& k, uint32_t& r)
+{
+  const uint64_t ok = lanes::exchange<STRIDE>(k);
+  const uint32_t orr = lanes::exchange<STRIDE>(r);
+  const bool lower  = (threadIdx.x & STRIDE) == 0;
+  const bool up     = (threadIdx.x & SIZE & 63) == 0;
+  if (pair_less(k, r, ok, orr) != (lower == up)) {
+    k = ok;
+    r = orr;
+  }
+  if constexpr (STRIDE > 1) { wave_pair_strides<SIZE, STRIDE / 2>(k, r); }
+}
+template <int SIZE>
+__device__ __forceinline__ void wave_pair_sort(uint64_t& k, uint32_t& r)
+{
+  wave_pair_strides<SIZE, SIZE / 2>(k, r);
+  if constexpr (SIZE < 64) { wave_pair_sort<SIZE * 2>(k, r); }
+}
+
+/** Survivors per thread of the small float re-rank, in registers. */
+constexpr int kSmallValues = 4;
+
+/**
+ * The ordered re-rank (verify_topk_f_kernel) of queries with at most 64 W kSmallValues survivors
+ * (small_bucket_f) and k <= 64: W waves per query. What bounds such a query is the chain of its phases, each a round of
+ * memory or barriers, not their work: here the survivors' screen values stay in registers, the k
+ * best values come from a sort over the lanes and a merge of the waves' lists (no radix passes),
+ * and the results from one wave's sort, with 6 barriers in the usual case instead of about 40.
+ * Queries with more survivors are left to the block kernel. 2,048 queries over 300 float32
+ * coordinates, k = 15: 47 -> 26 us; 16 queries over 768, k = 10: 29 -> 17 us; 1,000 over 128: 30 ->
+ * 19 us.
+ */
+template <int L, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(L == 64 ? 6 : 4)))
+void verify_topk_f_small_kernel(verify_f_args a)
+{
+  publish_words(a.publish);
+  constexpr int NT = 64 * W;
+  constexpr int RV = kSmallValues;
+  constexpr int CAP = 64 + NT > 512 ? 2048 : 512;  // entries: the k best and one round of survivors
+  static_assert(CAP >= 64 + NT, "the buffer takes a round");
+  extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];
+  auto* qv  = reinterpret_cast<double*>(dyn);  // [query_coords]
+  __shared__ uint64_t key[CAP];
+  __shared__ uint32_t rid[CAP];
+  __shared__ int hist[256];
+  __shared__ int wave_tot[16];
+  __shared__ uint32_t sel_digit;
+  __shared__ int sel_rank, sel_count, kept, fill;
+
+  const int64_t q = blockIdx.x;
+  const int tid   = threadIdx.x;
+  const int lane  = tid & 63, wave = tid >> 6;
+  const int k     = a.k;
+  const int64_t qr = a.query_rows != nullptr ? int64_t(a.query_rows[q]) : q;
+  const int n_cand = int(a.cand_count[q] < a.cap ? int64_t(a.cand_count[q]) : a.cap);
+  if (n_cand > RV * NT) { return; }
+  const uint32_t* cand = a.cand_rows + q * a.cap;
+  const float* vals    = a.cand_vals + q * a.cap;
+  auto to_id = [&](uint32_t r) {
+    return (a.part_ids != nullptr && r < a.n_part) ? uint32_t(a.part_ids[r]) : listed_id(a.filter, r);
+  };
+  // survivor e = i NT + tid of round i: its descending screen value (0xffffffff past the bucket)
+  uint32_t kk[RV];
+#pragma unroll
+  for (int i = 0; i < RV; ++i) {
+    const int e = i * NT + tid;
+    kk[i]       = e < n_cand ? ~fkey(vals[e]) : 0xffffffffu;
+  }
+  const int64_t qn = query_coords(L, a.dim);
+  for (int64_t j = tid; j < qn; j += NT) { qv[j] = j < a.dim ? fcoord(a.queries, a.t, qr * a.dim + j) : 0.0; }
+  auto kth_of = [&](uint64_t b) {  // lane k - 1's of a sorted list
+    const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(b)), k - 1));
+    const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(b >> 32), k - 1));
+    return (uint64_t(hi) << 32) | lo;
+  };
+  // the wave's k best (and some more, up to 64) of its survivors by (value, place)
+  uint64_t best = ~0ull;
+#pragma unroll
+  for (int i = 0; i < RV; ++i) {
+    if (i * NT + wave * 64 >= n_cand) { break; }  // uniform
+    const uint64_t x = (uint64_t(kk[i]) << 32) | uint32_t(i * NT + tid);
+    if (i == 0) {
+      best = wave_sizes<2>(x, false);
+    } else if (__any(x < kth_of(best))) {
+      const uint64_t y = wave_sizes<2>(x, true);
+      best             = y < best ? y : best;
+      best             = wave_strides<64, 32>(best, true);
+    }
+  }
+  if (wave > 0 && wave * 64 < n_cand) { key[wave * 64 + 63 - lane] = best; }  // descending, for the merge
+  __syncthreads();
+  double qq = 0;
+  if (a.metric == metric_kind::cosine) { qq = query_square(qv, qn); }
+  const int top = n_cand < k ? n_cand : k;  // scored first
+  uint64_t* kth = key + CAP - 1;
+  if (wave == 0) {
+    for (int w = 1; w < W && w * 64 < n_cand; ++w) {
+      const uint64_t x = key[w * 64 + lane];
+      if (!__any(x < best)) { continue; }  // x descends: none of it is among the 64 smallest
+      best = x < best ? x : best;
+      best = wave_strides<64, 32>(best, true);
+    }
+    if (lane < top) { rid[lane] = to_id(cand[uint32_t(best)]); }
+    if (lane == top - 1) { *kth = best; }
+    if (lane == 0) { fill = 0; }
+  }
+  __syncthreads();
+  const uint64_t last = *kth;  // (value, place) of the last one scored first
+  int64_t n_scored    = 0;
+  auto score          = [&](int from, int to) {
+    n_scored += to - from;
+    score_rows_l<L, NT>(qv, qq, a.vectors, a.t, a.dim, a.metric, rid, key, from, to);
+    __syncthreads();
+  };
+  int have = top;
+  __syncthreads();  // *kth is read before the scores take its place
+  if (top > 0) { score(0, top); }
+  if (n_cand > k) {
+    // the rest: the survivors whose certified lower bound does not exceed the k-th score so far
+    const double nw = a.qscal[3 * q + 1], ew = a.qscal[3 * q + 2];
+    const double nz = a.maxima[0], ez = a.maxima[1];
+    const double aq = a.qscal[3 * q];
+    const double C  = a.gamma * nw * nz + ew * nz + nw * ez + ew * ez;
+    double U        = key_score(lanes::max<64>(lane < k ? key[lane] : 0ull));
+    int pending     = have;
+#pragma unroll
+    for (int i = 0; i < RV; ++i) {
+      if (i * NT >= n_cand) { break; }  // uniform over the block
+      const uint64_t x = (uint64_t(kk[i]) << 32) | uint32_t(i * NT + tid);
+      bool take        = kk[i] != 0xffffffffu && x > last;
+      if (take) { take = screen_lower_bound(key_value(~kk[i]), aq, C, a.alpha2, a.metric) <= U; }
+      const int slot = wave_append(take, &fill);
+      if (take) { rid[have + slot] = to_id(cand[i * NT + tid]); }
+      const bool end = (i + 1) * NT >= n_cand;
+      __syncthreads();
+      const int added = fill;
+      __syncthreads();
+      have += added;
+      if (tid == 0) { fill = 0; }
+      if (have > pending && (end || have + NT > CAP)) {
+        score(pending, have);
+        pending = have;
+        if (!end && have > k) {
+          U = key_score(keep_k_best<NT>(key, rid, have, k, hist, wave_tot, &sel_digit, &sel_rank, &sel_count, &kept));
+          have = pending = k;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  // the k best in (score, id) order
+  if (have > 64) {
+    const int P = pow2_at_least(have);
+    for (int j = have + tid; j < P; j += NT) {
+      key[j] = ~0ull;
+      rid[j] = ~0u;
+    }
+    __syncthreads();
+    bitonic_sort<NT>(key, rid, P);
+    for (int j = tid; j < k; j += NT) { put_result(a, q, j, key_score(key[j]), int64_t(rid[j])); }
+  } else if (wave == 0) {
+    uint64_t x = lane < have ? key[lane] : ~0ull;
+    uint32_t r = lane < have ? rid[lane] : ~0u;
+    wave_pair_sort<2>(x, r);
+    if (lane < k) { put_result(a, q, lane, lane < have ? key_score(x) : 0.0, lane < have ? int64_t(r) : -1); }
+  }
+  if (a.scored != nullptr && tid == 0) { atomicAdd(a.scored, (unsigned long long)n_scored); }
+}
+
+
 }  // namespace
 
 void threshold_i8(const int32_t* gmax, int64_t n_groups, int64_t nq, int64_t nq_pad, int k,
@@ -1980,9 +2154,43 @@ void certificate_bounds(const threshold_f_args& a, const uint32_t* count, const 
   certificate_bounds_kernel<<<grid, 256, 0, stream>>>(a, count, vals, cap, lb, ub);
 }
 
+int64_t small_bucket_f(int64_t nq) { return 64 * (nq <= kBigBlockQueries ? 8 : 4) * kSmallValues; }
+
+namespace {
+
+void verify_small_f(const verify_f_args& a, hipStream_t stream)
+{
+  const int L         = score_lanes(a.dim);
+  const size_t bytes  = size_t(query_coords(L, a.dim)) * 8;
+  const unsigned grid = unsigned(a.nq);
+  const auto go       = [&](auto lanes) {
+    constexpr int N = decltype(lanes)::value;
+    if (a.nq <= kBigBlockQueries) {
+      launch_dyn<512>(verify_topk_f_small_kernel<N, 8>, grid, bytes, stream, a);
+    } else {
+      launch_dyn<256>(verify_topk_f_small_kernel<N, 4>, grid, bytes, stream, a);
+    }
+  };
+  switch (L) {
+    case 16: go(std::integral_constant<int, 16>{}); break;
+    case 32: go(std::integral_constant<int, 32>{}); break;
+    default: go(std::integral_constant<int, 64>{}); break;
+  }
+}
+
+}  // namespace
+
 void verify_topk_f(const verify_f_args& a, hipStream_t stream)
 {
   if (a.nq == 0) { return; }
+  verify_f_args b = a;
+  b.small_max     = -1;
+  if (!a.all_rows && a.cand_vals != nullptr && a.k <= 64) {
+    b.small_max = small_bucket_f(a.nq);
+    b.publish   = {};
+    if (a.part != 2) { verify_small_f(a, stream); }
+    if (a.part == 1) { return; }
+  }
   // room for k scored rows plus a chunk of k / 2 more (at least the final sort's power of two):
   // less LDS per block than 4 k, so more blocks share a CU
   int cap = (3 * a.k / 2 + 255) / 256 * 256;
@@ -1995,9 +2203,9 @@ void verify_topk_f(const verify_f_args& a, hipStream_t stream)
   const auto go = [&](auto lanes) {
     constexpr int N = decltype(lanes)::value;
     if (big) {
-      launch_dyn<1024>(verify_topk_f_kernel<N, 1024>, grid, bytes, stream, a, cap);
+      launch_dyn<1024>(verify_topk_f_kernel<N, 1024>, grid, bytes, stream, b, cap);
     } else {
-      launch_dyn<kThreads>(verify_topk_f_kernel<N, kThreads>, grid, bytes, stream, a, cap);
+      launch_dyn<kThreads>(verify_topk_f_kernel<N, kThreads>, grid, bytes, stream, b, cap);
     }
   };
   switch (L) {

@@ -86,6 +86,22 @@ def test_scoring_slots(gpu, dtype, metric):
         check(Xt.float().numpy(), Qt.float().numpy(), 37, metric, D.cpu().numpy(), I.cpu().numpy())
 
 
+@pytest.mark.parametrize("d", [64, 200, 300])  # 16, 32 and 64 lanes per scored row
+@pytest.mark.parametrize("nq", [3, 256, 257])  # 8 and 4 waves per query
+@pytest.mark.parametrize("metric", ["l2", "cosine"])
+def test_small_rerank(gpu, metric, nq, d):
+    """The small re-rank next to the block one, k up to 64: repeated rows leave some queries more
+    survivors than it holds (2,048 or 1,024 values), equal screen values around the k-th, and more
+    rows to score than one round takes; k = 65 takes the block re-rank alone."""
+    X, Q = correlated(12_001, d, nq, seed=d + nq)
+    X[:4_000] = X[4_000:8_000]
+    X[9_000:10_500] = Q[0] + np.float32(1e-4) * X[9_000:10_500]  # 1,500 rows next to one query
+    X[10_500:10_800] = Q[1]
+    for k in (1, 10, 63, 64, 65):
+        D, I, _ = run(X, Q, k, metric)
+        check(X, Q, k, metric, D, I)
+
+
 def test_inner_product_unequal_norms(gpu):
     X, Q = correlated(20_000, 64, 500, scale_norms=True)
     D, I, _ = run(X, Q, 10, "ip")
