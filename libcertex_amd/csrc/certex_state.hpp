@@ -121,6 +121,7 @@ enum ws_slot : int {
   ws_spill,       // screen spill pool: packed query and row of each entry (+ value, fp16 rows)
   ws_qpaired,     // the batch's fp16 query rows in the paired layout (the tiled screen)
   ws_qlabels,     // query labels given in host memory, copied for the label filter
+  ws_terms,       // row terms under a bitset filter: the stored rows', then the anchors'
   ws_n_slots
 };
 

@@ -204,6 +204,8 @@ struct screen_args {
   int chunk_steps;       // steps of kStepRows rows per workgroup: 4 waves x a whole number of
                          // anchor groups
   filter_args filter;
+  // row terms of the anchor copy in place of the index's (a bitset's, mask_terms); null: the index's
+  const void* anchor_rowc = nullptr;
   // screen: candidate buckets
   uint32_t* cand_count = nullptr;  // [nq_pad]
   uint32_t* cand_rows  = nullptr;  // [nq_pad, cap]
@@ -281,6 +283,15 @@ __host__ __device__ inline int64_t screen_group_tile0(int64_t tiles, int64_t nq,
 
 /** Steps of kStepRows rows that cover n_scan rows. */
 __host__ __device__ inline int64_t screen_steps(int64_t n_scan) { return (n_scan + kStepRows - 1) / kStepRows; }
+
+/**
+ * Row terms under a bitset filter (f.kind 1): terms[r] = rowc[r] for the stored rows r < n whose id
+ * passes, else the term of a removed row (int32 or float); and anchor_terms[j] likewise of
+ * anchor_rowc[j], j < n_anchor, the anchors of the ids j * stride. A pass over these terms keeps no
+ * excluded row, without a filter test of its own.
+ */
+void mask_terms(const void* rowc, int64_t n, const void* anchor_rowc, int64_t n_anchor, int64_t stride,
+                bool f16, const filter_args& f, void* terms, void* anchor_terms, hipStream_t stream);
 
 /** Int8 MFMA pass that keeps (query, row) pairs whose screen value reaches the query threshold
  *  (rows of more than 256 bytes: screen_i8_tile). */

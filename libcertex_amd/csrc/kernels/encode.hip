@@ -8,6 +8,7 @@
 #include "../kernels.hpp"
 #include "lanes.hpp"
 
+#include <cmath>
 #include <type_traits>
 
 namespace certex_amd {
@@ -110,6 +111,24 @@ __global__ void fill_kernel(T* p, int64_t n, T v)
   for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
        i += int64_t(gridDim.x) * blockDim.x) {
     p[i] = v;
+  }
+}
+
+template <typename V>
+__global__ __launch_bounds__(256) void mask_terms_kernel(const V* rowc, int64_t n, const V* anchor_rowc,
+                                                         int64_t n_anchor, int64_t stride, filter_args f,
+                                                         V dead, V* terms, V* anchor_terms)
+{
+  const int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  if (t >= n + n_anchor) { return; }
+  const bool anchor = t >= n;
+  const uint32_t id = anchor ? uint32_t((t - n) * stride) : listed_id(f, uint32_t(t));
+  const V term      = anchor ? anchor_rowc[t - n] : rowc[t];
+  const V v         = (f.words[id >> 5] >> (id & 31)) & 1u ? term : dead;
+  if (anchor) {
+    anchor_terms[t - n] = v;
+  } else {
+    terms[t] = v;
   }
 }
 
@@ -823,6 +842,23 @@ void fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t stream)
   if (n == 0) { return; }
   const unsigned b = blocks_for(n) < 4096 ? blocks_for(n) : 4096;
   fill_kernel<int32_t><<<b, 256, 0, stream>>>(p, n, v);
+}
+
+void mask_terms(const void* rowc, int64_t n, const void* anchor_rowc, int64_t n_anchor, int64_t stride,
+                bool f16, const filter_args& f, void* terms, void* anchor_terms, hipStream_t stream)
+{
+  if (n + n_anchor == 0) { return; }
+  const auto go = [&](auto dead) {
+    using V = decltype(dead);
+    mask_terms_kernel<V><<<blocks_for(n + n_anchor), 256, 0, stream>>>(
+      static_cast<const V*>(rowc), n, static_cast<const V*>(anchor_rowc), n_anchor, stride, f, dead,
+      static_cast<V*>(terms), static_cast<V*>(anchor_terms));
+  };
+  if (f16) {
+    go(-float(INFINITY));
+  } else {
+    go(kDeadRow);
+  }
 }
 
 void pack_bits(const uint8_t* mask, int64_t n, uint32_t* words, hipStream_t stream)

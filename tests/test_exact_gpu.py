@@ -256,3 +256,50 @@ def test_integer_rerank_waves(gpu, d, nq):
         s, i = oracle.knn(X, Q, k, metric)
         np.testing.assert_array_equal(I.cpu().numpy(), i)
         np.testing.assert_array_equal(D.cpu().numpy(), oracle.distances(s, i, metric))
+
+
+@pytest.mark.parametrize("keep", [0.0, 0.004, 0.3, 1.0])
+@pytest.mark.parametrize("dtype, d, lists", [
+    (np.uint8, 128, 0), (np.uint8, 128, 40), (np.int8, 200, 0), (np.uint8, 300, 0),
+    (np.float32, 100, 0), (np.float32, 64, 40), (np.float32, 200, 0),
+])
+def test_bitset_by_row_terms(gpu, dtype, d, lists, keep):
+    """A bitset masks the row terms of the screen and of the anchors (row counts off the word and
+    the 4-term load, removed rows, more neighbours asked for than pass, lists with and without a
+    probe): the oracle's answer, and that of the filtered kernels, which a search without
+    allocation takes."""
+    import ctypes
+
+    from libcertex_amd import _capi as C
+    from libcertex_amd.index import _pack
+
+    n, k = 30_003, 9
+    if dtype == np.float32:
+        rng = np.random.default_rng(d)
+        X, Q = rng.standard_normal((n, d)).astype(dtype), rng.standard_normal((70, d)).astype(dtype)
+    else:
+        X, Q = data.uniform_int(n, d, seed=d, dtype=dtype), data.uniform_int(70, d, seed=d + 1, dtype=dtype)
+    mask = np.random.default_rng(int(1000 * keep)).random(n) < keep
+    gone = np.arange(0, n, 17)
+    idx = certex.Index(d, n_lists=lists)
+    idx.add(torch.from_numpy(X).cuda())
+    idx.remove(torch.from_numpy(gone))
+    live = mask.copy()
+    live[gone] = False
+    rows = np.nonzero(live)[0]
+    want = np.full((70, k), -1, np.int64)
+    if rows.size:
+        kk = min(k, rows.size)
+        want[:, :kk] = rows[oracle.knn(X[rows], Q, kk, "l2")[1]]
+    Qg, mg = torch.from_numpy(Q).cuda(), torch.from_numpy(mask).cuda()
+    for probe in (2, 0) if lists else (2,):
+        D, I = idx.search(Qg, k=k, filter=mg, probe_lists=probe)
+        np.testing.assert_array_equal(I.cpu().numpy(), want)
+        I2, D2 = torch.empty_like(I), torch.empty_like(D)
+        sp = C.SearchParams(128, 2048, probe)
+        qb, ib, db = C.Borrowed(Qg), C.Borrowed(I2), C.Borrowed(D2)
+        wb = C.Borrowed(_pack(mg), dtype_override=(C.kDLUInt, 32))
+        C.check(C.lib().cuvsCertexSearchNoAlloc(C.resources(), ctypes.byref(sp), idx.core.h, qb.ptr, ib.ptr, db.ptr,
+                                                C.Filter(ctypes.addressof(wb.m), C.BITSET)))
+        torch.cuda.synchronize()
+        assert torch.equal(I, I2) and torch.equal(D, D2)
