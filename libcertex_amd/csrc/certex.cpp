@@ -368,7 +368,21 @@ struct route_plan {
 
 constexpr int kScreenChunk = 128;      // most steps per screen workgroup
 constexpr int kRoutedChunk = 32;       // most steps per workgroup of a routed screen
-constexpr int64_t kMinTiles = 2048;    // workgroups a launch should have (8 per CU)
+constexpr int64_t kMinTiles = 2048;    // workgroups an anchor pass should have (8 per CU)
+
+/**
+ * Workgroups a narrow screen should have. A workgroup first copies its queries into LDS (up to 128
+ * KB) and ends with a flush; with fewer, longer workgroups these weigh less, until CUs run idle. 384
+ * (three for every two CUs), measured against 2,048: 1,000 queries x 1M rows of 128 bytes 270 -> 235
+ * us a search, 128 queries 102 -> 83, 1,000 x 500,000 rows of 256 bytes 389 -> 280, 2,048 x 1M rows of
+ * 64 halves 696 -> 610. fp16 rows of 256 bytes keep far more survivors, in 128-query workgroups of 32
+ * KB, and need more of them to overlap epilogues with MFMAs: 1,536 (1,000 queries x 100,000 rows 115
+ * -> 112 us, 128 x 1M 117 -> 113; with 384: 121 and 104, but 2,048 x 100,000 189 against 167).
+ */
+auto screen_min_tiles(index_state const& st) -> int64_t
+{
+  return !is_int(st.type) && st.row_bytes == 256 ? 1536 : 384;
+}
 
 auto anchor_chunk_steps(bool wide, int64_t g) -> int
 {
@@ -377,26 +391,26 @@ auto anchor_chunk_steps(bool wide, int64_t g) -> int
 
 /**
  * Steps per workgroup: the largest of cap, cap / 2, ... (multiples of unit) that still gives the
- * launch kMinTiles workgroups; small batches and short scans split into smaller chunks so that
+ * launch min_tiles workgroups; small batches and short scans split into smaller chunks so that
  * every CU gets work.
  */
 template <typename F>
-auto pick_chunk(int64_t unit, int64_t cap, F&& tiles) -> int
+auto pick_chunk(int64_t unit, int64_t cap, int64_t min_tiles, F&& tiles) -> int
 {
   int64_t c = std::max(unit, cap / unit * unit);
-  while (c > unit && tiles(c) < kMinTiles) { c = std::max(unit, c / 2 / unit * unit); }
+  while (c > unit && tiles(c) < min_tiles) { c = std::max(unit, c / 2 / unit * unit); }
   return int(c);
 }
 
 /** Chunk of a plain (unrouted) pass over n_scan scan indices. */
 auto plain_chunk(index_state const& st, int64_t nq, int64_t nq_pad, int64_t n_scan, int64_t unit,
-                 int64_t cap) -> int
+                 int64_t cap, int64_t min_tiles) -> int
 {
   const bool f16      = !is_int(st.type);
   const int64_t qb    = certex_amd::screen_query_block(f16, st.row_bytes, nq_pad);
   const int64_t n_qb  = (nq + qb - 1) / qb;
   const int64_t steps = certex_amd::screen_steps(n_scan);
-  return pick_chunk(unit, cap, [&](int64_t c) { return n_qb * ((steps + c - 1) / c); });
+  return pick_chunk(unit, cap, min_tiles, [&](int64_t c) { return n_qb * ((steps + c - 1) / c); });
 }
 
 auto waves_of(index_state const& st) -> int64_t
@@ -429,7 +443,7 @@ void anchor_pass(index_state const& st, certex_amd::screen_args aa, anchor_plan 
     aa.row_base    = ap.first;
     aa.id_scale    = ap.stride;
     aa.n_scan      = ap.n_anchor;
-    aa.chunk_steps = plain_chunk(st, aa.nq, aa.nq_pad, aa.n_scan, unit, cap);
+    aa.chunk_steps = plain_chunk(st, aa.nq, aa.nq_pad, aa.n_scan, unit, cap, kMinTiles);
     launch(aa, stream);
     return;
   }
@@ -462,7 +476,7 @@ void anchor_pass(index_state const& st, certex_amd::screen_args aa, anchor_plan 
     t.row_base                = st.label_part.n;
     t.n_scan                  = (tail + ap.stride - 1) / ap.stride;
     t.grp_base                = route->part_groups;
-    t.chunk_steps             = plain_chunk(st, t.nq, t.nq_pad, t.n_scan, unit, cap);
+    t.chunk_steps             = plain_chunk(st, t.nq, t.nq_pad, t.n_scan, unit, cap, kMinTiles);
     launch(t, stream);
   }
 }
@@ -476,7 +490,8 @@ auto screen_pass(index_state const& st, route_plan const* route, F&& launch)
   return [&st, route, launch, tiled](certex_amd::screen_args& sa, hipStream_t stream) {
     auto chunk = [&](certex_amd::screen_args const& x) {
       return tiled ? certex_amd::tile_chunk_steps()
-                   : plain_chunk(st, x.nq, x.nq_pad, x.n_scan, waves_of(st), kScreenChunk);
+                   : plain_chunk(st, x.nq, x.nq_pad, x.n_scan, waves_of(st), kScreenChunk,
+                               screen_min_tiles(st));
     };
     if (route == nullptr) {
       sa.chunk_steps = chunk(sa);
@@ -727,7 +742,7 @@ bool plan_probe(cuvs::resources const& res, index_state const& st, const void* q
   const int qb        = certex_amd::screen_query_block(f16, st.row_bytes, pp.nq_pad);
   const int64_t waves = waves_of(st);
   const int64_t gs    = std::max<int64_t>(1, g);
-  pp.chunk = pick_chunk(waves * gs, anchor_chunk_steps(wide, gs), [&](int64_t c) {
+  pp.chunk = pick_chunk(waves * gs, anchor_chunk_steps(wide, gs), kMinTiles, [&](int64_t c) {
     int64_t t = 0;
     for (auto const& e : pp.groups) { t += certex_amd::screen_group_tiles(e.nq, e.nx, qb, int(c)); }
     return t;
@@ -1414,7 +1429,8 @@ void routed_batch(cuvs::resources const& res, index_state const& st, batch_fn ba
   route.anchor_chunk  = route.anchor_tiled
                           ? certex_amd::tile_chunk_steps()
                           : pick_chunk(waves * route.ap.group_steps,
-                                       anchor_chunk_steps(wide, route.ap.group_steps), [&](int64_t c) {
+                                       anchor_chunk_steps(wide, route.ap.group_steps), kMinTiles,
+                                       [&](int64_t c) {
                                          int64_t t = 0;
                                          for (auto const& e : ga) {
                                            t += certex_amd::screen_group_tiles(e.nq, anchors_of(e), qb, int(c));
@@ -1423,7 +1439,7 @@ void routed_batch(cuvs::resources const& res, index_state const& st, batch_fn ba
                                        });
   const int qbs    = tiled ? certex_amd::tile_block_queries() : qb;
   route.screen_chunk =
-    tiled ? certex_amd::tile_chunk_steps() : pick_chunk(waves, kRoutedChunk, [&](int64_t c) {
+    tiled ? certex_amd::tile_chunk_steps() : pick_chunk(waves, kRoutedChunk, screen_min_tiles(st), [&](int64_t c) {
       int64_t t = 0;
       for (auto const& e : gs) { t += certex_amd::screen_group_tiles(e.nq, e.nx, qb, int(c)); }
       return t;
