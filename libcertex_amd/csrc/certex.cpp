@@ -443,7 +443,11 @@ void anchor_pass(index_state const& st, certex_amd::screen_args aa, anchor_plan 
     aa.row_base    = ap.first;
     aa.id_scale    = ap.stride;
     aa.n_scan      = ap.n_anchor;
-    aa.chunk_steps = plain_chunk(st, aa.nq, aa.nq_pad, aa.n_scan, unit, cap, kMinTiles);
+    // wide rows without a filter: tiles of the tiled screen, which record groups of 4 anchors or of
+    // one step (longer groups and filters: the K-loop pass)
+    aa.tiled = uses_tile_screen(st) && (ap.fine || ap.group_steps == 1) && aa.filter.kind == 0;
+    aa.chunk_steps = aa.tiled ? certex_amd::tile_chunk_steps()
+                              : plain_chunk(st, aa.nq, aa.nq_pad, aa.n_scan, unit, cap, kMinTiles);
     launch(aa, stream);
     return;
   }

@@ -197,8 +197,8 @@ struct screen_args {
   const int8_t* qpaired = nullptr;
   bool rows_paired      = false;
   // routed anchor pass over a paired partition: the anchors of a group are row pairs
-  // (paired_anchor_count), row_stride the pairs' half spacing; with tiled, the pass runs as tiles
-  // of the tiled screen (fine groups, paired queries, chunk_steps = tile_chunk_steps())
+  // (paired_anchor_count), row_stride the pairs' half spacing. tiled: the anchor pass runs as tiles
+  // of the tiled screen (paired queries, chunk_steps = tile_chunk_steps(); anchors_f16_tile)
   bool anchor_pairs = false;
   bool tiled        = false;
   int chunk_steps;       // steps of kStepRows rows per workgroup: 4 waves x a whole number of
@@ -317,10 +317,10 @@ void anchors_i8_wide(const screen_args& a, hipStream_t stream);
  */
 void screen_f16_tile(const screen_args& a, hipStream_t stream);
 /**
- * The routed fp16 anchor pass over a paired partition with anchor pairs and fine groups, as tiles
- * of the same kernel (256 anchors x tile_block_queries() queries): each lane writes the best
- * screen value of its 4 consecutive anchors of every row tile and query tile to the group table.
- * anchors_f16_wide runs it for a pass with `tiled`.
+ * The fp16 anchor pass as tiles of the same kernel (256 anchors per workgroup), without a filter:
+ * the routed pass over a paired partition with anchor pairs and fine groups, or the pass over the
+ * anchor copy with fine groups or groups of one step. anchors_f16_wide runs it for a pass with
+ * `tiled`.
  */
 void anchors_f16_tile(const screen_args& a, hipStream_t stream);
 /** The tiled screen and tiled anchor pass over int8 rows of more than 256 bytes (exact int32

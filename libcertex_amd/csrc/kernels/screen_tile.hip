@@ -41,11 +41,16 @@
 // Workgroup b runs on XCD b % 8; the query blocks of one row tile run on one XCD (work_of), so a
 // row tile is fetched from HBM about once.
 //
-// The same kernel (ANCH) runs the routed anchor pass over a paired partition with fine groups: a
-// tile's 256 rows are anchors taken in row pairs (scan index i is stored row base + (i / 2) 2 s +
-// i % 2), and instead of survivors each lane writes the maximum of its 4 accumulators of every row
-// tile and query tile, the screen value of one fine group of 4 anchors, to the group table.
+// The same kernel (ANCH) runs anchor passes: the routed pass over a paired partition with fine groups
+// (a tile's 256 rows are anchors taken in row pairs: scan index i is stored row base + (i / 2) 2 s +
+// i % 2), and the pass over the anchor copy (consecutive rows) with fine groups or groups of one
+// step. Instead of survivors each lane writes the maximum of its 4 accumulators of every row tile and
+// query tile, the screen value of one fine group of 4 anchors, to the group table; a step's group is
+// the maximum over the 4 lanes of a query and 4 row tiles. A tile of 256 anchors has four times the
+// workgroups of the K-loop pass, whose 8 waves take a step each: 3,750 anchors of 384 halves x 2,048
+// queries 19.6 -> 14.7 us, 62,500 of 768 x 16 queries 35 -> 21.7 us.
 
+#include "lanes.hpp"
 #include "screen_common.hpp"
 
 #include <algorithm>
@@ -103,8 +108,11 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p)
 /** Staging LDS of a workgroup of TQ queries: three stage buffers of (256 + TQ) rows x 64 bytes. */
 constexpr int tile_lds(int tq) { return kBufs * (kTileRows + tq) * kStageB; }
 
-/** All LDS of a workgroup: the staging, then the TQ query thresholds and the 256 row terms. */
-constexpr int tile_lds_total(int tq) { return tile_lds(tq) + 4 * tq + 4 * kTileRows; }
+/** Words of the query thresholds: a copy writes 64 of them. */
+constexpr int tile_theta(int tq) { return tq < 64 ? 64 : tq; }
+
+/** All LDS of a workgroup: the staging, then the query thresholds and the 256 row terms. */
+constexpr int tile_lds_total(int tq) { return tile_lds(tq) + 4 * tile_theta(tq) + 4 * kTileRows; }
 
 /** Survivor list entries that fit the staging LDS: 12 bytes each plus the flush's rank word,
  *  after the flush's 2 TQ counters and the waves' 8 KB of parked screen values. */
@@ -145,10 +153,13 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void screen_tile_kernel(screen_
   constexpr int TQ  = S::TQ;
   static_assert(TQ <= (1 << (32 - kSpillRowBits)), "a spill entry holds the query within the tile");
   constexpr int CA  = kTileRows / 16 / kTileWaves;  // row copies per wave and stage
-  constexpr int CB  = TQ / 16 / kTileWaves;         // query copies per wave and stage
+  constexpr int CB  = TQ < 64 ? 1 : TQ / 16 / kTileWaves;  // query copies per wave and stage
   constexpr int NC  = CA + CB;                      // copies per wave and stage
-  static_assert(CA * 16 * kTileWaves == kTileRows && CB * 16 * kTileWaves == TQ,
+  static_assert(CA * 16 * kTileWaves == kTileRows && (TQ < 64 || CB * 16 * kTileWaves == TQ),
                 "every wave issues the same copies (the stage waits count them)");
+  // 16 query rows per copy; tiles of fewer than 64 queries have fewer copies than waves, and waves
+  // wave and wave + TQ / 16 write the same bytes
+  const auto qcopy = [](int w, int j) { return (w * CB + j) % (TQ / 16); };
   constexpr int CPT = (NC + RT - 1) / RT;           // copies per row tile
   constexpr int BUF = (kTileRows + TQ) * kStageB;   // one stage buffer: rows, then queries
   constexpr int CAP = tile_hit_cap(TQ);
@@ -179,8 +190,9 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void screen_tile_kernel(screen_
   // every 2 row_stride rows from the tile's first pair (scan index i = stored row
   // base + (i / 2) 2 row_stride + i % 2; scan0 is even)
   const int64_t s2     = ANCH ? 2 * int64_t(a.row_stride) : 2;
-  const int64_t row_t0 = ANCH ? w.base + (scan0 >> 1) * s2 : w.base + scan0;
-  auto tile_rel        = [&](int64_t r) { return ANCH ? (r >> 1) * s2 + (r & 1) : r; };
+  const int64_t row_t0 = ANCH && a.anchor_pairs ? w.base + (scan0 >> 1) * s2 : w.base + scan0;
+  const bool pairs     = ANCH && a.anchor_pairs;
+  auto tile_rel        = [&](int64_t r) { return pairs ? (r >> 1) * s2 + (r & 1) : r; };
 
   if (tid == 0) { n_hits = 0; }
 
@@ -189,7 +201,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void screen_tile_kernel(screen_
   // first live one reads its neighbour, in the same allocation)
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   val_t* th_lds    = reinterpret_cast<val_t*>(lds + tile_lds(TQ));
-  val_t* rc_lds    = th_lds + TQ;
+  val_t* rc_lds    = th_lds + tile_theta(TQ);
   {
     const int64_t r = wave_u * 64 + lane;
     lds_copy<4>(static_cast<const val_t*>(a.rowc) + row_t0 + tile_rel(r < n_rows ? r : n_rows - 1),
@@ -222,7 +234,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void screen_tile_kernel(screen_
   }
 #pragma unroll
   for (int j = 0; j < CB; ++j) {
-    int64_t q = (wave * CB + j) * 16 + crow;
+    int64_t q = qcopy(wave, j) * 16 + crow;
     q         = q < n_q ? q : n_q - 1;
     qoff[j]   = uint32_t((q & ~int64_t(1)) * RB + (q & 1) * 64);
   }
@@ -234,7 +246,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void screen_tile_kernel(screen_
       lds_copy<16>(rbase + s * rstep + roff[j], lds_addr(buf + ((wave_u * CA + j) * 16) * kStageB));
     } else {
       lds_copy<16>(qbase + s * 128 + qoff[j - CA],
-                   lds_addr(buf + (kTileRows + (wave_u * CB + j - CA) * 16) * kStageB));
+                   lds_addr(buf + (kTileRows + qcopy(wave_u, j - CA) * 16) * kStageB));
     }
   };
   auto issue = [&](int s) {
@@ -314,6 +326,30 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void screen_tile_kernel(screen_
   stage(s, std::true_type{}, std::false_type{});
   stage(s + 1, std::false_type{}, std::false_type{});
 
+  if (ANCH && !a.fine) {
+    // groups of one step: 64 of the wave's rows, 16 accumulators of each of a query's 4 lanes
+    val_t* gmax      = static_cast<val_t*>(a.gmax);
+    const int64_t g0 = scan0 / kStepRows + wr * RT / 4;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const int qloc = wq * 16 * QT + qt * 16 + frow;
+#pragma unroll
+      for (int h = 0; h < RT / 4; ++h) {
+        val_t m = R::lowest();
+#pragma unroll
+        for (int bt = 4 * h; bt < 4 * h + 4; ++bt) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) { m = R::vmax(m, acc[bt][qt][r]); }
+        }
+        m = lanes::fold16(m, [](val_t x, val_t y) { return R::vmax(x, y); });
+        m = lanes::fold32(m, [](val_t x, val_t y) { return R::vmax(x, y); });
+        if (fch == 0 && qloc >= q_lo && qloc < n_q && (g0 + h) * kStepRows < w.n_scan) {
+          gmax[table_entry(a, w.q0 + qloc, g0 + h)] = m;
+        }
+      }
+    }
+    return;
+  }
   if constexpr (ANCH) {
     // fine groups: the 4 consecutive anchors of a lane's row tile are one group of the table.
     // Lane (query frow, fch) holds group 4 bt + fch of the wave's 16 RT / 4 consecutive groups
@@ -468,14 +504,16 @@ void launch_shape(const screen_args& a, hipStream_t stream)
     blocks                 = n_steps == 0 ? 0 : 8 * n_qb * ((n_chunks + 7) / 8);
   }
   if (blocks == 0) { return; }
-  const bool shape = ANCH ? a.groups != nullptr && a.anchor_pairs && a.rows_paired && a.fine &&
-                             a.filter.kind == 0 && a.gmax != nullptr
+  // anchor passes: over the anchor pairs of a routed pass, or the anchor copy (consecutive rows)
+  const bool from = a.groups != nullptr ? a.anchor_pairs && a.rows_paired
+                                        : !a.anchor_pairs && !a.rows_paired && a.row_stride == 1;
+  const bool shape = ANCH ? from && (a.fine || a.group_steps == 1) && a.filter.kind == 0 && a.gmax != nullptr
                            : a.row_stride == 1 && !(a.rows_paired && a.groups == nullptr);
   if (!shape || a.chunk_steps != kTileSteps || a.row_bytes % 128 != 0 || a.qpaired == nullptr) {
     throw std::logic_error(
       "certex: the tiled screen needs chunks of 4 steps over rows of 128-byte multiples, paired "
-      "queries, and paired rows only in routed passes (anchor passes: routed over anchor pairs, "
-      "fine groups, no filter)");
+      "queries, and paired rows only in routed passes (anchor passes: over anchor pairs of a routed "
+      "pass or the anchor copy, groups of 4 anchors or of one step, no filter)");
   }
   screen_args b = a;
   b.spill_cap   = !ANCH && a.spill != nullptr ? a.spill_pool / blocks : 0;
@@ -489,6 +527,24 @@ void launch_shape(const screen_args& a, hipStream_t stream)
   k<<<dim3(unsigned(blocks)), 64 * kTileWaves, lds, stream>>>(b);
 }
 
+/**
+ * The tile of a pass. Routed passes: 256 rows x 128 queries (their group tables count that). Plain
+ * passes of at most 64 (16) queries: 64 (16) queries, each wave on 64 rows of the tile: the rows
+ * still stream at the memory's rate, but the padding queries' MFMAs and LDS reads, which bounded a
+ * 16-query pass, go: 1M rows of 768 halves (1.5 GB) x 16 queries 284 -> 274 us, 5.7 TB/s.
+ */
+template <typename R, bool FILT, bool ANCH>
+void launch_tile(const screen_args& a, hipStream_t stream)
+{
+  if (a.groups == nullptr && a.nq <= 16) {
+    launch_shape<R, 4, 1, FILT, ANCH>(a, stream);
+  } else if (a.groups == nullptr && a.nq <= 64) {
+    launch_shape<R, 4, 4, FILT, ANCH>(a, stream);
+  } else {
+    launch_shape<R, 8, 4, FILT, ANCH>(a, stream);
+  }
+}
+
 }  // namespace
 
 int tile_chunk_steps() { return kTileSteps; }
@@ -498,29 +554,29 @@ int tile_block_queries() { return tile_shape<8, 4>::TQ; }
 void screen_f16_tile(const screen_args& a, hipStream_t stream)
 {
   if (a.filter.kind != 0) {
-    launch_shape<f16_rows, 8, 4, true, false>(a, stream);
+    launch_tile<f16_rows, true, false>(a, stream);
   } else {
-    launch_shape<f16_rows, 8, 4, false, false>(a, stream);
+    launch_tile<f16_rows, false, false>(a, stream);
   }
 }
 
 void anchors_f16_tile(const screen_args& a, hipStream_t stream)
 {
-  launch_shape<f16_rows, 8, 4, false, true>(a, stream);
+  launch_tile<f16_rows, false, true>(a, stream);
 }
 
 void screen_i8_tile(const screen_args& a, hipStream_t stream)
 {
   if (a.filter.kind != 0) {
-    launch_shape<int8_rows, 8, 4, true, false>(a, stream);
+    launch_tile<int8_rows, true, false>(a, stream);
   } else {
-    launch_shape<int8_rows, 8, 4, false, false>(a, stream);
+    launch_tile<int8_rows, false, false>(a, stream);
   }
 }
 
 void anchors_i8_tile(const screen_args& a, hipStream_t stream)
 {
-  launch_shape<int8_rows, 8, 4, false, true>(a, stream);
+  launch_tile<int8_rows, false, true>(a, stream);
 }
 
 }  // namespace certex_amd

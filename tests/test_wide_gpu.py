@@ -177,3 +177,26 @@ def test_widths_beyond_the_limit_refused(gpu):
         certex.Index(4097).add(np.zeros((10, 4097), np.uint8))
     with pytest.raises(ValueError, match="4096"):
         certex.Index(4100).add(np.zeros((10, 4100), np.float32))
+
+
+@pytest.mark.parametrize("nq", [1, 16, 17, 64, 65, 130])  # tiles of 16, 64 and 128 queries
+@pytest.mark.parametrize("dtype, d", [(np.float32, 200), (np.uint8, 300)])
+def test_wide_tiles_of_few_queries(gpu, dtype, d, nq):
+    """The tiled screen and the tiled anchor pass of plain searches in their three query widths, with
+    anchor groups of one step (k = 1), of 4 anchors (k = 20) and, filtered, without tiles."""
+    n = 70_001
+    if dtype == np.uint8:
+        X, Q = mixture(n, d, seed=nq), mixture(nq, d, seed=nq + 1)
+    else:
+        rng = np.random.default_rng(nq)
+        X, Q = rng.standard_normal((n, d)).astype(dtype), rng.standard_normal((nq, d)).astype(dtype)
+    X[:300] = X[300:600]
+    Q[0] = X[400]  # ties and many equal screen values
+    idx = certex.Index(d)
+    idx.add(torch.from_numpy(X).cuda())
+    mask = np.random.default_rng(5).random((nq, n)) < 0.5
+    for k in (1, 20):
+        D, I = idx.search(torch.from_numpy(Q).cuda(), k=k)
+        check(X, Q, k, "l2", D, I)
+    D, I = idx.search(torch.from_numpy(Q).cuda(), k=5, filter=torch.from_numpy(mask).cuda())
+    check(X, Q, 5, "l2", D, I, bitmap=words(mask))
