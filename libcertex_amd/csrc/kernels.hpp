@@ -486,8 +486,8 @@ void threshold_f16(const threshold_f_args& a, hipStream_t stream);
 
 /**
  * Testing only: the certificate's bounds of the exact score of every bucket entry of the live
- * queries, from its screen value v: lb[q, slot] = the lower bound that the ordered verification
- * uses, ub[q, slot] = the upper bound that the threshold uses (both for slot < min(count[q], cap)).
+ * queries, from its screen value v: lb[q, slot] = the lower bound that inverts the
+ * threshold map (the ordered verification tests values against that map), ub[q, slot] = the upper bound that the threshold uses (both for slot < min(count[q], cap)).
  */
 void certificate_bounds(const threshold_f_args& a, const uint32_t* count, const float* vals,
                         int64_t cap, double* lb, double* ub, hipStream_t stream);

@@ -1115,7 +1115,8 @@ __device__ inline float key_value(uint32_t k)
  * pair (cross) plus the fp32 accumulation of its products (accum), from the query's |fp16(W)|,
  * |W - fp16(W)| (qscal) and the index's largest |fp16(Z)|, |Z - fp16(Z)| (maxima).
  */
-__device__ inline double screen_error(const threshold_f_args& a, int64_t q)
+template <typename A>  // threshold_f_args or verify_f_args
+__device__ inline double screen_error(const A& a, int64_t q)
 {
   const double nw = a.qscal[3 * q + 1], ew = a.qscal[3 * q + 2];
   const double nz = a.maxima[0], ez = a.maxima[1];
@@ -1130,7 +1131,8 @@ __device__ inline double screen_error(const threshold_f_args& a, int64_t q)
  * C = screen_error: inner products t(U) = -U / alpha2 - C; l2 t(U) = (|W|^2 - U / alpha2) / 2 - C
  * (cosine: l2 on the unit vectors with U_l2 = 2 + 2 U); both less 1e-10 of their scale.
  */
-__device__ inline float theta_of(double U, const threshold_f_args& a, int64_t q)
+template <typename A>
+__device__ inline float theta_of(double U, const A& a, int64_t q)
 {
   const double aq = a.qscal[3 * q];
   double th, scale;
@@ -1231,8 +1233,8 @@ __global__ __launch_bounds__(kThreads) void threshold_f16_cert_kernel(threshold_
 
 
 /**
- * A lower bound of the exact score of a pair whose fp16 screen value is v: the inverse of the
- * threshold map theta_of (a pair with score s has v >= t(s), where t(U) is the
+ * Testing (certificate_bounds): a lower bound of the exact score of a pair whose fp16 screen value is
+ * v, the inverse of the threshold map theta_of (a pair with score s has v >= t(s), where t(U) is the
  * threshold before rounding), with 20 times its relative slack and a margin for the fp64 rounding
  * of this expression. C = the query's cross and accumulation terms; aq = |W|^2 (lower bound).
  */
@@ -1666,9 +1668,9 @@ struct threshold_f_regs_launch {
  * Exact re-rank of one query's survivors, one block per query. With screen values (fp16 rows),
  * the verification is ordered (the reference's verify_rounds, detail/verify.cuh:371-487): first
  * the k survivors with the largest screen values are scored, which bounds the k-th neighbour's
- * score by U; then only the survivors whose screen lower bound does not exceed U are scored
- * (U tightens as better rows arrive). Scores use one wave per row; the best k by (score, row)
- * stay in LDS. With 64-lane slots (d above 256) eight waves per SIMD, as many blocks as the LDS of a
+ * score by U; then only the survivors whose screen value reaches theta_of(U), the certified least
+ * value of a pair within U, are scored (U tightens as better rows arrive; one compare per survivor,
+ * where a bound of each one's score took 30 fp64 operations). The best k by (score, row) stay in LDS. With 64-lane slots (d above 256) eight waves per SIMD, as many blocks as the LDS of a
  * CU holds at config 3 (18 spilled registers; against six waves per SIMD, verify 0.82 -> 0.79 ms).
  */
 template <int L, int NT>
@@ -1738,7 +1740,7 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
   // phase A: the survivors whose screen value is at least the k-th largest (descending keys)
   bool ordered = vals != nullptr && n_cand > k;
   uint32_t tk  = 0;
-  double U = INFINITY, aq = 0, C = 0;
+  float least  = -INFINITY;  // ordered: the screen value that a row of the k best cannot be below
   if (REGS && ordered && n_cand <= int64_t(NT) * RV) {
     // the survivors' screen values read once into registers (RV per thread; 0xffffffff past the
     // bucket sorts last), selected there, and the k best collected from the same registers
@@ -1749,14 +1751,29 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
       kk[i]           = e < n_cand ? ~fkey(vals[e]) : 0xffffffffu;
     }
     tk = radix_select_regs<NT, RV>(kk, k, hist, wave_tot, red, &sel_digit, &sel_rank);
-    if (tid == 0) { fill = 0; }
-    __syncthreads();
+    // the taken ones' rows, all loads in flight (a load behind each test waited for one after the
+    // other), each thread's at the places that one scan of the counts gives it
+    uint32_t rr[RV];
+    int taken = 0;
 #pragma unroll
     for (int i = 0; i < RV; ++i) {
       const int64_t e = int64_t(i) * NT + tid;
-      const bool take = e < n_cand && kk[i] <= tk;
-      const int slot  = wave_append(take, &fill);
-      if (take && slot < cap) { rid[slot] = to_id(cand[e]); }
+      rr[i]           = cand[e < n_cand ? e : n_cand - 1];
+      taken += e < n_cand && kk[i] <= tk ? 1 : 0;
+    }
+    const int incl = scan_incl_t<NT>(taken, wave_tot);
+    if (tid == NT - 1) { fill = incl; }
+#pragma unroll
+    for (int i = 0; i < RV; ++i) {
+      if (int64_t(i) * NT + tid < n_cand && kk[i] <= tk) { rr[i] = to_id(rr[i]); }
+    }
+    int slot = incl - taken;
+#pragma unroll
+    for (int i = 0; i < RV; ++i) {
+      if (int64_t(i) * NT + tid < n_cand && kk[i] <= tk) {
+        if (slot < cap) { rid[slot] = rr[i]; }
+        ++slot;
+      }
     }
     __syncthreads();
   } else if (ordered) {
@@ -1795,11 +1812,7 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
       score(0, c);
       __syncthreads();
       keep_best();
-      U                = key_score(kth);  // k distinct live rows: bounds the k-th score
-      const double nw  = a.qscal[3 * q + 1], ew = a.qscal[3 * q + 2];
-      const double nz  = a.maxima[0], ez = a.maxima[1];
-      aq               = a.qscal[3 * q];
-      C                = a.gamma * nw * nz + ew * nz + nw * ez + ew * ez;
+      least = theta_of(key_score(kth), a, q);  // k distinct live rows: kth bounds the k-th score
     } else {
       ordered = false;  // more ties at the k-th screen value than the buffer holds: score all
     }
@@ -1809,7 +1822,7 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
   // room. A cut back to the k best (which also tightens U) is a select over the whole buffer: it
   // runs once the rows scored past the k best come to k / 8 (U then moves enough to save
   // scores), or when the free room falls below a quarter of the buffer. The ordered scan keeps
-  // few candidates (those whose lower bound reaches U), so its chunk spans the whole rest of
+  // few candidates (those whose value reaches theta_of(U)), so its chunk spans the whole rest of
   // them: a chunk no longer than the room would cost one round of barriers and loads per room's
   // worth of candidates (1,024 at k = 2,048). When it keeps more than the room holds, that chunk
   // is scanned again at the room's size, and so is every chunk after it.
@@ -1830,7 +1843,7 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
           take[i] = a.rowc[idx] != -INFINITY && keeps(a.filter, q, uint32_t(idx));
         } else if (ordered) {
           const float v = vals[idx];
-          take[i] = ~fkey(v) > tk && screen_lower_bound(v, aq, C, a.alpha2, a.metric) <= U;
+          take[i] = ~fkey(v) > tk && v >= least;
         } else {
           take[i] = true;
         }
@@ -1863,7 +1876,7 @@ void verify_topk_f_kernel(verify_f_args a, int cap)
       if (have > k && c0 < n_cand && (8 * (have - k) >= k || cap - have < cap / 4)) {
         keep_best();
         pending = have;
-        if (ordered) { U = key_score(kth); }
+        if (ordered) { least = theta_of(key_score(kth), a, q); }
       }
     }
   }
@@ -2007,19 +2020,14 @@ void verify_topk_f_small_kernel(verify_f_args a)
   __syncthreads();  // *kth is read before the scores take its place
   if (top > 0) { score(0, top); }
   if (n_cand > k) {
-    // the rest: the survivors whose certified lower bound does not exceed the k-th score so far
-    const double nw = a.qscal[3 * q + 1], ew = a.qscal[3 * q + 2];
-    const double nz = a.maxima[0], ez = a.maxima[1];
-    const double aq = a.qscal[3 * q];
-    const double C  = a.gamma * nw * nz + ew * nz + nw * ez + ew * ez;
-    double U        = key_score(lanes::max<64>(lane < k ? key[lane] : 0ull));
-    int pending     = have;
+    // the rest: the survivors whose screen value a row within the k-th score so far could have
+    float least = theta_of(key_score(lanes::max<64>(lane < k ? key[lane] : 0ull)), a, q);
+    int pending = have;
 #pragma unroll
     for (int i = 0; i < RV; ++i) {
       if (i * NT >= n_cand) { break; }  // uniform over the block
       const uint64_t x = (uint64_t(kk[i]) << 32) | uint32_t(i * NT + tid);
-      bool take        = kk[i] != 0xffffffffu && x > last;
-      if (take) { take = screen_lower_bound(key_value(~kk[i]), aq, C, a.alpha2, a.metric) <= U; }
+      const bool take  = kk[i] != 0xffffffffu && x > last && key_value(~kk[i]) >= least;
       const int slot = wave_append(take, &fill);
       if (take) { rid[have + slot] = to_id(cand[i * NT + tid]); }
       const bool end = (i + 1) * NT >= n_cand;
@@ -2032,7 +2040,8 @@ void verify_topk_f_small_kernel(verify_f_args a)
         score(pending, have);
         pending = have;
         if (!end && have > k) {
-          U = key_score(keep_k_best<NT>(key, rid, have, k, hist, wave_tot, &sel_digit, &sel_rank, &sel_count, &kept));
+          least = theta_of(key_score(keep_k_best<NT>(key, rid, have, k, hist, wave_tot, &sel_digit, &sel_rank,
+                                                     &sel_count, &kept)), a, q);
           have = pending = k;
         }
       }
