@@ -139,6 +139,21 @@ CUVS_EXPORT cuvsError_t cuvsCertexSearchWithLabels(cuvsResources_t res,
                                                    DLManagedTensor* neighbors,
                                                    DLManagedTensor* distances);
 
+/**
+ * cuvsCertexSearchWithLabels whose neighbours are reported through `id_map`, an int64 device vector
+ * of at least one entry per vector added (cuvsCertexIndexGetSize): id_map[id] instead of id. An
+ * addition: a cache that keeps several sequences in one index maps its ids to each one's own as the
+ * results are written, not in a pass over them.
+ */
+CUVS_EXPORT cuvsError_t cuvsCertexSearchWithLabelsMapped(cuvsResources_t res,
+                                                         cuvsCertexSearchParams_t params,
+                                                         cuvsCertexIndex_t index,
+                                                         DLManagedTensor* queries,
+                                                         DLManagedTensor* query_labels,
+                                                         DLManagedTensor* id_map,
+                                                         DLManagedTensor* neighbors,
+                                                         DLManagedTensor* distances);
+
 /** Save the index with its vectors (reference certex.h:213-215). */
 CUVS_EXPORT cuvsError_t cuvsCertexSerialize(cuvsResources_t res,
                                             const char* filename,

@@ -148,6 +148,16 @@ def lib():
                         P(DLManagedTensor),
                         P(DLManagedTensor),
                     ],
+                    "cuvsCertexSearchWithLabelsMapped": [
+                        ctypes.c_size_t,
+                        P(SearchParams),
+                        P(IndexHandle),
+                        P(DLManagedTensor),
+                        P(DLManagedTensor),
+                        P(DLManagedTensor),
+                        P(DLManagedTensor),
+                        P(DLManagedTensor),
+                    ],
                     "cuvsCertexSerialize": [ctypes.c_size_t, ctypes.c_char_p, P(IndexHandle)],
                     "cuvsCertexDeserialize": [ctypes.c_size_t, ctypes.c_char_p, P(IndexHandle)],
                     "cuvsCertexIndexGetRemoved": [P(IndexHandle), P(i64)],

@@ -156,11 +156,11 @@ class KeyCache:
             # read-back from the GPU
             self._labels[key] = (torch.arange(H, dtype=torch.int32) // r).repeat_interleave(m)
         labels = self._labels[key]
-        D, I = self.index.search(
-            Q.reshape(H * m, d), k=k, batch=batch or max(2048, H * m), labels=labels
+        D, I = self.index._search(
+            Q.reshape(H * m, d), k, batch or max(2048, H * m), labels, None, id_map=self.local
         )
         scores = D.reshape(H, m, k)
-        ids = self.local[I].reshape(H, m, k)
+        ids = I.reshape(H, m, k)
         return (scores[:, 0], ids[:, 0]) if single else (scores, ids)
 
 

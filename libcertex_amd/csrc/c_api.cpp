@@ -450,6 +450,19 @@ cuvsError_t cuvsCertexSearchWithLabels(cuvsResources_t res,
                                        DLManagedTensor* neighbors,
                                        DLManagedTensor* distances)
 {
+  return cuvsCertexSearchWithLabelsMapped(res, params, index, queries, query_labels, nullptr, neighbors,
+                                          distances);
+}
+
+cuvsError_t cuvsCertexSearchWithLabelsMapped(cuvsResources_t res,
+                                             cuvsCertexSearchParams_t params,
+                                             cuvsCertexIndex_t index,
+                                             DLManagedTensor* queries,
+                                             DLManagedTensor* query_labels,
+                                             DLManagedTensor* id_map,
+                                             DLManagedTensor* neighbors,
+                                             DLManagedTensor* distances)
+{
   return translate([=] {
     auto& r      = res_of(res);
     const auto p = to_cpp(*params);
@@ -471,7 +484,13 @@ cuvsError_t cuvsCertexSearchWithLabels(cuvsResources_t res,
                         distances->dl_tensor.shape[0] == q.rows &&
                         distances->dl_tensor.shape[1] == k,
                       "output shapes do not match the queries");
-      certex::search<T>(r, p, idx, q, ql, nb, ds, k, is_host(lt));
+      const int64_t* map = nullptr;
+      if (id_map != nullptr) {
+        map = device_data<const int64_t>(id_map, 1, "the id map");
+        certex::expects(id_map->dl_tensor.shape[0] >= idx.size(),
+                        "certex: the id map needs one entry per vector");
+      }
+      certex::search<T>(r, p, idx, q, ql, nb, ds, k, is_host(lt), map);
     });
   });
 }

@@ -2270,13 +2270,14 @@ void search(cuvs::resources const& res, search_params const& params, index<T> co
 template <typename T>
 void search(cuvs::resources const& res, search_params const& params, index<T> const& idx,
             matrix_view<const T> queries, const int32_t* query_labels, int64_t* neighbors,
-            float* distances, int64_t k, bool labels_on_host)
+            float* distances, int64_t k, bool labels_on_host, const int64_t* id_map)
 {
   expects(idx.has_labels(), "certex: the index has no labels");
   certex_amd::filter_args fa{};
   fa.kind         = 3;
   fa.row_labels   = idx.state().labels.template as<int32_t>();
   fa.query_labels = labels_on_host ? nullptr : query_labels;
+  fa.id_map       = id_map;
   search_impl(res, params, idx, queries, neighbors, distances, k, fa, false,
               labels_on_host ? query_labels : nullptr);
 }
@@ -2552,7 +2553,7 @@ void deserialize(cuvs::resources const& res, std::string const& filename, index<
                           matrix_view<const T>, int64_t*, float*, int64_t, filter);            \
   template void search<T>(cuvs::resources const&, search_params const&, index<T> const&,       \
                           matrix_view<const T>, const int32_t*, int64_t*, float*, int64_t,     \
-                          bool);                                                               \
+                          bool, const int64_t*);                                                               \
   template void serialize<T>(cuvs::resources const&, std::string const&, index<T> const&);     \
   template void deserialize<T>(cuvs::resources const&, std::string const&, index<T>*);
 

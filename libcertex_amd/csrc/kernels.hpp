@@ -155,6 +155,8 @@ struct filter_args {
   // report ids.
   const int32_t* row_ids = nullptr;
   int64_t n_listed       = 0;
+  // the exact-score kernels write id_map[id] as the neighbour (null: the id itself)
+  const int64_t* id_map = nullptr;
 };
 
 /** The id held by stored row `row`. */

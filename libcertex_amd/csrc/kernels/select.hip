@@ -202,7 +202,7 @@ __device__ inline void put_result(const A& a, int64_t q, int j, double s, int64_
     d = float(s);
   }
   a.distances[t] = d;
-  a.neighbors[t] = id < 0 ? -1 : id;
+  a.neighbors[t] = id < 0 ? -1 : (a.filter.id_map != nullptr ? a.filter.id_map[id] : id);
 }
 
 __device__ inline bool keeps(const filter_args& f, int64_t q, uint32_t row)

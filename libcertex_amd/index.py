@@ -364,6 +364,11 @@ class Index:
     def search(self, q, k=10, batch=2048, labels=None, filter=None, anchors=128, probe_lists=2):
         """Exact k nearest neighbours of every query: (distances or similarities, ids), best first
         (certex/index.py:320-351)."""
+        return self._search(q, k, batch, labels, filter, anchors, probe_lists)
+
+    def _search(self, q, k, batch, labels, filter, anchors=128, probe_lists=2, id_map=None):
+        """search(); with labels and id_map (an int64 GPU tensor, an entry per id or more) the ids
+        come back as id_map[id], written so by the search."""
         _require(self.core is not None, "the index is empty: add vectors first")
         single = _to_torch(q).ndim == 1
         Q, kind = self._vectors(q, device=True)
@@ -394,7 +399,13 @@ class Index:
             res = C.resources()
             if ql is not None:
                 lb = C.Borrowed(ql)
-                C.check(L.cuvsCertexSearchWithLabels(res, ctypes.byref(sp), self.core.h, qb.ptr, lb.ptr, ib.ptr, db.ptr))
+                if id_map is not None:
+                    mb = C.Borrowed(id_map)
+                    C.check(L.cuvsCertexSearchWithLabelsMapped(res, ctypes.byref(sp), self.core.h, qb.ptr, lb.ptr,
+                                                               mb.ptr, ib.ptr, db.ptr))
+                else:
+                    C.check(L.cuvsCertexSearchWithLabels(res, ctypes.byref(sp), self.core.h, qb.ptr, lb.ptr, ib.ptr,
+                                                         db.ptr))
             else:
                 wb = None
                 f = C.Filter(0, C.NO_FILTER)

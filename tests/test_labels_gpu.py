@@ -260,3 +260,27 @@ def test_many_labels(gpu):
     for batch in (2048, 257):
         D, I = search(idx, Q, 10, lq, batch=batch)
         check(X, Q, 10, "l2", D, I, row_labels=lx, query_labels=lq)
+
+
+@pytest.mark.parametrize("dtype, d", [(np.uint8, 128), (np.float32, 96)])
+def test_ids_through_a_map(gpu, dtype, d):
+    """The mapped label search writes id_map[id] where the plain one writes id, with labels on the
+    GPU and on the host, -1 where a label holds fewer than k rows; a map that is too short is refused."""
+    rng = np.random.default_rng(d)
+    X = rng.integers(0, 256, (5_003, d)).astype(dtype)
+    Q = rng.integers(0, 256, (200, d)).astype(dtype)
+    lx, lq = rng.integers(0, 6, 5_003).astype(np.int32), rng.integers(0, 8, 200).astype(np.int32)
+    lx[lx == 5] = 4
+    lx[:3] = 5  # three rows
+    idx = certex.Index(d)
+    idx.add(torch.from_numpy(X).cuda(), labels=lx)
+    idx.add(torch.from_numpy(X[:100]).cuda(), labels=lx[:100])
+    m = torch.randint(0, 1 << 40, (6_000,), dtype=torch.int64, device="cuda")
+    for labels in (torch.from_numpy(lq), torch.from_numpy(lq).cuda()):
+        for k in (7, 90):
+            D0, I0 = idx.search(torch.from_numpy(Q).cuda(), k=k, labels=labels)
+            D1, I1 = idx._search(torch.from_numpy(Q).cuda(), k, 2048, labels, None, id_map=m)
+            assert (I0 == -1).any() and torch.equal(D0, D1)
+            assert torch.equal(I1, torch.where(I0 < 0, I0, m[I0.clamp_min(0)]))
+    with pytest.raises(ValueError, match="id map"):
+        idx._search(torch.from_numpy(Q).cuda(), 7, 2048, labels, None, id_map=m[:5_000])
