@@ -211,7 +211,9 @@ struct screen_args {
   // screen: candidate buckets
   uint32_t* cand_count = nullptr;  // [nq_pad]
   uint32_t* cand_rows  = nullptr;  // [nq_pad, cap]
-  float* cand_vals     = nullptr;  // [nq_pad, cap] screen values (fp16 rows only)
+  // [nq_pad, cap] screen values: of fp16 rows, and of int8 rows of more than 256 bytes where the
+  // re-rank asks for them (int32 values in the floats' bits)
+  float* cand_vals     = nullptr;
   int64_t cap          = 0;
   // *most: at least the largest bucket count past cap (exactly where flushes alone fill the
   // bucket), else some count past most_above when a bucket passes that, else as it was
@@ -363,6 +365,10 @@ struct verify_args {
   // candidates: the bucket of each query, or every row when all_rows
   const uint32_t* cand_count;
   const uint32_t* cand_rows;
+  // the candidates' int32 screen values, or null: a larger value is a nearer row (for l2 a value's
+  // rows differ by at most 1 in their score, the parity of |x'|^2), so only the rows that reach the
+  // k-th largest value are scored
+  const int32_t* cand_vals = nullptr;
   int64_t cap;
   bool all_rows;
   // part 1: buckets of at most kSmallBucket candidates (k <= 64), part 2: the others, 0: both. A

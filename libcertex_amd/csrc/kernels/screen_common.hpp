@@ -36,6 +36,11 @@ struct int8_rows {
   __device__ static val_t vmax(val_t a, val_t b) { return max(a, b); }
 };
 
+/** int8 rows whose survivors carry their (exact) screen value, as the bits of a float. */
+struct int8_value_rows : int8_rows {
+  static constexpr bool kValues = true;
+};
+
 struct f16_rows {
   using acc_t  = v4f;
   using frag_t = v8h;

@@ -567,7 +567,13 @@ void anchors_f16_tile(const screen_args& a, hipStream_t stream)
 
 void screen_i8_tile(const screen_args& a, hipStream_t stream)
 {
-  if (a.filter.kind != 0) {
+  if (a.cand_vals != nullptr) {
+    if (a.filter.kind != 0) {
+      launch_tile<int8_value_rows, true, false>(a, stream);
+    } else {
+      launch_tile<int8_value_rows, false, false>(a, stream);
+    }
+  } else if (a.filter.kind != 0) {
     launch_tile<int8_rows, true, false>(a, stream);
   } else {
     launch_tile<int8_rows, false, false>(a, stream);

@@ -64,3 +64,23 @@ def mixture_u8_cuda(n, d=128, n_centres=1000, seed=2, centre_seed=1, sigma=20.0,
         v = centres[c] + torch.randn((m, d), generator=g, device="cuda") * sigma
         out[i : i + m] = v.round().clamp_(0, 255).to(torch.uint8)
     return out
+
+
+def on_fresh_resources(fn):
+    """Runs fn in a thread of its own, whose resources have learned no bucket size from other
+    searches and leave none to them."""
+    import threading
+
+    failed = []
+
+    def body():
+        try:
+            fn()
+        except BaseException as e:  # noqa: B036
+            failed.append(e)
+
+    t = threading.Thread(target=body)
+    t.start()
+    t.join()
+    if failed:
+        raise failed[0]

@@ -292,14 +292,18 @@ def test_bitset_by_row_terms(gpu, dtype, d, lists, keep):
         kk = min(k, rows.size)
         want[:, :kk] = rows[oracle.knn(X[rows], Q, kk, "l2")[1]]
     Qg, mg = torch.from_numpy(Q).cuda(), torch.from_numpy(mask).cuda()
-    for probe in (2, 0) if lists else (2,):
-        D, I = idx.search(Qg, k=k, filter=mg, probe_lists=probe)
-        np.testing.assert_array_equal(I.cpu().numpy(), want)
-        I2, D2 = torch.empty_like(I), torch.empty_like(D)
-        sp = C.SearchParams(128, 2048, probe)
-        qb, ib, db = C.Borrowed(Qg), C.Borrowed(I2), C.Borrowed(D2)
-        wb = C.Borrowed(_pack(mg), dtype_override=(C.kDLUInt, 32))
-        C.check(C.lib().cuvsCertexSearchNoAlloc(C.resources(), ctypes.byref(sp), idx.core.h, qb.ptr, ib.ptr, db.ptr,
-                                                C.Filter(ctypes.addressof(wb.m), C.BITSET)))
-        torch.cuda.synchronize()
-        assert torch.equal(I, I2) and torch.equal(D, D2)
+    def body():
+        for probe in (2, 0) if lists else (2,):
+            D, I = idx.search(Qg, k=k, filter=mg, probe_lists=probe)
+            np.testing.assert_array_equal(I.cpu().numpy(), want)
+            I2, D2 = torch.empty_like(I), torch.empty_like(D)
+            sp = C.SearchParams(128, 2048, probe)
+            qb, ib, db = C.Borrowed(Qg), C.Borrowed(I2), C.Borrowed(D2)
+            wb = C.Borrowed(_pack(mg), dtype_override=(C.kDLUInt, 32))
+            C.check(C.lib().cuvsCertexSearchNoAlloc(C.resources(), ctypes.byref(sp), idx.core.h, qb.ptr, ib.ptr, db.ptr,
+                                                    C.Filter(ctypes.addressof(wb.m), C.BITSET)))
+            torch.cuda.synchronize()
+            assert torch.equal(I, I2) and torch.equal(D, D2)
+
+    torch.cuda.synchronize()
+    data.on_fresh_resources(body)

@@ -200,3 +200,34 @@ def test_wide_tiles_of_few_queries(gpu, dtype, d, nq):
         check(X, Q, k, "l2", D, I)
     D, I = idx.search(torch.from_numpy(Q).cuda(), k=5, filter=torch.from_numpy(mask).cuda())
     check(X, Q, 5, "l2", D, I, bitmap=words(mask))
+
+
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+@pytest.mark.parametrize("k", [32, 33, 64, 65, 600])
+def test_int_wide_by_screen_values(gpu, metric, k):
+    """Wide integer rows with k above 32 rank their survivors by the screen value first: rows whose
+    l2 scores differ only by the parity of the norm, more equal values at the k-th place than the
+    buffer holds (2,500 copies of a row), labels (a partition and a tail) and a bitmap."""
+    def body():
+        d, n = 520, 40_003
+        X = data.uniform_int(n, d, seed=k, dtype=np.uint8) // 4  # many close scores
+        X[100:2_600] = X[99]
+        X[2_600:2_900] = X[2_600]
+        X[2_600:2_900, :300] += np.eye(300, dtype=np.uint8)  # one coordinate off: equal or adjacent scores
+        Q = np.concatenate([X[95:105], X[2_595:2_605], data.uniform_int(50, d, seed=7, dtype=np.uint8) // 4])
+        idx = certex.Index(d, metric=metric)
+        idx.add(torch.from_numpy(X).cuda())
+        D, I = idx.search(torch.from_numpy(Q).cuda(), k=k)
+        check(X, Q, k, metric, D, I)
+        mask = np.random.default_rng(k).random((len(Q), n)) < 0.7
+        D, I = idx.search(torch.from_numpy(Q).cuda(), k=k, filter=torch.from_numpy(mask).cuda())
+        check(X, Q, k, metric, D, I, bitmap=words(mask))
+        lx, lq = np.arange(n, dtype=np.int32) % 3, np.arange(len(Q), dtype=np.int32) % 3
+        lab = certex.Index(d, metric=metric, partition_labels=False)
+        lab.add(torch.from_numpy(X[:39_000]).cuda(), labels=lx[:39_000])
+        lab.partition()
+        lab.add(torch.from_numpy(X[39_000:]).cuda(), labels=lx[39_000:])
+        D, I = lab.search(torch.from_numpy(Q).cuda(), k=k, labels=torch.from_numpy(lq))
+        check(X, Q, k, metric, D, I, row_labels=lx, query_labels=lq)
+
+    data.on_fresh_resources(body)
