@@ -141,9 +141,10 @@ CUVS_EXPORT cuvsError_t cuvsCertexSearchWithLabels(cuvsResources_t res,
 
 /**
  * cuvsCertexSearchWithLabels whose neighbours are reported through `id_map`, an int64 device vector
- * of at least one entry per vector added (cuvsCertexIndexGetSize): id_map[id] instead of id. An
- * addition: a cache that keeps several sequences in one index maps its ids to each one's own as the
- * results are written, not in a pass over them.
+ * of at least one entry per vector added (cuvsCertexIndexGetSize): id_map[id] instead of id. The
+ * map is held against the index in every batch: vectors that another thread adds past it end the
+ * search with an error. An addition: a cache that keeps several sequences in one index maps its ids
+ * to each one's own as the results are written, not in a pass over them.
  */
 CUVS_EXPORT cuvsError_t cuvsCertexSearchWithLabelsMapped(cuvsResources_t res,
                                                          cuvsCertexSearchParams_t params,

@@ -240,13 +240,15 @@ auto no_alloc_scratch_bytes() -> size_t;
  * Exact k nearest neighbours of every query among the vectors of its label (int32 labels, one per
  * query). The labels are in device memory, or in host memory with labels_on_host: the search over
  * the label partition plans its launches from them on the host, and host labels spare it a copy
- * back and a wait for the stream. With id_map (device memory, one entry per id) the neighbours are
- * reported as id_map[id].
+ * back and a wait for the stream. With id_map (n_map entries in device memory, one per id or more)
+ * the neighbours are reported as id_map[id]; a search that meets more ids than entries, also those
+ * that another thread adds between two of its batches, ends with an error.
  */
 template <typename T>
 void search(cuvs::resources const& res, search_params const& params, index<T> const& idx,
             matrix_view<const T> queries, const int32_t* query_labels, int64_t* neighbors,
-            float* distances, int64_t k, bool labels_on_host = false, const int64_t* id_map = nullptr);
+            float* distances, int64_t k, bool labels_on_host = false, const int64_t* id_map = nullptr,
+            int64_t n_map = 0);
 
 /**
  * The ids in the order of the stored rows (reference Index.list_order, certex/index.py:353-359,

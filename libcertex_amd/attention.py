@@ -112,14 +112,10 @@ class KeyCache:
         if key not in self._labels:
             heads = torch.arange(self.n_kv_heads, device="cuda", dtype=torch.int32)
             self._labels[key] = heads.repeat_interleave(n)
+        rows = _fit(K, self.dtype, "keys").reshape(self.n_kv_heads * n, self.head_dim).contiguous()
         n0 = self.n_kv_heads * self.size  # the shared index's first new id
-        # the head labels are built here (non-negative): no check that would wait for the GPU
-        self.index._add(
-            _fit(K, self.dtype, "keys").reshape(self.n_kv_heads * n, self.head_dim).contiguous(),
-            self._labels[key],
-            check_labels=False,
-        )
         need = n0 + self.n_kv_heads * n
+        # the ids' map first: a search may report the new keys as soon as the index holds them
         if self.local is None or self.local.shape[0] < need:
             grown = torch.empty(max(need, 2 * (0 if self.local is None else self.local.shape[0])),
                                 device="cuda", dtype=torch.int64)
@@ -128,6 +124,8 @@ class KeyCache:
             self.local = grown
         self.local[n0:need].view(self.n_kv_heads, n).copy_(
             torch.arange(self.size, self.size + n, device="cuda", dtype=torch.int64))
+        # the head labels are built here (non-negative): no check that would wait for the GPU
+        self.index._add(rows, self._labels[key], check_labels=False)
         self.size += n
         core = self.index.core
         if (core.size - core.n_partitioned) * 16 > core.size:
@@ -156,9 +154,16 @@ class KeyCache:
             # read-back from the GPU
             self._labels[key] = (torch.arange(H, dtype=torch.int32) // r).repeat_interleave(m)
         labels = self._labels[key]
-        D, I = self.index._search(
-            Q.reshape(H * m, d), k, batch or max(2048, H * m), labels, None, id_map=self.local
-        )
+        while True:
+            local = self.local
+            try:
+                D, I = self.index._search(
+                    Q.reshape(H * m, d), k, batch or max(2048, H * m), labels, None, id_map=local
+                )
+                break
+            except ValueError:
+                if local is self.local:  # else another thread's append outgrew this map: take the new one
+                    raise
         scores = D.reshape(H, m, k)
         ids = I.reshape(H, m, k)
         return (scores[:, 0], ids[:, 0]) if single else (scores, ids)

@@ -485,12 +485,13 @@ cuvsError_t cuvsCertexSearchWithLabelsMapped(cuvsResources_t res,
                         distances->dl_tensor.shape[1] == k,
                       "output shapes do not match the queries");
       const int64_t* map = nullptr;
+      int64_t n_map      = 0;
       if (id_map != nullptr) {
-        map = device_data<const int64_t>(id_map, 1, "the id map");
-        certex::expects(id_map->dl_tensor.shape[0] >= idx.size(),
-                        "certex: the id map needs one entry per vector");
+        map   = device_data<const int64_t>(id_map, 1, "the id map");
+        n_map = id_map->dl_tensor.shape[0];
+        certex::expects(n_map >= idx.size(), "certex: the id map needs one entry per vector");
       }
-      certex::search<T>(r, p, idx, q, ql, nb, ds, k, is_host(lt), map);
+      certex::search<T>(r, p, idx, q, ql, nb, ds, k, is_host(lt), map, n_map);
     });
   });
 }

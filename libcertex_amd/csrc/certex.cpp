@@ -1574,6 +1574,12 @@ void search_impl(cuvs::resources const& res, search_params const& params, index<
   expects(queries.cols == st.dim, "dimension mismatch");
   expects(k >= 1 && k <= 2048, "certex returns at most 2048 neighbors per query");
   expects(st.size >= k, "the index holds fewer than k vectors");
+  // an entry per id that a batch may report; checked again under the lock of each batch, whose rows
+  // an update of another thread may have added after this call began
+  const auto check_map = [&] {
+    expects(fa.id_map == nullptr || fa.n_map >= st.size, "certex: the id map needs one entry per vector");
+  };
+  check_map();
   const int64_t nq = queries.rows;
   if (nq == 0) { return; }
   if (t_stats_on) { res.sync(); }
@@ -1617,6 +1623,7 @@ void search_impl(cuvs::resources const& res, search_params const& params, index<
   };
   for (int64_t b0 = 0; b0 < nq; b0 += bs) {
     std::shared_lock batch_view(st.rw);  // the rows of this batch stay fixed during updates
+    check_map();
     st.await_updates(res.state().stream);
     run(b0, std::min(bs, nq - b0));
   }
@@ -2279,7 +2286,7 @@ void search(cuvs::resources const& res, search_params const& params, index<T> co
 template <typename T>
 void search(cuvs::resources const& res, search_params const& params, index<T> const& idx,
             matrix_view<const T> queries, const int32_t* query_labels, int64_t* neighbors,
-            float* distances, int64_t k, bool labels_on_host, const int64_t* id_map)
+            float* distances, int64_t k, bool labels_on_host, const int64_t* id_map, int64_t n_map)
 {
   expects(idx.has_labels(), "certex: the index has no labels");
   certex_amd::filter_args fa{};
@@ -2287,6 +2294,7 @@ void search(cuvs::resources const& res, search_params const& params, index<T> co
   fa.row_labels   = idx.state().labels.template as<int32_t>();
   fa.query_labels = labels_on_host ? nullptr : query_labels;
   fa.id_map       = id_map;
+  fa.n_map        = n_map;
   search_impl(res, params, idx, queries, neighbors, distances, k, fa, false,
               labels_on_host ? query_labels : nullptr);
 }
@@ -2562,7 +2570,7 @@ void deserialize(cuvs::resources const& res, std::string const& filename, index<
                           matrix_view<const T>, int64_t*, float*, int64_t, filter);            \
   template void search<T>(cuvs::resources const&, search_params const&, index<T> const&,       \
                           matrix_view<const T>, const int32_t*, int64_t*, float*, int64_t,     \
-                          bool, const int64_t*);                                                               \
+                          bool, const int64_t*, int64_t);                                     \
   template void serialize<T>(cuvs::resources const&, std::string const&, index<T> const&);     \
   template void deserialize<T>(cuvs::resources const&, std::string const&, index<T>*);
 

@@ -155,8 +155,9 @@ struct filter_args {
   // report ids.
   const int32_t* row_ids = nullptr;
   int64_t n_listed       = 0;
-  // the exact-score kernels write id_map[id] as the neighbour (null: the id itself)
+  // the exact-score kernels write id_map[id] as the neighbour (null: the id itself); n_map entries
   const int64_t* id_map = nullptr;
+  int64_t n_map         = 0;
 };
 
 /** The id held by stored row `row`. */

@@ -108,3 +108,28 @@ def test_group_table_of_an_earlier_search(gpu):
     cache.append(keys[:, :19_000]).append(keys[:, 19_000:])  # the partition, then a tail
     scores, ids = cache.topk(q, 16)
     assert_exact(q, keys, scores, ids, 16)
+
+
+def test_append_beside_a_search(gpu):
+    """The map from the shared index's ids to a head's own holds the new keys before the index does,
+    and a search whose map an append outgrew takes the new one."""
+    q, K = data(n_kv=2, H=4, n=900, m=3, d=64, seed=9)
+    cache = certex.KeyCache(2, 64, k=5).append(K[:, :300])
+    index, add, search = cache.index, cache.index._add, cache.index._search
+    seen = []
+
+    def add_checked(rows, labels, check_labels):
+        n0 = index.core.size
+        new = cache.local[n0 : n0 + len(rows)].cpu().numpy()
+        seen.append(np.array_equal(new, np.tile(np.arange(300, 900), 2)))
+        return add(rows, labels, check_labels)
+
+    def search_late(*args, **kw):  # with the map of before an append
+        index._search = search
+        cache.append(K[:, 300:])
+        return search(*args, **kw)
+
+    index._add, index._search = add_checked, search_late
+    scores, ids = cache.topk(q)
+    assert seen == [True]
+    assert_exact(q, K, scores, ids, 5)

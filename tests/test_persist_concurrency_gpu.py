@@ -4,6 +4,7 @@ answer over one of the published prefixes."""
 
 import os
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -76,6 +77,51 @@ def test_load_rejects_foreign_files(gpu, tmp_path):
     with pytest.raises(ValueError):
         (tmp_path / "junk").write_bytes(b"hello world")
         certex.Index.load(tmp_path / "junk")
+
+
+def search_while_adding(search, add):
+    """search(nq) in a thread of its own and add() while it runs: what the search returned (or the
+    exception that ended it). A search that was over before the rows were added runs again with more
+    queries."""
+    for nq in (5_000, 20_000, 80_000):
+        out = []
+
+        def body():
+            try:
+                with torch.cuda.stream(torch.cuda.Stream()):
+                    out.append(search(nq))
+                    torch.cuda.current_stream().synchronize()
+            except BaseException as e:  # noqa: B036
+                out.append(e)
+
+        t = threading.Thread(target=body)
+        t.start()
+        time.sleep(0.1)
+        add()
+        torch.cuda.synchronize()
+        running = t.is_alive()
+        t.join()
+        if running or isinstance(out[0], BaseException):
+            return out[0]
+    pytest.fail("no search was running when rows were added")
+
+
+def test_rows_added_past_an_id_map(gpu):
+    """A mapped label search of many batches: rows that another thread adds past its map between two
+    of them end it. The map is the start of a longer tensor, whose other entries no result may hold."""
+    X = data.mixture_u8(3_000, seed=41)
+    Xg = torch.from_numpy(X).cuda()
+    idx = certex.Index(128)
+    idx.add(Xg[:2_000], labels=torch.zeros(2_000, dtype=torch.int32))
+    whole = torch.arange(40_000, device="cuda")
+
+    def search(nq):
+        n = idx.core.size
+        return idx._search(Xg[2_000:].repeat(nq // 1_000, 1), 5, 1, torch.zeros(nq, dtype=torch.int32), None,
+                           id_map=whole[:n])
+
+    got = search_while_adding(search, lambda: idx.add(Xg[2_000:], labels=torch.zeros(1_000, dtype=torch.int32)))
+    assert isinstance(got, ValueError) and "id map" in str(got), got
 
 
 @pytest.mark.parametrize("dtype", [np.uint8, np.float32])
