@@ -106,11 +106,13 @@ struct matrix_view {
   bool on_device = true;
 };
 
-/** Filter of a search (reference Filter, detail/kernels.hpp:39-62). */
+/** Filter of a search (reference Filter, detail/kernels.hpp:39-62). Vectors that another thread
+ *  adds during the search, past the ids that the filter covers, are excluded. */
 struct filter {
   enum class kind : int { none = 0, bitset = 1, bitmap = 2 };
   kind type             = kind::none;
   const uint32_t* words = nullptr;  // device words; bit j of word i is entry 32 i + j
+  int64_t ids           = 0;  // ids that each mask covers; 0: the index's vectors as the search begins
 };
 
 /** Counters of the searches of the calling thread (reference detail/kernels.hpp:256-263). */

@@ -400,10 +400,13 @@ cuvsError_t search_c(cuvsResources_t res,
         auto* m = reinterpret_cast<DLManagedTensor*>(filter.addr);
         check_tensor<uint32_t>(m, 1, "the filter words");
         certex::expects(is_device(m->dl_tensor), "certex: the filter words must be on the device");
-        const int64_t bits = filter.type == BITSET ? idx.size() : q.rows * idx.size();
-        certex::expects(m->dl_tensor.shape[0] * 32 >= bits, "certex: too few filter words");
+        const int64_t size = idx.size();  // once: it grows while other threads add
+        const int64_t bits = m->dl_tensor.shape[0] * 32;
+        certex::expects(bits >= (filter.type == BITSET ? size : q.rows * size),
+                        "certex: too few filter words");
         f.type  = filter.type == BITSET ? certex::filter::kind::bitset : certex::filter::kind::bitmap;
         f.words = data_of<const uint32_t>(m->dl_tensor);
+        f.ids   = filter.type == BITSET ? bits : size;
       } else {
         certex::expects(filter.type == NO_FILTER, "certex: unsupported filter type");
       }

@@ -330,13 +330,23 @@ void size_groups(anchor_plan& p, int64_t max_anchors, int64_t tail_anchors, int6
   p.n_groups    = *part_groups + (tail_steps + g - 1) / g;
 }
 
-/** The anchors of the anchor copy from anchor `first` on. */
-auto plan_anchors(index_state const& st, int64_t first, int64_t nq_pad, int k) -> anchor_plan
+/**
+ * Rows that a batch looks at: all, or the ids that its bitset or bitmap covers. Ids past those, which
+ * another thread added after the search began, are the last stored rows (lists hold the ids of the
+ * build alone, and every filter covers at least them).
+ */
+auto rows_in_view(index_state const& st, certex_amd::filter_args const& fa) -> int64_t
+{
+  return fa.kind == 1 || fa.kind == 2 ? std::min<int64_t>(st.size, fa.n_ids) : int64_t(st.size);
+}
+
+/** The anchors of the anchor copy among the ids [0, size), from anchor `first` on. */
+auto plan_anchors(index_state const& st, int64_t size, int64_t first, int64_t nq_pad, int k) -> anchor_plan
 {
   anchor_plan p{};
   p.stride   = std::max(1, st.anchor_stride);
   p.first    = first;
-  p.n_anchor = (st.size + p.stride - 1) / p.stride - first;
+  p.n_anchor = (size + p.stride - 1) / p.stride - first;
   int64_t part = 0;
   size_groups(p, p.n_anchor, 0, nq_pad, k, &part);
   return p;
@@ -897,15 +907,15 @@ auto plan_table(cuvs::resources const& res, index_state const& st, const void* q
   if (probe) {  // the anchors of the ids added after the lists (the first id >= n_listed on)
     const int64_t s     = std::max(1, st.anchor_stride);
     const int64_t first = (st.n_listed + s - 1) / s;
-    tp.anchors          = first < (st.size + s - 1) / s;
-    if (tp.anchors) { tp.ap = plan_anchors(st, first, nq_pad, k); }
+    tp.anchors          = first < (rows_in_view(st, fa) + s - 1) / s;
+    if (tp.anchors) { tp.ap = plan_anchors(st, rows_in_view(st, fa), first, nq_pad, k); }
     const int64_t acols = tp.anchors ? tp.ap.n_groups : 0;
     probe = nq_pad * (acols + tp.pp.cols) * 4 <= kTableBytes;
   }
   if (!probe) {  // anchors over every row
     tp.pp      = probe_plan{};
     tp.anchors = true;
-    tp.ap      = plan_anchors(st, 0, nq_pad, k);
+    tp.ap      = plan_anchors(st, rows_in_view(st, fa), 0, nq_pad, k);
   }
   tp.n_groups = (tp.anchors ? tp.ap.n_groups : 0) + tp.pp.cols;
   return tp;
@@ -989,8 +999,9 @@ void mask_rows(cuvs::resources const& res, index_state const& st, certex_amd::fi
 {
   auto& rs               = res.state();
   const int64_t stride   = std::max(1, st.anchor_stride);
-  const int64_t n_anchor = (st.size + stride - 1) / stride;
-  const int64_t rows     = (st.size + 3) / 4 * 4;  // the anchors' terms start 16-byte aligned too
+  const int64_t size     = rows_in_view(st, fa);
+  const int64_t n_anchor = (size + stride - 1) / stride;
+  const int64_t rows     = (size + 3) / 4 * 4;  // the anchors' terms start 16-byte aligned too
   const size_t bytes     = size_t(rows + n_anchor) * 4;
   if (fa.kind != 1 || rs.arena != nullptr || bytes > kMaskBytes) { return; }
   char* terms = nullptr;
@@ -1000,7 +1011,7 @@ void mask_rows(cuvs::resources const& res, index_state const& st, certex_amd::fi
     return;
   }
   char* anchor_terms = terms + size_t(rows) * 4;
-  certex_amd::mask_terms(st.rowc.p, st.size, st.anchor_rowc.p, n_anchor, stride, !is_int(st.type), fa,
+  certex_amd::mask_terms(st.rowc.p, size, st.anchor_rowc.p, n_anchor, stride, !is_int(st.type), fa,
                          terms, anchor_terms, rs.stream);
   sa.rowc        = terms;
   sa.anchor_rowc = anchor_terms;
@@ -1015,7 +1026,7 @@ void search_batch_int(cuvs::resources const& res, index_state const& st, const v
 {
   auto& rs             = res.state();
   hipStream_t stream   = rs.stream;
-  const int64_t size   = st.size;
+  const int64_t size   = rows_in_view(st, fa);
   const int64_t nq_pad = certex_amd::pad_queries(B);
   const uint8_t flip   = st.type == vtype::u8 ? 0x80 : 0;
   fa.q0                = q0;
@@ -1152,7 +1163,7 @@ void search_batch_float(cuvs::resources const& res, index_state const& st, const
 {
   auto& rs             = res.state();
   hipStream_t stream   = rs.stream;
-  const int64_t size   = st.size;
+  const int64_t size   = rows_in_view(st, fa);
   const int64_t nq_pad = certex_amd::pad_queries(B);
   const auto t         = elem_of(st.type);
   const bool wide      = st.halves > 128;  // the K-loop screen
@@ -1563,6 +1574,19 @@ void routed_batch(cuvs::resources const& res, index_state const& st, batch_fn ba
   // no wait here: the next use of the staging waits for this batch's copy of the tables
 }
 
+/** The filter of a search over an index of `size` vectors. */
+auto to_args(filter const& f, int64_t size) -> certex_amd::filter_args
+{
+  certex_amd::filter_args fa{};
+  if (f.type != filter::kind::none) {
+    expects(f.words != nullptr, "certex: a filter needs its words");
+    fa.kind  = f.type == filter::kind::bitset ? 1 : 2;
+    fa.words = f.words;
+    fa.n_ids = f.ids > 0 ? f.ids : size;
+  }
+  return fa;
+}
+
 template <typename T>
 void search_impl(cuvs::resources const& res, search_params const& params, index<T> const& idx,
                  matrix_view<const T> queries, int64_t* neighbors, float* distances, int64_t k,
@@ -1714,13 +1738,7 @@ void search_without_allocation(cuvs::resources const& res, search_params const& 
                                index<T> const& idx, matrix_view<const T> queries,
                                int64_t* neighbors, float* distances, int64_t k, filter f)
 {
-  certex_amd::filter_args fa{};
-  if (f.type != filter::kind::none) {
-    expects(f.words != nullptr, "certex: a filter needs its words");
-    fa.kind      = f.type == filter::kind::bitset ? 1 : 2;
-    fa.words     = f.words;
-    fa.bitmap_ld = idx.size();
-  }
+  const certex_amd::filter_args fa = to_args(f, idx.size());
   expects(!t_capture.on, "certex: a capture covers the allocating search");
   char* base = scratch_of(res.device());
   scratch_turn turn(res.device(), static_cast<hipStream_t>(res.stream()));
@@ -2273,13 +2291,7 @@ void search(cuvs::resources const& res, search_params const& params, index<T> co
             matrix_view<const T> queries, int64_t* neighbors, float* distances, int64_t k,
             filter f)
 {
-  certex_amd::filter_args fa{};
-  if (f.type != filter::kind::none) {
-    expects(f.words != nullptr, "certex: a filter needs its words");
-    fa.kind      = f.type == filter::kind::bitset ? 1 : 2;
-    fa.words     = f.words;
-    fa.bitmap_ld = idx.size();
-  }
+  const certex_amd::filter_args fa = to_args(f, idx.size());
   search_impl(res, params, idx, queries, neighbors, distances, k, fa);
 }
 

@@ -146,7 +146,9 @@ void iota_i32(int32_t* p, int64_t n, int32_t first, hipStream_t stream);
 struct filter_args {
   int kind = 0;                     // 0 none, 1 bitset over rows, 2 bitmap per query, 3 labels
   const uint32_t* words = nullptr;  // bitset / bitmap words
-  int64_t bitmap_ld = 0;            // bits per bitmap row (= index size when built)
+  // ids that each mask covers (of a bitmap: its bits per query). Later ids, which another thread adds
+  // during the search, are the last stored rows, and no pass of a filtered search reaches them
+  int64_t n_ids = 0;
   int64_t q0 = 0;                   // first query of the batch (bitmap row, label offset)
   const int32_t* row_labels = nullptr;
   const int32_t* query_labels = nullptr;  // of all queries of the search

@@ -196,7 +196,7 @@ __device__ inline bool keeps_id(const filter_args& f, int64_t q, uint32_t id)
   switch (f.kind) {
     case 1: return (f.words[id >> 5] >> (id & 31)) & 1u;
     case 2: {
-      const int64_t bit = (f.q0 + q) * f.bitmap_ld + id;
+      const int64_t bit = (f.q0 + q) * f.n_ids + id;
       return (f.words[bit >> 5] >> (bit & 31)) & 1u;
     }
     case 3: return f.row_labels[id] == f.query_labels[f.q0 + q];

@@ -212,7 +212,7 @@ __device__ inline bool keeps(const filter_args& f, int64_t q, uint32_t row)
   switch (f.kind) {
     case 1: return (f.words[row >> 5] >> (row & 31)) & 1u;
     case 2: {
-      const int64_t bit = (f.q0 + q) * f.bitmap_ld + row;
+      const int64_t bit = (f.q0 + q) * f.n_ids + row;
       return (f.words[bit >> 5] >> (bit & 31)) & 1u;
     }
     case 3: return f.row_labels[row] == f.query_labels[f.q0 + q];

@@ -124,6 +124,42 @@ def test_rows_added_past_an_id_map(gpu):
     assert isinstance(got, ValueError) and "id map" in str(got), got
 
 
+@pytest.mark.parametrize("entry", ["cuvsCertexSearch", "cuvsCertexSearchNoAlloc"])
+@pytest.mark.parametrize("per_query", [False, True])
+def test_rows_added_past_a_filter(gpu, per_query, entry):
+    """A filtered search of many batches (row terms, or the filtered kernels of a search without
+    allocation and of a mask per query): rows that another thread adds between two of them, whose ids
+    the filter does not cover, are in no result. The filter words are the start of a longer tensor
+    with every later bit set."""
+    import ctypes
+
+    from libcertex_amd import _capi as C
+
+    X = data.mixture_u8(3_008, seed=43)
+    Xg = torch.from_numpy(X).cuda()
+    idx = certex.Index(128)
+    idx.add(Xg[:2_048])
+    words = torch.full((6_000_000,), -1, dtype=torch.int32, device="cuda")
+
+    def search(nq):
+        nq //= 2 if per_query else 1
+        n = idx.core.size
+        Q = Xg[2_048:].repeat(nq // 960 + 1, 1)[:nq].contiguous()
+        I = torch.empty((nq, 5), dtype=torch.int64, device="cuda")
+        D = torch.empty((nq, 5), dtype=torch.float32, device="cuda")
+        sp = C.SearchParams(128, 1, 2)
+        w = words[: (n * (nq if per_query else 1) + 31) // 32]
+        qb, ib, db, wb = C.Borrowed(Q), C.Borrowed(I), C.Borrowed(D), C.Borrowed(w, dtype_override=(C.kDLUInt, 32))
+        C.check(getattr(C.lib(), entry)(C.resources(), ctypes.byref(sp), idx.core.h, qb.ptr, ib.ptr, db.ptr,
+                                        C.Filter(ctypes.addressof(wb.m), C.BITMAP if per_query else C.BITSET)))
+        torch.cuda.current_stream().synchronize()
+        return n, I
+
+    n, I = search_while_adding(search, lambda: idx.add(Xg[2_048:]))
+    assert bool((I >= 0).all()) and int(I.max()) < n
+    assert bool((idx.search(Xg[2_048:], k=1)[1][:, 0] >= 2_048).all())
+
+
 @pytest.mark.parametrize("dtype", [np.uint8, np.float32])
 def test_concurrent_search_and_add(gpu, dtype):
     """Searches on three streams while a fourth adds rows: every search equals the oracle on one
