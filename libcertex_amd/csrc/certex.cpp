@@ -1610,17 +1610,23 @@ void search_impl(cuvs::resources const& res, search_params const& params, index<
   const int64_t bs   = std::max(1, params.batch_size);
   const size_t qrow  = size_t(st.dim) * sizeof(T);
   const batch_fn batch = is_int(st.type) ? search_batch_int : search_batch_float;
-  // a search without allocation screens label queries through the label filter: routing a
-  // batch over the label partition stages its tables in pinned host memory
-  const bool route = fa.kind == 3 && st.label_part.n > 0 && !no_alloc;
-  if (host_labels != nullptr && !route) {
-    // the label filter reads the query labels on the GPU: one copy through pinned staging
-    auto& rs  = res.state();
-    auto* dev = static_cast<int32_t*>(rs.get(cuvs::detail::ws_qlabels, size_t(nq) * 4));
-    std::memcpy(rs.stage(size_t(nq) * 4), host_labels, size_t(nq) * 4);
-    rs.copy_staged(dev, size_t(nq) * 4);
-    fa.query_labels = dev;
-  }
+  bool route = false;
+  // a label search's view of the index, under the lock of each batch: additions move the row labels,
+  // and labels set for partitioned rows drop the partition
+  const auto view_labels = [&] {
+    fa.row_labels = st.labels.as<int32_t>();
+    // a search without allocation screens label queries through the label filter: routing a
+    // batch over the label partition stages its tables in pinned host memory
+    route = st.label_part.n > 0 && !no_alloc;
+    if (host_labels != nullptr && !route && fa.query_labels == nullptr) {
+      // the label filter reads the query labels on the GPU: one copy through pinned staging
+      auto& rs  = res.state();
+      auto* dev = static_cast<int32_t*>(rs.get(cuvs::detail::ws_qlabels, size_t(nq) * 4));
+      std::memcpy(rs.stage(size_t(nq) * 4), host_labels, size_t(nq) * 4);
+      rs.copy_staged(dev, size_t(nq) * 4);
+      fa.query_labels = dev;
+    }
+  };
   std::function<void(int64_t, int64_t)> run = [&](int64_t b0, int64_t B) {
     if (no_alloc) { res.state().arena_reset(); }
     try {
@@ -1648,6 +1654,7 @@ void search_impl(cuvs::resources const& res, search_params const& params, index<
   for (int64_t b0 = 0; b0 < nq; b0 += bs) {
     std::shared_lock batch_view(st.rw);  // the rows of this batch stay fixed during updates
     check_map();
+    if (fa.kind == 3) { view_labels(); }
     st.await_updates(res.state().stream);
     run(b0, std::min(bs, nq - b0));
   }
@@ -2302,8 +2309,7 @@ void search(cuvs::resources const& res, search_params const& params, index<T> co
 {
   expects(idx.has_labels(), "certex: the index has no labels");
   certex_amd::filter_args fa{};
-  fa.kind         = 3;
-  fa.row_labels   = idx.state().labels.template as<int32_t>();
+  fa.kind         = 3;  // row_labels: search_impl, under its lock
   fa.query_labels = labels_on_host ? nullptr : query_labels;
   fa.id_map       = id_map;
   fa.n_map        = n_map;

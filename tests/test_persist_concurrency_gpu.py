@@ -160,6 +160,56 @@ def test_rows_added_past_a_filter(gpu, per_query, entry):
     assert bool((idx.search(Xg[2_048:], k=1)[1][:, 0] >= 2_048).all())
 
 
+@pytest.mark.parametrize("host_labels", [True, False])
+def test_row_labels_moved_during_a_label_search(gpu, host_labels):
+    """A label search of many batches while rows added past the index's capacity move its row labels:
+    the last queries, searched after that, see the new rows."""
+    X = data.mixture_u8(3_008, seed=45)
+    Xg = torch.from_numpy(X).cuda()
+    labels = lambda n: torch.zeros(n, dtype=torch.int32)  # noqa: E731
+    idx = certex.Index(128, partition_labels=False)
+    idx.add(Xg[:2_048], labels=labels(2_048))
+    new = len(X) - 2_048
+
+    def search(nq):
+        n, lq = idx.core.size, labels(nq)
+        Q = Xg[2_048:].repeat(nq // new + 1, 1)[:nq]
+        return n, nq, idx.search(Q, k=1, batch=1, labels=lq if host_labels else lq.cuda())[1]
+
+    n, nq, I = search_while_adding(search, lambda: idx.add(Xg[2_048:], labels=labels(new)))
+    last = int(I[-1, 0])
+    assert last >= 2_048 and np.array_equal(X[2_048 + (last - 2_048) % new], X[2_048 + (nq - 1) % new])
+    assert int(I.max()) < idx.core.size
+
+
+@pytest.mark.parametrize("host_labels", [True, False])
+def test_partition_dropped_during_a_label_search(gpu, host_labels):
+    """A routed label search of many batches while another thread gives partitioned rows new labels,
+    which drops the partition: the last query is answered by the new labels, every id once."""
+    import ctypes
+
+    from libcertex_amd import _capi as C
+
+    X = data.mixture_u8(4_000, seed=47)
+    Q = data.mixture_u8(1_000, seed=48)
+    idx = certex.Index(128)
+    idx.add(X, labels=torch.zeros(4_000, dtype=torch.int32))
+    Qg = torch.from_numpy(Q).cuda()
+
+    def search(nq):
+        lq = torch.zeros(nq, dtype=torch.int32)
+        return idx.search(Qg.repeat(nq // 1_000, 1), k=20, batch=1, labels=lq if host_labels else lq.cuda())[1]
+
+    def relabel():
+        lb = C.Borrowed(torch.ones(1_500, dtype=torch.int32, device="cuda"))
+        C.check(C.lib().cuvsCertexSetLabels(C.resources(), lb.ptr, 0, idx.core.h))
+
+    I = search_while_adding(search, relabel)
+    assert idx.core.n_partitioned == 0
+    want = oracle.knn(X[1_500:], Q[-1:], 20, "l2")[1] + 1_500
+    np.testing.assert_array_equal(I[-1:].cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("dtype", [np.uint8, np.float32])
 def test_concurrent_search_and_add(gpu, dtype):
     """Searches on three streams while a fourth adds rows: every search equals the oracle on one
