@@ -1282,20 +1282,34 @@ void search_batch_float(cuvs::resources const& res, index_state const& st, const
   bool verified = false;
   // a capture reads the buckets before the verification (which compacts them in place)
   const bool capture = t_capture.on;
-  const bool waves   = k <= 64;  // part 1 of the re-rank covers buckets of up to small_bucket_f
-  bool large         = true;
+  // k <= 64: the small kernel behind the screen (part 1) and, when the host then learns of larger
+  // buckets than it takes, the block kernel for those (part 2). The GPU idles before part 2, so that
+  // where some bucket is bound to be larger the block kernel takes them all (part 0): a query
+  // leaves k rows per anchor on average, the fullest of a batch about 1.6 times as many; or the latest
+  // such batch had larger ones. 2,048 queries over 100,000 x 128 float32 at an anchor stride of 16,
+  // parts 1 and 2 / part 0: k = 32 (none larger) 179 / 207 us, k = 40 218 / 212, k = 48 223 / 218, k =
+  // 64 259 / 234; 400 over 30,000 x 512: k = 40 (none larger) 94 / 96, k = 48 116 / 98, k = 64 128 / 101
+  const int64_t small   = certex_amd::small_bucket_f(B);
+  const int64_t average = tp.pp.n_pairs > 0 ? k : k * std::max<int64_t>(1, tp.ap.stride);
+  const bool parts      = k <= 64 && 8 * average <= 5 * small && average < rs.large_from;
+  bool large            = true;
   if (!all_rows) {
     sa.theta = theta;
     all_rows = !screen_into_buckets(
       res, nq_pad, size, sa,
       screen_pass(st, route, wide ? certex_amd::screen_f16_tile : certex_amd::screen_f16), bc, rows,
-      cap, &vals, waves ? certex_amd::small_bucket_f(B) : INT32_MAX, &large,
+      cap, &vals, k <= 64 ? small : INT32_MAX, &large,
       [&](certex_amd::publish_args pub) {
-        if (!capture) { verify(false, waves ? 1 : 0, pub); }
+        if (!capture) { verify(false, parts ? 1 : 0, pub); }
         return !capture;
       });
     verified = !all_rows && !capture;
-    if (verified && waves && large) { verify(false, 2, {}); }
+    if (verified && parts && large) { verify(false, 2, {}); }
+    if (k <= 64 && large) {
+      rs.large_from = std::min(rs.large_from, average);
+    } else if (k <= 64 && average >= rs.large_from) {
+      rs.large_from = INT64_MAX;
+    }
   }
   if (capture) {
     capture_common(st, tp, B, nq_pad, k, all_rows, cap, route, stream);

@@ -133,6 +133,9 @@ struct resources_state {
   bool owns_stream    = false;
   int64_t bucket_cap  = 1024;  // survivors per query kept by the last searches
   bool spill_pool     = false;  // a screen's LDS survivor lists overflowed: provide a spill pool
+  // float searches of k <= 64: k times the rows per anchor from which the latest batch had buckets
+  // larger than the small re-rank takes (it only picks the kernels of the next batch's re-rank)
+  int64_t large_from  = INT64_MAX;
   device_buffer slots[ws_n_slots];
   void* host_small    = nullptr;  // pinned host words for counters read back by the host
   uint32_t ticket      = 0;  // of the latest publication into host_small (publish_args)

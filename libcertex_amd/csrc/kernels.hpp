@@ -532,7 +532,9 @@ struct verify_f_args {
   int64_t* neighbors;
   const int32_t* out_rows = nullptr;  // as in verify_args
   publish_args publish;
-  int part          = 0;   // as in verify_args, buckets of at most small_bucket_f candidates
+  // 0: the block kernel for every bucket; with screen values and k <= 64 in two parts, 1: the small
+  // kernel for the buckets of at most small_bucket_f candidates, 2: the block kernel for the others
+  int part          = 0;
   int64_t small_max = -1;  // set by the launcher: buckets up to this size are the small kernel's
 };
 

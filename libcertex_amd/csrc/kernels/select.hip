@@ -2240,12 +2240,10 @@ void verify_topk_f(const verify_f_args& a, hipStream_t stream)
 {
   if (a.nq == 0) { return; }
   verify_f_args b = a;
-  b.small_max     = -1;
-  if (!a.all_rows && a.cand_vals != nullptr && a.k <= 64) {
-    b.small_max = small_bucket_f(a.nq);
-    b.publish   = {};
-    if (a.part != 2) { verify_small_f(a, stream); }
-    if (a.part == 1) { return; }
+  b.small_max     = a.part == 2 ? small_bucket_f(a.nq) : -1;
+  if (a.part == 1) {
+    verify_small_f(a, stream);
+    return;
   }
   // room for k scored rows plus a chunk of k / 2 more (at least the final sort's power of two):
   // less LDS per block than 4 k, so more blocks share a CU

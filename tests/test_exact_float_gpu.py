@@ -263,3 +263,43 @@ def test_bfloat16_vectors(gpu, metric, d, tmp_path):
     D2, I2 = again.search(Qb.cuda(), k=20)
     torch.cuda.synchronize()
     assert torch.equal(I2, I) and torch.equal(D2, D)
+
+
+def test_rerank_launches_behind_the_screen(gpu):
+    """The float re-rank (k <= 64) is launched whole behind the screen where the buckets are bound to
+    exceed the small kernel's (k = 64 at a stride of 16), or did in the latest batch of as many
+    neighbours; else its small kernel is, and the block kernel follows only for larger buckets. All of
+    them give the exhaustive answer."""
+    import ctypes
+
+    from libcertex_amd import _capi as C
+
+    X = data.gaussian(60_000, 32, 91)
+    heavy = X.copy()
+    heavy[20_000:23_000] = heavy[20_000]
+    Q = data.gaussian(300, 32, 92)
+    Q[::7] = heavy[20_000] + 1e-3 * Q[::7]
+
+    def search(idx, base, k):
+        ms, launches = (ctypes.c_double * 4)(), (ctypes.c_int64 * 4)()
+        C.check(C.lib().cuvsCertexTimingBegin())
+        D, I = idx.search(Q, k=k)
+        C.check(C.lib().cuvsCertexTimingEnd(ms, launches))
+        s, i = oracle.knn(base, Q, k, "l2")
+        np.testing.assert_array_equal(I, i)
+        np.testing.assert_array_equal(D, s.astype(np.float32))
+        return launches[3]
+
+    def body():
+        light, dense = certex.Index(32, anchor_stride=16), certex.Index(32, anchor_stride=16)
+        light.add(X)
+        dense.add(heavy)
+        search(light, X, 64)  # the buckets' capacity grows to what k = 64 keeps
+        assert search(light, X, 64) == 1
+        assert [search(light, X, 10) for _ in range(2)] == [1, 1]
+        search(dense, heavy, 10)  # grows the buckets again, parts 1 and 2
+        assert [search(dense, heavy, 10) for _ in range(2)] == [1, 1]
+        assert [search(light, X, 10) for _ in range(2)] == [1, 1]
+        assert search(dense, heavy, 10) == 2
+
+    data.on_fresh_resources(body)
