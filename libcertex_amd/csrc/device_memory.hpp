@@ -15,10 +15,14 @@ namespace cuvs::detail {
  * - the pool of a device holds at most kPoolBytes: its oldest blocks go back to the driver to make
  *   room, a larger block at once, and an allocation the driver refuses empties the pool and is tried
  *   again;
+ * - other allocators of the process cannot empty it, so that it keeps nothing on a device that is short
+ *   of memory: with less than a sixteenth free (asked for after every kPoolCheckBytes that come in,
+ *   once in a millisecond) the released block and the whole pool go back to the driver;
  * - device_trim gives the pool of a device back to the driver (cuvsCertexTrimPool).
  * A block serves requests of at least three quarters of its size, so that little of it is unused.
  */
-constexpr size_t kPoolBytes = size_t(4) << 30;
+constexpr size_t kPoolBytes      = size_t(4) << 30;
+constexpr size_t kPoolCheckBytes = size_t(64) << 20;
 
 /** At least `bytes` bytes on the current device (*capacity: how many, *device: where), or null when
  *  the device has no memory left. The contents are undefined. */

@@ -128,9 +128,12 @@ def auto_width(X, metric, target=0.95, sample=200_000):
 
 
 def trim_pool():
-    """Free the scratch memory that the calling thread's searches on the current device have grown
-    (certex/index.py:165-169, which returns the unused memory of the device's stream-ordered pool
-    to the driver), after waiting for the thread's current stream; later searches grow it again."""
+    """Free the scratch memory that the calling thread's searches on the current device have grown,
+    after waiting for the thread's current stream, and the memory of dropped indexes and scratch that
+    the library keeps on that device for its next allocations (at most 4 GiB, and none once less than
+    a sixteenth of the device is free); later calls allocate again. For an allocation outside the
+    library that fails for want of that memory (certex/index.py:165-169, which returns the unused
+    memory of the device's stream-ordered pool to the driver)."""
     C.check(C.lib().cuvsCertexTrimPool(C.resources()))
 
 

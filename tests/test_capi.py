@@ -82,3 +82,21 @@ def test_null_resources_rejected():
     L = C.lib()
     assert L.cuvsStreamSync(0) == C.CUVS_ERROR
     assert b"NULL" in L.cuvsGetLastErrorText()
+
+
+def test_rules_of_the_memory_pool(tmp_path):
+    """device_memory.cpp over a fake HIP runtime: what is reused, the pool's bound, oldest blocks out
+    first, a refused allocation and a device short of memory empty it, one wait under a device_idle."""
+    import os
+    import subprocess
+
+    here = os.path.dirname(__file__)
+    csrc = os.path.join(os.path.dirname(C.__file__), "csrc")
+    exe = tmp_path / "pool_rules"
+    subprocess.run(
+        ["g++", "-std=c++17", "-O1", "-I", os.path.join(here, "c", "fake_hip"), "-I", csrc,
+         os.path.join(here, "c", "pool_rules.cpp"), os.path.join(csrc, "device_memory.cpp"), "-o", str(exe)],
+        check=True,
+    )
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stdout
