@@ -608,8 +608,8 @@ bool screen_into_buckets(cuvs::resources const& res, int64_t nq_pad, int64_t siz
     if (past != nullptr) { *past = worst > limit; }
     if (worst <= cap) { return true; }
     if (worst > all_rows_above) { return false; }
-    int64_t c = 1024;
-    while (c < worst) { c *= 2; }
+    int64_t c = 1024;  // covers the largest count, which `worst` may be kCountStep - 1 short of
+    while (c < worst + certex_amd::kCountStep - 1) { c *= 2; }
     cap           = c;
     rs.bucket_cap = c;
   }

@@ -179,6 +179,8 @@ struct screen_group {
   int64_t tile0;
 };
 
+constexpr uint32_t kCountStep = 64;  // a power of two (screen_args::most)
+
 struct screen_args {
   const int8_t* codes;   // stored rows [*, row_bytes]: int8 codes or fp16 values
   const void* rowc;      // row terms: int32 (int8 rows) or float (fp16 rows)
@@ -218,8 +220,9 @@ struct screen_args {
   // re-rank asks for them (int32 values in the floats' bits)
   float* cand_vals     = nullptr;
   int64_t cap          = 0;
-  // *most: at least the largest bucket count past cap (exactly where flushes alone fill the
-  // bucket), else some count past most_above when a bucket passes that, else as it was
+  // *most: above cap when some bucket's count is, and then at most kCountStep - 1 below the largest
+  // count (survivors that are counted one by one note every kCountStep-th past cap); else some count
+  // past most_above when a bucket passes that, else as it was
   uint32_t* most      = nullptr;
   uint32_t most_above = 0;
   // screen: survivors past a workgroup's LDS list go to the workgroup's own region of a pool of

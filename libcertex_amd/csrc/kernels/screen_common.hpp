@@ -302,11 +302,12 @@ __device__ __forceinline__ void note_count(const screen_args& a, uint32_t old, u
   }
 }
 
-/** A survivor counted by an atomic of its own, at slot `at`: every 64th of them past the bucket is
- *  noted, and the ones that pass a limit. */
+/** A survivor counted by an atomic of its own, at slot `at`: every kCountStep-th of them past the
+ *  bucket is noted, and the ones that pass a limit. */
 __device__ __forceinline__ void note_slot(const screen_args& a, uint32_t at)
 {
-  if (at == a.most_above || at == a.cap || ((at & 63u) == 63u && at >= a.cap)) { note_count(a, at, at + 1); }
+  constexpr uint32_t last = kCountStep - 1;
+  if (at == a.most_above || at == a.cap || ((at & last) == last && at >= a.cap)) { note_count(a, at, at + 1); }
 }
 
 /**
