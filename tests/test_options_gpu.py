@@ -165,21 +165,26 @@ def test_pooled_memory_across_threads_and_streams(gpu):
         want[t] = oracle.knn(X[t * 10_000:][: 20_000 + 1_000 * t], Q, 5, "l2")[1]
     Xg, Qg = torch.from_numpy(X).cuda(), torch.from_numpy(Q).cuda()
     torch.cuda.synchronize()
-    bad = []
+    done, failed = [0] * 4, []
 
     def work(t):
-        with torch.cuda.stream(torch.cuda.Stream()):
-            for _ in range(15):
-                idx = certex.Index(128)
-                idx.add(Xg[t * 10_000:][: 20_000 + 1_000 * t])
-                D, I = idx.search(Qg, k=5)
-                del idx
-                if not np.array_equal(I.cpu().numpy(), want[t]):
-                    bad.append(t)
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(15):
+                    idx = certex.Index(128)
+                    idx.add(Xg[t * 10_000:][: 20_000 + 1_000 * t])
+                    D, I = idx.search(Qg, k=5)
+                    del idx
+                    np.testing.assert_array_equal(I.cpu().numpy(), want[t])
+                    done[t] += 1
+        except BaseException as e:  # noqa: B036
+            failed.append(e)
 
     threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
     for th in threads:
         th.start()
     for th in threads:
         th.join()
-    assert not bad
+    if failed:
+        raise failed[0]
+    assert done == [15] * 4
