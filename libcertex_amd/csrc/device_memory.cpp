@@ -166,12 +166,6 @@ void device_trim(int device) noexcept
   for (auto const& b : blocks) { (void)hipFree(b.second.p); }
 }
 
-size_t device_pooled(int device)
-{
-  std::lock_guard lk(g_mutex);
-  return pools()[device].held;
-}
-
 void device_idle::enter(int device) noexcept
 {
   on_device at(device);

@@ -32,8 +32,6 @@ void* device_allocate(size_t bytes, size_t* capacity, int* device);
 void device_release(void* p, size_t capacity, int device) noexcept;
 /** Gives every pooled block of `device` back to the driver. */
 void device_trim(int device) noexcept;
-/** Bytes that the pool of `device` holds. */
-size_t device_pooled(int device);
 
 /**
  * Between enter() and the guard's end, blocks of `device` that this thread releases enter the pool
