@@ -102,6 +102,7 @@ CUVS_EXPORT cuvsError_t cuvsCertexPartitionByLabels(cuvsResources_t res, cuvsCer
 /**
  * Exact k nearest neighbours, k = the second extent of `neighbors` (reference certex.h:183-189):
  * queries [nq, dim] (device, index type), neighbors [nq, k] int64, distances [nq, k] float32.
+ * Vectors that another thread adds during a filtered search, past the ids its words cover, are excluded.
  */
 CUVS_EXPORT cuvsError_t cuvsCertexSearch(cuvsResources_t res,
                                          cuvsCertexSearchParams_t params,

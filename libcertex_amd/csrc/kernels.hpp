@@ -334,7 +334,7 @@ void screen_f16_tile(const screen_args& a, hipStream_t stream);
  */
 void anchors_f16_tile(const screen_args& a, hipStream_t stream);
 /** The tiled screen and tiled anchor pass over int8 rows of more than 256 bytes (exact int32
- *  screen values; survivors carry no value). */
+ *  screen values; survivors carry theirs where cand_vals is given). */
 void screen_i8_tile(const screen_args& a, hipStream_t stream);
 void anchors_i8_tile(const screen_args& a, hipStream_t stream);
 int tile_chunk_steps();
