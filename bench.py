@@ -35,7 +35,7 @@ SCREEN_I8_SOURCES = ("kernels/screen.hip", "kernels/screen_common.hpp", "kernels
 # every kernel source: the stamp of the config 3 and 4 counter profiles
 KERNEL_SOURCES = ("kernels/screen.hip", "kernels/screen_tile.hip", "kernels/screen_wide.hip",
                   "kernels/screen_common.hpp", "kernels/select.hip", "kernels/encode.hip",
-                  "kernels/partition.hip", "kernels/lists.hip", "kernels.hpp")
+                  "kernels/partition.hip", "kernels/lists.hip", "kernels/lanes.hpp", "kernels.hpp")
 PROFILE_C3 = os.path.join(ROOT, "profiles", "screen_f16_c3_counters.txt")
 PROFILE_C4 = os.path.join(ROOT, "profiles", "screen_f16_c4_counters.txt")
 

@@ -100,3 +100,14 @@ def test_rules_of_the_memory_pool(tmp_path):
     )
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout
+
+
+def test_profile_stamp_covers_every_kernel_source():
+    """The stamp of the counter profiles changes with every file that device code comes from."""
+    import os
+
+    import bench
+
+    csrc = os.path.join(os.path.dirname(C.__file__), "csrc")
+    files = {"kernels/" + f for f in os.listdir(os.path.join(csrc, "kernels"))} | {"kernels.hpp"}
+    assert set(bench.KERNEL_SOURCES) == files
