@@ -203,6 +203,15 @@ __device__ inline _Float16 to_f16(double z)
   return fabs(double(h)) < 6.103515625e-05 ? _Float16(0.0f) : h;
 }
 
+/** to_f16 for queries, which may lie any distance from the rows: a finite value past the range of fp16
+ *  becomes its largest one, and the difference goes into the query's |W - fp16(W)| (an infinite half
+ *  made NaN screen values, which pass no threshold). */
+__device__ inline _Float16 query_f16(double w)
+{
+  constexpr double most = 65504.0;
+  return to_f16(fabs(w) > most && fabs(w) < INFINITY ? copysign(most, w) : w);
+}
+
 /** Sum of v over the 64 lanes of a wave (xor butterfly: every lane gets the sum). */
 __device__ inline double wave_sum(double v) { return lanes::sum<64>(v); }
 
@@ -646,7 +655,7 @@ __global__ __launch_bounds__(256) void encode_queries_f16_kernel(const void* q, 
       const int64_t j = j0 + 64 * u + lane;
       if (j < dim) {
         const double w   = (v[u] / nrm - c[u]) * inv_alpha;
-        const _Float16 h = to_f16(w);
+        const _Float16 h = query_f16(w);
         const double e   = w - double(h);
         put(j, h);
         a  = fma(w, w, a);

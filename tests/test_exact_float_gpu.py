@@ -303,3 +303,18 @@ def test_rerank_launches_behind_the_screen(gpu):
         assert search(dense, heavy, 10) == 2
 
     data.on_fresh_resources(body)
+
+
+@pytest.mark.parametrize("d", [32, 300])
+@pytest.mark.parametrize("metric, spread", [("l2", 1e-5), ("cosine", 1e-5), ("cosine", 0.0)])
+def test_queries_far_outside_the_rows(gpu, metric, spread, d):
+    """Rows in a ball of a hundred-thousandth of the queries' distance (or all alike): the queries'
+    screening coordinates pass the range of fp16, and the results are the exhaustive ones."""
+    for n in (7, 1_500, 20_000):
+        X = (1 + spread * data.gaussian(n, d, 61)).astype(np.float32)
+        Q = np.concatenate([data.gaussian(8, d, 62), X[:4], 1e4 * data.gaussian(4, d, 63)]).astype(np.float32)
+        D, I, _ = run(X, Q, 5, metric)
+        s, i = oracle.knn(X, Q, 5, metric)
+        np.testing.assert_array_equal(I, i)
+        want = oracle.distances(s, i, metric)
+        np.testing.assert_array_equal(D, np.float32(1) - want if metric == "cosine" else want)
