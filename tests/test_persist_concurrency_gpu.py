@@ -81,29 +81,30 @@ def test_load_rejects_foreign_files(gpu, tmp_path):
 
 def search_while_adding(search, add):
     """search(nq) in a thread of its own and add() while it runs: what the search returned (or the
-    exception that ended it). A search that was over before the rows were added runs again with more
-    queries."""
-    for nq in (5_000, 20_000, 80_000):
+    exception that ended it). A search that did not go on for 20 ms (hundreds of batches) after the rows
+    were added runs again with more queries."""
+    for nq in (10_000, 40_000, 80_000):
         out = []
 
         def body():
             try:
                 with torch.cuda.stream(torch.cuda.Stream()):
                     out.append(search(nq))
+                    out.append(time.perf_counter())
                     torch.cuda.current_stream().synchronize()
             except BaseException as e:  # noqa: B036
-                out.append(e)
+                out[:] = [e]
 
         t = threading.Thread(target=body)
         t.start()
-        time.sleep(0.1)
+        time.sleep(0.05)
         add()
         torch.cuda.synchronize()
-        running = t.is_alive()
+        added = time.perf_counter()
         t.join()
-        if running or isinstance(out[0], BaseException):
+        if isinstance(out[0], BaseException) or out[1] - added > 0.02:
             return out[0]
-    pytest.fail("no search was running when rows were added")
+    pytest.fail("no search went on after the rows were added")
 
 
 def test_rows_added_past_an_id_map(gpu):
