@@ -1588,15 +1588,16 @@ void routed_batch(cuvs::resources const& res, index_state const& st, batch_fn ba
   // no wait here: the next use of the staging waits for this batch's copy of the tables
 }
 
-/** The filter of a search over an index of `size` vectors. */
-auto to_args(filter const& f, int64_t size) -> certex_amd::filter_args
+/** The filter of a search. */
+auto to_args(filter const& f, index_state const& st) -> certex_amd::filter_args
 {
   certex_amd::filter_args fa{};
   if (f.type != filter::kind::none) {
     expects(f.words != nullptr, "certex: a filter needs its words");
     fa.kind  = f.type == filter::kind::bitset ? 1 : 2;
     fa.words = f.words;
-    fa.n_ids = f.ids > 0 ? f.ids : size;
+    fa.n_ids = f.ids > 0 ? f.ids : int64_t(st.size);
+    expects(fa.n_ids >= st.n_listed, "certex: a filter covers the vectors of the index");
   }
   return fa;
 }
@@ -1759,7 +1760,7 @@ void search_without_allocation(cuvs::resources const& res, search_params const& 
                                index<T> const& idx, matrix_view<const T> queries,
                                int64_t* neighbors, float* distances, int64_t k, filter f)
 {
-  const certex_amd::filter_args fa = to_args(f, idx.size());
+  const certex_amd::filter_args fa = to_args(f, idx.state());
   expects(!t_capture.on, "certex: a capture covers the allocating search");
   char* base = scratch_of(res.device());
   scratch_turn turn(res.device(), static_cast<hipStream_t>(res.stream()));
@@ -2312,7 +2313,7 @@ void search(cuvs::resources const& res, search_params const& params, index<T> co
             matrix_view<const T> queries, int64_t* neighbors, float* distances, int64_t k,
             filter f)
 {
-  const certex_amd::filter_args fa = to_args(f, idx.size());
+  const certex_amd::filter_args fa = to_args(f, idx.state());
   search_impl(res, params, idx, queries, neighbors, distances, k, fa);
 }
 

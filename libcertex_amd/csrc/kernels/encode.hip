@@ -329,12 +329,12 @@ struct unit_scale {
 
 /**
  * v / |x|: the product with the correctly rounded reciprocal, corrected once by its exact remainder
- * (Markstein's method), at a fifth of the division's instructions (an index of 240,000 x
- * 300 cosine halves built, searched and dropped: 660 us, 730 with the division). The corrected value is off the quotient by
- * at most 1.5 x 2^-53 ulp before its one rounding, so that it is the division's result unless a
- * quotient lies that close to the midpoint of two doubles: coordinates have at most 24 bits, and of
- * 4e8 quotients, and of the 102 closest to a midpoint found among 8.6e9 norms, every one is the
- * division's.
+ * (Markstein's method), at a fifth of the division's instructions (an index of 240,000 x 300 cosine
+ * halves built, searched and dropped: 660 us, 730 with the division). The corrected value is off the
+ * quotient by at most 1.5 x 2^-53 ulp before its one rounding, so that it is the division's result
+ * unless a quotient lies that close to the midpoint of two doubles: coordinates have at most 24 bits,
+ * and of 4e8 quotients, and of the 102 closest to a midpoint found among 8.6e9 norms, every one is
+ * the division's.
  */
 __device__ __forceinline__ double unit_coord(double v, const unit_scale& s)
 {
